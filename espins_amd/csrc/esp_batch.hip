@@ -28,17 +28,24 @@ namespace {
 // ---- batched kernels -------------------------------------------------------------------
 // tiles: (chain, replica, block, 0); chain < 0 = padding tile (XCD interleave)
 template <int MODE, int LAY, bool HB, bool HD, bool SELF, int CH>
-__global__ __launch_bounds__(kBlock) ESP_PHASE_ATTR void k_bphase(const KArgs *chains, const int4 *tiles, int colour,
+__global__ __launch_bounds__(kPhaseBlock) ESP_PHASE_ATTR void k_bphase(const KArgs *chains, const int4 *tiles, int colour,
                                                    int sweep_off) {
   extern __shared__ double s_ctab[];
   const int4 t = tiles[blockIdx.x];
   if (t.x < 0) return;
   KArgs a = chains[t.x];
   a.col = colour;
-  a.c_begin = gldi(a.col_off, colour);
-  a.c_count = gldi(a.col_off, colour + 1) - a.c_begin;
+  a.c_begin = cldi(a.col_off, colour);
+  a.c_count = cldi(a.col_off, colour + 1) - a.c_begin;
+  if (LAY == LAY_IMP && a.tseg) {
+    const uint32_t *d = reinterpret_cast<const uint32_t *>(a.cngc + colour);
+    a.dngc = {cldi(d, 0), cldi(d, 1), cldi(d, 2), cldi(d, 3)};
+  }
   a.sweep_off = sweep_off;
-  phase_body<MODE, LAY, HB, HD, SELF, CH>(a, t.y, t.z, s_ctab);
+  // chains with and without geometry-group tiles share the launch (a launch of their own would
+  // run after the others'): 12 us per colour for the few small chains of a mixed batch
+  if (LAY == LAY_IMP && a.tseg == 0) phase_body<MODE, LAY_CMP, HB, HD, SELF, CH>(a, t.y, t.z, s_ctab);
+  else phase_body<MODE, LAY, HB, HD, SELF, CH>(a, t.y, t.z, s_ctab);
 }
 
 // LDS-resident chains: one block per (chain, replica)
@@ -92,8 +99,9 @@ using BPhaseFn = void (*)(const KArgs *, const int4 *, int, int);
 using BLdsFn = void (*)(const KArgs *, const LdsMeas *, const int2 *, int, int);
 
 // variant bits: 0-1 coefficient layout (LAY_*), 2 biquadratic, 3 DM, 4 self bonds; launch
-// variants add bit 5: partner gathers in flight per lane 4 instead of 2 (global path)
+// variants add bit 5: the wide setting of the partner gathers in flight per lane (global path)
 constexpr int kVarChunk4 = 32;
+constexpr int kNarrow = 2;   // the narrow setting, as set_chain_chunk and info name it
 template <int MODE, int LAY, bool HB, bool HD, int CH>
 BPhaseFn bp4(bool self) { return self ? k_bphase<MODE, LAY, HB, HD, true, CH> : k_bphase<MODE, LAY, HB, HD, false, CH>; }
 template <int MODE, int LAY, bool HB, int CH>
@@ -103,10 +111,8 @@ BPhaseFn bp2(bool hb, bool hd, bool self) {
   return hb ? bp3<MODE, LAY, true, CH>(hd, self) : bp3<MODE, LAY, false, CH>(hd, self);
 }
 template <int MODE, int CH>
-BPhaseFn bp1(int v) {
-  const int lay = v & 3;
-  if (lay == LAY_IMP) return bp2<MODE, LAY_IMP, CH>(v & 4, v & 8, v & 16);
-  return lay == LAY_CMP ? bp2<MODE, LAY_CMP, CH>(v & 4, v & 8, v & 16) : bp2<MODE, LAY_BOND, CH>(v & 4, v & 8, v & 16);
+BPhaseFn bp1(int v) {   // launch variants: LAY_IMP (serves LAY_CMP chains too) or LAY_BOND
+  return (v & 3) ? bp2<MODE, LAY_IMP, CH>(v & 4, v & 8, v & 16) : bp2<MODE, LAY_BOND, CH>(v & 4, v & 8, v & 16);
 }
 template <int MODE>
 BPhaseFn bp0(int v) { return (v & kVarChunk4) ? bp1<MODE, 4>(v) : bp1<MODE, kChunk>(v); }
@@ -149,7 +155,8 @@ struct Chain {
   int R = 0, Ns = 0;
   std::vector<double> tems, spins;       // initial spins, reference order
   int variant = 0, tps = 1, lds = 0, lds_fits = 0, red_blocks = 1;
-  int chunk = kChunk;                    // partner gathers in flight per lane (global path): 2 or 4
+  // partner gathers in flight per lane (global path): kNarrow runs kChunk (3, measured best), or 4
+  int chunk = kNarrow;
   // blocks per replica of the per-step sums (k_breduce): one per 4096 per-wave entries; the
   // direct energy's red_blocks cover 4096 spins each, 64 times the work of a per-wave sum
   int sum_blocks = 1;
@@ -163,14 +170,21 @@ struct Chain {
   uint8_t *basis = nullptr;
   unsigned long long *rej = nullptr, *nswap = nullptr, *nmeas = nullptr;
   double *mpart = nullptr;   // per-wave spin sums of the colour phases (global-path chains)
-  int mpart_nw = 0;
-  int *grp = nullptr, *gslot = nullptr;   // implicit geometry (esp_geo.h)
-  double *magb = nullptr;
+  int mpart_nw = 0, mpart_tps = 0;
+  // implicit geometry: group records (esp_geo.h) and bond lists (SegTables, esp_model.h)
+  int *grp = nullptr, *gcnt = nullptr;
+  unsigned long long *gbond = nullptr;
+  double *gcoef = nullptr;
+  espg::FastDiv *cngc = nullptr;
 };
 
-// Kernel grouping of a chain's colour phases: its Hamiltonian variant and, on the global path,
-// the chunk width.
-int launch_variant(const Chain &c) { return c.variant | (!c.lds && c.chunk == 4 ? kVarChunk4 : 0); }
+// Kernel grouping of a chain's colour phases: its Hamiltonian variant (one for both compressed
+// layouts) and, on the global path, the chunk width.
+int launch_variant(const Chain &c) {
+  const int v = (c.variant & 3) == LAY_CMP ? (c.variant & ~3) | LAY_IMP : c.variant;
+  return v | (!c.lds && c.chunk == 4 ? kVarChunk4 : 0);
+}
+bool chain_geo(const Chain &c) { return geo_tiles(c.hm, c.tps); }
 
 }  // namespace
 
@@ -254,7 +268,7 @@ void free_chain(Chain &c) {
   bfree(c.slot_rep); bfree(c.rep_slot); bfree(c.basis); bfree(c.rej); bfree(c.nswap); bfree(c.nmeas);
   bfree(c.mpart);
   c.mpart_nw = 0;
-  bfree(c.grp); bfree(c.gslot); bfree(c.magb);
+  bfree(c.grp); bfree(c.gcnt); bfree(c.gbond); bfree(c.gcoef); bfree(c.cngc);
 }
 
 void drop_plan(esp_batch *b) {
@@ -280,8 +294,8 @@ KArgs chain_args(const Chain &c, int k) {
   a.mpart_nw = c.mpart_nw;
   a.stream_base = (uint32_t)k << 16;
   a.geo = c.hm.geo;
-  a.grp = c.grp; a.gslot = c.gslot; a.magb = c.magb;
-  a.rows_max = c.hm.rows_max;
+  a.grp = c.grp; a.gcnt = c.gcnt; a.gbond = c.gbond; a.gcoef = c.gcoef; a.cngc = c.cngc;
+  if (chain_geo(c)) geo_args(a, c.hm);
   return a;
 }
 
@@ -290,10 +304,9 @@ KArgs chain_args(const Chain &c, int k) {
 // accumulators are re-laid out their sums move into e_base.
 int size_wave_sums(esp_batch *b, Chain &c) {
   int nw = 1;
-  for (int col = 0; col < c.hm.ncol; ++col)
-    nw = std::max(nw, ((c.hm.col_off[col + 1] - c.hm.col_off[col]) * c.tps + 63) / 64);
+  for (int col = 0; col < c.hm.ncol; ++col) nw = std::max(nw, colour_waves(c.hm, col, c.tps, chain_geo(c)));
   const size_t n = (size_t)c.R * c.hm.ncol * nw;
-  if (nw == c.mpart_nw && c.mpart && c.w) {
+  if (nw == c.mpart_nw && c.tps == c.mpart_tps && c.mpart && c.w) {
     BCHK(b, hipMemsetAsync(c.mpart, 0, 3 * n * sizeof(double), b->stream));
     return ESP_OK;
   }
@@ -307,6 +320,7 @@ int size_wave_sums(esp_batch *b, Chain &c) {
   BCHK(b, hipMemsetAsync(c.mpart, 0, 3 * n * sizeof(double), b->stream));
   BCHK(b, hipMemsetAsync(c.w, 0, n * sizeof(double), b->stream));
   c.mpart_nw = nw;
+  c.mpart_tps = c.tps;
   return ESP_OK;
 }
 
@@ -366,34 +380,27 @@ int build_plan(esp_batch *b, double tilt, uint64_t seed) {
       b->vars.back().variant = launch_variant(c);
     }
   for (auto &v : b->vars) {
-    // global-path tiles per colour, interleaved so that tile t runs on XCD t % 8 and all
-    // tiles of one replica share an XCD (and its L2)
+    // Global-path tiles per colour.  Tile t runs on XCD t % 8 and all tiles of one replica share
+    // an XCD (and its L2).  Replicas go, largest first, to the XCD with the fewest tiles so far:
+    // dealt out in turn, the replicas of a chain differ by one between XCDs, and a few large
+    // chains left XCDs idle at the end of the launch.
     v.d_tiles.assign(b->maxcol, nullptr);
     v.ntiles.assign(b->maxcol, 0);
     for (int col = 0; col < b->maxcol; ++col) {
-      std::vector<std::vector<int4>> q(8);
-      int qi = 0;
+      std::vector<std::pair<int, int>> unit;           // (blocks per replica, chain)
       for (int k = 0; k < nc; ++k) {
         const Chain &c = b->chains[k];
         if (launch_variant(c) != v.variant || c.lds || col >= c.hm.ncol) continue;
-        const int cnt = c.hm.col_off[col + 1] - c.hm.col_off[col];
-        const int nblk = (cnt * c.tps + kBlock - 1) / kBlock;
-        // Implicit geometry: every group of the colour has the same sub-cell layout, so the
-        // blocks go in sub-cell order across the groups (block (g, t) of every group g before
-        // any block t + 1).  Blocks that run together then gather from the same region of the
-        // lattice and share its lines in L2 (about 30 % fewer L2 misses than group order).
-        std::vector<int> order(nblk);
-        for (int bb = 0; bb < nblk; ++bb) order[bb] = bb;
-        if (c.hm.implicit) {
-          const int per = kBlock / c.tps, mt = (int)c.hm.geo.mt.d;
-          std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-            const int ox = x * per, oy = y * per;
-            return std::make_pair(ox % mt, ox / mt) < std::make_pair(oy % mt, oy / mt);
-          });
-        }
-        for (int r = 0; r < c.R; ++r, ++qi)
-          for (int bb = 0; bb < nblk; ++bb) q[qi % 8].push_back(make_int4(k, r, order[bb], 0));
+        // (geometry-group tiles are numbered in sub-cell order across the groups)
+        unit.push_back({colour_blocks(c.hm, col, c.tps, chain_geo(c)), k});
       }
+      std::stable_sort(unit.begin(), unit.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
+      std::vector<std::vector<int4>> q(8);
+      for (const auto &[nblk, k] : unit)
+        for (int r = 0; r < b->chains[k].R; ++r) {
+          auto &x = *std::min_element(q.begin(), q.end(), [](const auto &m, const auto &n) { return m.size() < n.size(); });
+          for (int bb = 0; bb < nblk; ++bb) x.push_back(make_int4(k, r, bb, 0));
+        }
       size_t longest = 0;
       for (auto &x : q) longest = std::max(longest, x.size());
       std::vector<int4> tiles;
@@ -410,7 +417,8 @@ int build_plan(esp_batch *b, double tilt, uint64_t seed) {
     for (int k = 0; k < nc; ++k) {
       const Chain &c = b->chains[k];
       if (launch_variant(c) != v.variant) continue;
-      shm_p = std::max(shm_p, phase_lds_bytes(c.variant & 3, c.hm.nb, c.hm.zmax, c.hm.rows_max));
+      shm_p = std::max(shm_p, phase_lds_bytes((c.variant & 3) == LAY_BOND ? LAY_BOND : chain_geo(c) ? LAY_IMP : LAY_CMP,
+                                              c.hm.nb, c.hm.zmax));
       if (!c.lds) continue;
       shm_l = std::max(shm_l, c.lds_bytes);
       for (int r = 0; r < c.R; ++r) li.push_back(make_int2(k, r));
@@ -448,7 +456,7 @@ int enqueue_round(esp_batch *b, int steps, int M, bool measure, bool exchange, i
       for (int col = 0; col < b->maxcol; ++col)
         for (auto &v : b->vars)
           if (v.ntiles[col] > 0)
-            hipLaunchKernelGGL(bphase_fn(mode, v.variant), dim3(v.ntiles[col]), dim3(kBlock), v.shm_phase,
+            hipLaunchKernelGGL(bphase_fn(mode, v.variant), dim3(v.ntiles[col]), dim3(kPhaseBlock), v.shm_phase,
                                b->stream, (const KArgs *)b->d_chains, (const int4 *)v.d_tiles[col], col,
                                s * M + m);
     BCHK(b, hipGetLastError());
@@ -581,8 +589,6 @@ int esp_batch_add_chain(esp_batch *b, int N, int nb, const double *mag, int zJ, 
     c.hm.implicit = false;
   }
   if (!c.hm.compressed) c.ctab_bytes = 0;
-  if (c.hm.implicit && phase_lds_bytes(LAY_IMP, c.hm.nb, c.hm.zmax, c.hm.rows_max) > 49152)
-    c.hm.implicit = false;
   if ((size_t)c.hm.zmax * N * sizeof(int) >= (1ull << 32)) return bfail(b, ESP_EINVAL, "bond table beyond 4 GiB");
   if (L3) std::memcpy(c.L, L3, sizeof c.L);
   c.R = R;
@@ -648,11 +654,15 @@ int esp_batch_commit(esp_batch *b) {
     if ((rc = bupload(b, c.basis, m.basis.data(), m.basis.size()))) return rc;
     if ((rc = bupload(b, c.si4, m.si4.data(), m.si4.size()))) return rc;
     if ((rc = bupload(b, c.h4, m.h4.data(), m.h4.size()))) return rc;
-    if (m.implicit) {
-      if ((rc = bupload(b, c.grp, m.grp.data(), m.grp.size()))) return rc;
-      if ((rc = bupload(b, c.gslot, m.gslot.data(), m.gslot.size()))) return rc;
-      if ((rc = bupload(b, c.magb, m.magb.data(), m.magb.size()))) return rc;
-    }
+    const esp::SegTables seg = m.implicit && m.compressed ? esp::segment_tables(m) : esp::SegTables{};
+    std::vector<espg::FastDiv> ngc;
+    for (int col = 0; !seg.cnt.empty() && col < m.ncol; ++col) ngc.push_back(geo_ngc(m, col));
+    if (!seg.cnt.empty() && ((rc = bupload(b, c.cngc, ngc.data(), ngc.size())) ||
+                             (rc = bupload(b, c.grp, m.grp.data(), m.grp.size())) ||
+                             (rc = bupload(b, c.gcnt, seg.cnt.data(), seg.cnt.size())) ||
+                             (rc = bupload(b, c.gbond, seg.bond.data(), seg.bond.size())) ||
+                             (rc = bupload(b, c.gcoef, seg.coef.data(), seg.coef.size()))))
+      return rc;
     if (m.compressed) {
       if ((rc = bupload(b, c.ctab, m.ctab.data(), m.ctab.size()))) return rc;
     } else {
@@ -870,7 +880,7 @@ namespace {
 // scales the work.
 int autotune_body(esp_batch *b, int nrounds, const char *cache_path) {
   struct Shape {
-    int lds = 0, tps = 1, chunk = kChunk;
+    int lds = 0, tps = 1, chunk = kNarrow;
   };
   std::map<std::string, Shape> decided;
   if (cache_path) {
@@ -881,7 +891,7 @@ int autotune_body(esp_batch *b, int nrounds, const char *cache_path) {
       while (std::fgets(line, sizeof line, f)) {
         const int n = std::sscanf(line, "%127s %d %d %lf %d", key, &l, &t, &ms, &ch);
         if (n >= 4 && (t == 1 || t == 2 || t == 4))
-          decided[key] = Shape{l, t, n == 5 && (ch == 2 || ch == 4) ? ch : kChunk};
+          decided[key] = Shape{l, t, n == 5 && (ch == 2 || ch == 4) ? ch : kNarrow};
       }
       std::fclose(f);
     }
@@ -931,8 +941,8 @@ int autotune_body(esp_batch *b, int nrounds, const char *cache_path) {
       for (int tps = 1; tps <= 4; tps *= 2) {
         if (tps > 1 && tps > c0.hm.zmax) break;
         for (int ch = 2; ch <= 4; ch += 2)
-          if (tps > 1 || ch != kChunk) cand.push_back(Shape{0, tps, ch});
-        if (c0.lds_fits) cand.push_back(Shape{1, tps, kChunk});
+          if (tps > 1 || ch != kNarrow) cand.push_back(Shape{0, tps, ch});
+        if (c0.lds_fits) cand.push_back(Shape{1, tps, kNarrow});
       }
       for (const Shape &sh : cand) {
         const Shape prev = decided[key];
@@ -994,7 +1004,7 @@ int esp_batch_time_sweeps(esp_batch *b, int nsweeps, int mode, uint64_t seed, ui
     for (int col = 0; col < b->maxcol; ++col)
       for (auto &v : b->vars)
         if (v.ntiles[col] > 0) {
-          hipExtLaunchKernelGGL(bphase_fn(mode, v.variant), dim3(v.ntiles[col]), dim3(kBlock), v.shm_phase,
+          hipExtLaunchKernelGGL(bphase_fn(mode, v.variant), dim3(v.ntiles[col]), dim3(kPhaseBlock), v.shm_phase,
                                 b->stream, ev[2 * k], ev[2 * k + 1], 0, (const KArgs *)b->d_chains,
                                 (const int4 *)v.d_tiles[col], col, s);
           ++k;

@@ -30,8 +30,10 @@ struct esp_ctx {
   double *d_cJ = nullptr, *d_cB = nullptr, *d_cD = nullptr, *d_ctab = nullptr;
   double *d_mag = nullptr, *d_si4 = nullptr, *d_h4 = nullptr;
   uint8_t *d_basis = nullptr;
-  int *d_grp = nullptr, *d_gslot = nullptr;   // implicit geometry (esp_geo.h)
-  double *d_magb = nullptr;
+  // implicit geometry: group records (esp_geo.h) and bond lists (SegTables, esp_model.h)
+  int *d_grp = nullptr, *d_gcnt = nullptr;
+  unsigned long long *d_gbond = nullptr;
+  double *d_gcoef = nullptr;
   bool use_lds = false;
   size_t lds_bytes = 0, ctab_bytes = 0;
   // replicas
@@ -53,9 +55,11 @@ struct esp_ctx {
   double *d_prop = nullptr, *d_unif = nullptr;
   uint8_t *d_accd = nullptr;
   // per-wave spin sums of the colour phases: [R][ncol][mpart_nw][3]; valid while the last
-  // change of the spins was a full global-path sweep (d_w has the same wave layout)
+  // change of the spins was a full global-path sweep (d_w has the same wave layout).  The
+  // waves' layout: geometry-group tiles or not, lanes per site
   double *d_mpart = nullptr;
-  int mpart_nw = 0;
+  int mpart_nw = 0, mpart_tps = 0;
+  bool mpart_geo = false;
   bool mpart_valid = false;
   // per-measurement trace of E and |m| by slot (global-memory path only)
   double *d_trace = nullptr;      // [trace_cap][R][2]
@@ -179,7 +183,7 @@ void free_model(esp_ctx *c) {
   dfree(c->d_nbr); dfree(c->d_dev2ref); dfree(c->d_ref2dev); dfree(c->d_col_off);
   dfree(c->d_cJ); dfree(c->d_cB); dfree(c->d_cD); dfree(c->d_ctab); dfree(c->d_mag);
   dfree(c->d_si4); dfree(c->d_h4); dfree(c->d_basis);
-  dfree(c->d_grp); dfree(c->d_gslot); dfree(c->d_magb);
+  dfree(c->d_grp); dfree(c->d_gcnt); dfree(c->d_gbond); dfree(c->d_gcoef);
   c->have_model = false;
   drop_graph(c);
 }
@@ -200,8 +204,8 @@ KArgs base_args(esp_ctx *c) {
   a.has_si = m.has_si; a.has_h = m.has_h;
   a.stream_base = c->stream_base;
   a.geo = m.geo;
-  a.grp = c->d_grp; a.gslot = c->d_gslot; a.magb = c->d_magb;
-  a.rows_max = m.rows_max;
+  a.grp = c->d_grp; a.gcnt = c->d_gcnt; a.gbond = c->d_gbond; a.gcoef = c->d_gcoef;
+  if (m.implicit) espk::geo_args(a, m);
   return a;
 }
 

@@ -91,24 +91,27 @@ struct SiteGeo {
   int ir;             // reference site index (0-based): ((x2 L1 + x1) L0 + x0) nb + a
 };
 
-ESP_HD SiteGeo geo_site(const Geo &G, const int *grp, int d) {
+// Site k of group g, whose record is e.
+ESP_HD SiteGeo geo_place(const Geo &G, int e, int g, int k) {
   SiteGeo s;
-  const uint32_t ud = (uint32_t)d;
-  const uint32_t g = fdiv(ud, G.mt);
-  const uint32_t k = ud - g * (uint32_t)G.mt.d;
-  const uint32_t t = fdiv(k, G.m0);
-  s.g = (int)g;
-  s.s0 = (int)(k - t * (uint32_t)G.M0);
+  const uint32_t uk = (uint32_t)k;
+  const uint32_t t = fdiv(uk, G.m0);
+  s.g = g;
+  s.s0 = (int)(uk - t * (uint32_t)G.M0);
   const uint32_t u = fdiv(t, G.m1);
   s.s1 = (int)(t - u * (uint32_t)G.M1);
   s.s2 = (int)u;
-  const int e = grp[g];
   s.a = e & 0xff;
   const int x0 = s.s0 * G.P0 + ((e >> 8) & 0xff);
   const int x1 = s.s1 * G.P1 + ((e >> 16) & 0xff);
   const int x2 = s.s2 * G.P2 + ((e >> 24) & 0xff);
   s.ir = ((x2 * G.L1 + x1) * G.L0 + x0) * G.nb + s.a;
   return s;
+}
+
+ESP_HD SiteGeo geo_site(const Geo &G, const int *grp, int d) {
+  const uint32_t g = fdiv((uint32_t)d, G.mt);
+  return geo_place(G, grp[g], (int)g, (int)((uint32_t)d - g * (uint32_t)G.mt.d));
 }
 
 // (s + q) mod M for s, q in [0, M): t = s + q < 2M, and t - M wraps to a huge unsigned value
@@ -119,15 +122,19 @@ ESP_HD uint32_t wrap_add(uint32_t s, uint32_t q, uint32_t M) {
   return umin32(t, t - M);
 }
 
-// Device index of the partner of site s through the (group, slot) record (pg, qp), computed
-// without branches: padding slots (pg < 0) select the zero spin N.
+// Place inside its group of the sub-cell of s shifted by the packed shift q.
+ESP_HD int geo_shift(const Geo &G, const SiteGeo &s, uint32_t q) {
+  const uint32_t v0 = wrap_add((uint32_t)s.s0, q & 0xffu, (uint32_t)G.M0);
+  const uint32_t v1 = wrap_add((uint32_t)s.s1, (q >> 8) & 0xffu, (uint32_t)G.M1);
+  const uint32_t v2 = wrap_add((uint32_t)s.s2, (q >> 16) & 0xffu, (uint32_t)G.M2);
+  return (int)umad24(umad24(v2, (uint32_t)G.M1, v1), (uint32_t)G.M0, v0);
+}
+
+// Device index of the partner of site s through the (group, slot) record (pg, qp); padding
+// slots (pg < 0) give the zero spin N.
 ESP_HD int geo_partner(const Geo &G, const SiteGeo &s, int pg, int qp) {
-  const uint32_t uq = (uint32_t)qp;
-  const uint32_t v0 = wrap_add((uint32_t)s.s0, uq & 0xffu, (uint32_t)G.M0);
-  const uint32_t v1 = wrap_add((uint32_t)s.s1, (uq >> 8) & 0xffu, (uint32_t)G.M1);
-  const uint32_t v2 = wrap_add((uint32_t)s.s2, (uq >> 16) & 0xffu, (uint32_t)G.M2);
-  const uint32_t j = (uint32_t)pg + umad24(umad24(v2, (uint32_t)G.M1, v1), (uint32_t)G.M0, v0);
-  return pg < 0 ? G.N : (int)j;
+  const int j = pg + geo_shift(G, s, (uint32_t)qp);
+  return pg < 0 ? G.N : j;
 }
 
 }  // namespace espg

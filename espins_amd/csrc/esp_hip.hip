@@ -94,21 +94,23 @@ int64_t launch_lanes(const esp_ctx *c) {
   return (int64_t)c->hm.N * c->tps / std::max(1, c->hm.ncol) * c->R;
 }
 
-// Coefficient layout of the colour phases of this context.
+// Coefficient layout of this context, as reported; the colour phases use LAY_IMP only where
+// tiles of one geometry group fit (geo_tiles), else the tables.
 int phase_layout(const esp_ctx *c) {
   const esp::HostModel &m = c->hm;
   if (m.implicit && m.compressed && c->indexing == 0) return LAY_IMP;
   return m.compressed ? LAY_CMP : LAY_BOND;
 }
-size_t phase_shm(const esp_ctx *c) {
-  return phase_lds_bytes(phase_layout(c), c->hm.nb, c->hm.zmax, c->hm.rows_max);
+int phase_kernel_layout(const esp_ctx *c, int tps) {
+  const int lay = phase_layout(c);
+  return lay == LAY_IMP && !geo_tiles(c->hm, tps) ? LAY_CMP : lay;
 }
 
 // Wide chunks (more gathers in flight per lane, more registers) when one colour phase of all
 // replicas has too few waves to hide memory latency by occupancy: < 4 waves per SIMD.
 PhaseFn phase_fn(int mode, const esp_ctx *c, int64_t lanes_per_launch) {
   const bool wide = lanes_per_launch < 4 * 1024 * 64;
-  const int lay = phase_layout(c);
+  const int lay = phase_kernel_layout(c, mode == M_HOSTFED ? 1 : c->tps);
   return wide ? phase_fn_ch<kChunkWide>(mode, lay, c->hm) : phase_fn_ch<kChunk>(mode, lay, c->hm);
 }
 template <int MODE, bool CMP, bool HB, bool HD>
@@ -148,10 +150,11 @@ int check_ready(esp_ctx *c, bool need_replicas) {
 // Called before any capture, never inside one.
 int ensure_mpart(esp_ctx *c) {
   const esp::HostModel &m = c->hm;
+  const bool geo = phase_kernel_layout(c, c->tps) == LAY_IMP;
   int need = 1;
-  for (int col = 0; col < m.ncol; ++col)
-    need = std::max(need, ((m.col_off[col + 1] - m.col_off[col]) * c->tps + 63) / 64);
-  if (c->d_mpart && c->d_w && need == c->mpart_nw) return ESP_OK;
+  for (int col = 0; col < m.ncol; ++col)   // (host-fed sweeps take one lane per site)
+    need = std::max({need, colour_waves(m, col, c->tps, geo), colour_waves(m, col, 1, phase_kernel_layout(c, 1) == LAY_IMP)});
+  if (c->d_mpart && c->d_w && need == c->mpart_nw && geo == c->mpart_geo && c->tps == c->mpart_tps) return ESP_OK;
   drop_graph(c);   // a captured round may hold the old buffers
   if (c->d_w && c->mpart_nw > 0) {
     hipLaunchKernelGGL(k_fold_w, dim3((c->R + 255) / 256), dim3(256), 0, c->stream, c->d_w,
@@ -167,6 +170,8 @@ int ensure_mpart(esp_ctx *c) {
   HIPCHK(c, hipMemsetAsync(c->d_w, 0, n * sizeof(double), c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->mpart_nw = need;
+  c->mpart_geo = geo;
+  c->mpart_tps = c->tps;
   c->mpart_valid = false;
   return ESP_OK;
 }
@@ -182,12 +187,14 @@ KArgs phase_args(esp_ctx *c, double tilt, uint64_t seed) {
   return a;
 }
 
-// Colour `col` of `a` (block count for the lanes per site).
-void set_colour(KArgs &a, const esp::HostModel &m, int col) {
+// Colour `col` of `a` (block count for the lanes per site, or the geometry-group tiles).
+void set_colour(KArgs &a, const esp::HostModel &m, int col, int lay) {
   a.col = col;
   a.c_begin = m.col_off[col];
   a.c_count = m.col_off[col + 1] - m.col_off[col];
-  a.nblk = (a.c_count * a.tps + kBlock - 1) / kBlock;
+  a.nblk = colour_blocks(m, col, a.tps, lay == LAY_IMP);
+  a.dnblk = espg::make_fastdiv((uint32_t)std::max(1, a.nblk));
+  if (lay == LAY_IMP) a.dngc = geo_ngc(m, col);
 }
 
 // Enqueue `nsweeps` sweeps starting at clock->sweep + off0 (global-memory path).
@@ -199,13 +206,14 @@ int enqueue_phase_sweeps(esp_ctx *c, int mode, double tilt, uint64_t seed, int n
   const esp::HostModel &m = c->hm;
   KArgs a = phase_args(c, tilt, seed);
   PhaseFn fn = phase_fn(mode, c, launch_lanes(c));
-  const size_t shm = phase_shm(c);
+  const int lay = phase_kernel_layout(c, c->tps);
+  const size_t shm = phase_lds_bytes(lay, m.nb, m.zmax);
   for (int s = 0; s < nsweeps; ++s)
     for (int col = 0; col < m.ncol; ++col) {
-      set_colour(a, m, col);
+      set_colour(a, m, col, lay);
       if (a.c_count == 0) continue;
       a.sweep_off = off0 + s;
-      hipLaunchKernelGGL(fn, dim3(a.nblk * c->R), dim3(kBlock), shm, c->stream, a);
+      hipLaunchKernelGGL(fn, dim3(a.nblk * c->R), dim3(kPhaseBlock), shm, c->stream, a);
     }
   HIPCHK(c, hipGetLastError());
   if (nsweeps > 0) c->mpart_valid = a.mpart != nullptr;
@@ -452,7 +460,6 @@ int esp_set_model(esp_ctx *c, int N, int nb, const double *mag, int zJ, const in
     hm.ctab.clear();
     hm.implicit = false;
   }
-  if (hm.implicit && phase_lds_bytes(LAY_IMP, hm.nb, hm.zmax, hm.rows_max) > 49152) hm.implicit = false;
   if ((size_t)hm.zmax * N * sizeof(int) >= (1ull << 32) || (size_t)(N + 64) * 8 >= (1ull << 32))
     return fail(c, ESP_EINVAL, "bond table or replica beyond 4 GiB (32-bit device offsets)");
   free_replicas(c);
@@ -469,10 +476,12 @@ int esp_set_model(esp_ctx *c, int N, int nb, const double *mag, int zJ, const in
   if ((rc = upload(c, c->d_basis, m.basis))) return rc;
   if ((rc = upload(c, c->d_si4, m.si4))) return rc;
   if ((rc = upload(c, c->d_h4, m.h4))) return rc;
-  if (m.implicit) {
-    if ((rc = upload(c, c->d_grp, m.grp))) return rc;
-    if ((rc = upload(c, c->d_gslot, m.gslot))) return rc;
-    if ((rc = upload(c, c->d_magb, m.magb))) return rc;
+  if (m.implicit && m.compressed) {
+    const esp::SegTables t = esp::segment_tables(m);
+    if ((rc = upload(c, c->d_grp, m.grp)) || (rc = upload(c, c->d_gcnt, t.cnt)) ||
+        (rc = upload(c, c->d_gbond, t.bond)) || (rc = upload(c, c->d_gcoef, t.coef)))
+      return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
   }
   if (m.compressed) {
     if ((rc = upload(c, c->d_ctab, m.ctab))) return rc;
@@ -527,8 +536,7 @@ int esp_plan_model(int N, int nb, const double *mag, int zJ, const int *j_cnt, c
   std::memcpy(colour, hm.colour.data(), sizeof(int) * N);
   if (info) {
     const bool imp = hm.implicit && hm.compressed &&
-                     (size_t)hm.nb * hm.zmax * 5 * sizeof(double) <= 32768 &&
-                     phase_lds_bytes(LAY_IMP, hm.nb, hm.zmax, hm.rows_max) <= 49152;
+                     (size_t)hm.nb * hm.zmax * 5 * sizeof(double) <= 32768;
     info[0] = hm.N; info[1] = hm.zmax; info[2] = hm.ncol;
     info[3] = hm.compressed ? (imp ? LAY_IMP : LAY_CMP) : LAY_BOND;
     info[4] = 0;
@@ -743,15 +751,13 @@ int esp_sweep_hostfed(esp_ctx *c, const double *prop, const double *unif, uint8_
   c->mpart_valid = false;
   PhaseFn fn = phase_fn(M_HOSTFED, c, launch_lanes(c));
   if ((rc = set_clock(c, 0, 0, 1))) return rc;
+  a.tps = 1;
+  a.xcd_remap = (c->R % 8 == 0);
+  const int lay = phase_kernel_layout(c, 1);
   for (int col = 0; col < m.ncol; ++col) {
-    a.col = col;
-    a.c_begin = m.col_off[col];
-    a.c_count = m.col_off[col + 1] - m.col_off[col];
+    set_colour(a, m, col, lay);
     if (!a.c_count) continue;
-    a.tps = 1;
-    a.nblk = (a.c_count + kBlock - 1) / kBlock;
-    a.xcd_remap = (c->R % 8 == 0);
-    hipLaunchKernelGGL(fn, dim3(a.nblk * c->R), dim3(kBlock), phase_shm(c), c->stream, a);
+    hipLaunchKernelGGL(fn, dim3(a.nblk * c->R), dim3(kPhaseBlock), phase_lds_bytes(lay, m.nb, m.zmax), c->stream, a);
   }
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(accepted, c->d_accd, n, hipMemcpyDeviceToHost, c->stream));
@@ -855,14 +861,15 @@ int esp_time_sweeps(esp_ctx *c, int nsweeps, int mode, double tilt, uint64_t see
   } else {
     KArgs a = phase_args(c, tilt, seed);
     PhaseFn fn = phase_fn(mode, c, launch_lanes(c));
-    const size_t shm = phase_shm(c);
+    const int lay = phase_kernel_layout(c, c->tps);
+    const size_t shm = phase_lds_bytes(lay, m.nb, m.zmax);
     for (int sw = 0; sw < nsweeps; ++sw)
       for (int col = 0; col < m.ncol; ++col) {
-        set_colour(a, m, col);
+        set_colour(a, m, col, lay);
         if (a.c_count == 0) continue;
         a.sweep_off = sw;
         // start/stop stamped by the dispatch packet itself
-        hipExtLaunchKernelGGL(fn, dim3(a.nblk * c->R), dim3(kBlock), shm, c->stream, ev[2 * k],
+        hipExtLaunchKernelGGL(fn, dim3(a.nblk * c->R), dim3(kPhaseBlock), shm, c->stream, ev[2 * k],
                               ev[2 * k + 1], 0, a);
         ++k;
       }

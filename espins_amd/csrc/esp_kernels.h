@@ -16,6 +16,7 @@
 
 #include "esp_device.h"
 #include "esp_geo.h"
+#include "esp_model.h"
 
 namespace espk {
 struct Clock {                   // device-side schedule counters (graph-replayable)
@@ -28,16 +29,18 @@ struct Clock {                   // device-side schedule counters (graph-replaya
 namespace {  // internal linkage: each translation unit that launches these owns its copies
 using namespace espd;
 
-constexpr int kBlock = 256;      // phase / reduce kernels (4 waves)
+constexpr int kBlock = 256;      // reduce and measurement kernels (4 waves)
+constexpr int kPhaseBlock = 256; // colour-phase kernels (64 and 512 measured the same, 1024 slower)
 constexpr int kLdsBlock = 512;   // LDS-resident kernel (8 waves per replica)
 // Tuning constants (compile-time; the defaults are the measured best on MI355X).  Fewer
 // gathers in flight per lane means fewer registers and more waves per SIMD, which hides the
-// gather latency better than a wide chunk does.
+// gather latency better than a wide chunk does: FCC 32^3 x 64, us per step with 2 / 3 / 4 in
+// flight: 361 / 335 / 363; FCC 16^3 x 64 (two waves per SIMD) with 4 / 6 / 8: 139 / 133 / 150.
 #ifndef ESP_CHUNK
-#define ESP_CHUNK 2
+#define ESP_CHUNK 3
 #endif
 #ifndef ESP_CHUNK_WIDE
-#define ESP_CHUNK_WIDE 4
+#define ESP_CHUNK_WIDE 6
 #endif
 #ifndef ESP_PHASE_WAVES
 #define ESP_PHASE_WAVES 0        // > 0: ask the compiler for this many waves per SIMD
@@ -54,11 +57,12 @@ constexpr int kChunkLds = 8;     // ... in the LDS-resident sweep
 #define ESP_CHUNK_LEARN 8
 #endif
 constexpr int kChunkLearn = ESP_CHUNK_LEARN;  // ... in the learned sweep
-// Rejections are counted per slot in kRejSub sub-counters, rej[slot][kRejSub]: a wave adds
-// to the sub-counter its global wave index selects, so the thousands of waves of one replica
-// do not queue at one address (a single counter per slot cost 12-14 % of a colour phase).
-// Readers sum the sub-counters.
-constexpr int kRejSub = 16;
+// Rejections are counted per slot in kRejSub sub-counters, rej[kRejSub][R]: a wave adds to the
+// sub-counter its global wave index selects.  Atomics on one 128-byte line queue at about 30
+// cycles each, and a replica's waves run together on one XCD, so the sub-counters of a slot lie
+// on different lines: with 16 of them side by side in one line the queue bounded the sweep of
+// SC 64^3 x 32 (J + B + DM): 111 us per colour phase, 76 us so.  Readers sum the sub-counters.
+constexpr int kRejSub = 32;
 // Dynamic LDS of the LDS-resident kernel: [N+1 spins as double4][coefficient table]
 // [kLdsRed doubles of reduction scratch]; every byte of LDS it uses is in that one region.
 constexpr int kLdsRed = 4 * (512 / 64);
@@ -82,6 +86,7 @@ struct KArgs {
   uint8_t *accepted;
   int N, Ns, nb, zmax, R, ncol;
   int c_begin, c_count, nblk;
+  espg::FastDiv dnblk;           // by nblk
   int has_si, has_h, xcd_remap;
   int sweep_off, tps;            // tps: lanes cooperating on one site (1, 2, 4, 8)
   double tilt;
@@ -90,12 +95,15 @@ struct KArgs {
   // phase `col` overwrites its waves' entries
   double *mpart;
   int col, mpart_nw;
-  // implicit geometry (esp_geo.h), used by the global-memory colour phases when set
+  // implicit geometry (esp_geo.h): group records, bond lists and their coefficients (SegTables in
+  // esp_model.h); ngc geometry groups make up the colour, cut into tseg tiles of spt sites each, taken in runs
   espg::Geo geo;
-  const int *grp;                // [ngroups]
-  const int *gslot;              // [ngroups][zmax][2]
-  const double *magb;            // [nb]
-  int rows_max;                  // group rows one block stages in LDS
+  const int *grp, *gcnt;             // [ngroups]
+  const unsigned long long *gbond;   // [ngroups][zmax]
+  const double *gcoef;               // [ngroups][zmax][1 + has_B + 3 has_D]
+  int tseg, spt, run;
+  espg::FastDiv drun, dngc;
+  const espg::FastDiv *cngc;         // [ncol]: dngc of every colour (batched launches)
 };
 
 enum { M_RANDOM = 0, M_CONST = 1, M_HOSTFED = 2 };
@@ -127,6 +135,12 @@ __device__ __forceinline__ T ld_off(const T *base, unsigned byte_off) {
   return *(const ESP_GLOBAL T *)((const ESP_GLOBAL char *)base + byte_off);
 }
 
+// Scalar load of a wave-uniform element that the launch does not write.
+template <class T>
+__device__ __forceinline__ T cldi(const T *p, size_t i) {
+  return ((const __attribute__((address_space(4))) T *)p)[i];
+}
+
 struct GSpins {                  // one replica in global memory
   double *x, *y, *z;
   __device__ __forceinline__ V3 ld(unsigned j) const {
@@ -148,30 +162,14 @@ struct Proposal {
 };
 
 // What the update of one site needs besides the spins: device index, reference index (the
-// Philox counter and the host-fed arrays use it), basis atom and moment.  With the implicit
-// geometry they come from the device index and the group table in LDS (s_grp holds the rows
-// of groups g0..), else from the per-site tables.
+// Philox counter and the host-fed arrays use it), basis atom and moment.
 struct Site {
   int d, ir, a;
   double mag;
-  espg::SiteGeo sg;
 };
 
-template <bool IMP>
-__device__ __forceinline__ Site site_info(const KArgs &a, int d, const int *s_grp, int g0) {
-  Site s;
-  s.d = d;
-  if (IMP) {
-    s.sg = espg::geo_site(a.geo, s_grp - g0, d);
-    s.ir = s.sg.ir;
-    s.a = s.sg.a;
-    s.mag = gldi(a.magb, s.a);
-  } else {
-    s.ir = gldi(a.dev2ref, d);
-    s.a = gldi(a.basis, d);
-    s.mag = gldi(a.mag, d);
-  }
-  return s;
+__device__ __forceinline__ Site site_info(const KArgs &a, int d) {
+  return {d, gldi(a.dev2ref, d), gldi(a.basis, d), gldi(a.mag, d)};
 }
 
 // Proposal of one attempted update (identical on every lane of the site's group).
@@ -196,13 +194,25 @@ __device__ __forceinline__ Proposal propose(const KArgs &a, const SP &sp, const 
   return p;
 }
 
+// How a wave finds its sites' bonds: per-bond coefficient tables and the partner table; the
+// per-(basis, slot) coefficient table in LDS and the partner table; or, for a tile inside one
+// geometry group, the group's bond list (scalar loads) and computed partners.
+enum { LAY_BOND = 0, LAY_CMP = 1, LAY_IMP = 2 };
+
 // One bond's contribution to the J, B, D sums of delta_energy_get (get_quant.F90:288-336).
-template <bool CMP, bool HB, bool HD>
+// crow: the site's row of the coefficient table (LAY_CMP: in LDS; LAY_IMP: the group's list in
+// global memory, wave-uniform; unused with per-bond tables).
+template <int LAY, bool HB, bool HD>
 __device__ __forceinline__ void bond_term(const KArgs &a, const double *crow, int l, int d,
                                           const V3 &ds, const V3 &si, const V3 &sj, double &eJ,
                                           double &eB, double &eD) {
   double cj, cb = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
-  if (CMP) {
+  if (LAY == LAY_IMP) {
+    constexpr int NC = 1 + (HB ? 1 : 0) + (HD ? 3 : 0), oD = HB ? 2 : 1;
+    cj = cldi(crow, NC * l);
+    if (HB) cb = cldi(crow, NC * l + 1);
+    if (HD) { cx = cldi(crow, NC * l + oD); cy = cldi(crow, NC * l + oD + 1); cz = cldi(crow, NC * l + oD + 2); }
+  } else if (LAY == LAY_CMP) {
     cj = crow[5 * l];
     if (HB) cb = crow[5 * l + 1];
     if (HD) { cx = crow[5 * l + 2]; cy = crow[5 * l + 3]; cz = crow[5 * l + 4]; }
@@ -226,16 +236,16 @@ __device__ __forceinline__ void bond_term(const KArgs &a, const double *crow, in
 }
 
 // Partial bond sums over the slots l = g, g+tps, ... of site st.  Inactive lanes return
-// zeros.  Slots go in chunks of CH: the CH partner indices of the next chunk are loaded (or,
-// with the implicit geometry, computed from the (group, slot) rows staged in LDS at s_gs,
-// rows of groups g0..) while the current chunk's CH partner gathers are in flight, so a
+// zeros.  Slots go in chunks of CH: the CH partner indices of the next chunk are loaded
+// while the current chunk's CH partner gathers are in flight, so a
 // wave waits for one gather round trip per chunk.  Full chunks need no masks; only the last
 // partial chunk is masked (its spare lanes re-read slot g).  Padded slots point at the zero
 // spin (index N), so they need no test; a self bond (SELF) reads the new spin.
-template <int CH, bool CMP, bool HB, bool HD, bool SELF, bool IMP, class SP>
+template <int CH, bool CMP, bool HB, bool HD, bool SELF, class SP>
 __device__ __forceinline__ void bond_sums(const KArgs &a, const SP &sp, const double *ctab, const Site &st,
-                                          const int *s_gs, int g0, bool active, int g,
+                                          bool active, int g,
                                           const Proposal &p, double &eJ, double &eB, double &eD) {
+  constexpr int LAY = CMP ? LAY_CMP : LAY_BOND;
   eJ = 0.0; eB = 0.0; eD = 0.0;
   if (!active) return;
   const int d = st.d;
@@ -246,18 +256,12 @@ __device__ __forceinline__ void bond_sums(const KArgs &a, const SP &sp, const do
   const int nfull = nk - nk % CH;
   const double *crow = CMP ? ctab + (size_t)st.a * a.zmax * 5 : nullptr;
   const unsigned ud = (unsigned)d;
-  const int *grow = IMP ? s_gs + 2 * (st.sg.g - g0) * a.zmax : nullptr;
   unsigned jn[CH];   // partner indices of the next chunk
   auto load_idx = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       const int l = k0 + u < nk ? g + tps * (k0 + u) : g;
-      if (IMP) {
-        const int2 e = *reinterpret_cast<const int2 *>(grow + 2 * l);
-        jn[u] = (unsigned)espg::geo_partner(a.geo, st.sg, e.x, e.y);
-      } else {
-        jn[u] = (unsigned)ld_off(a.nbr, ((unsigned)l * (unsigned)a.N + ud) * 4u);
-      }
+      jn[u] = (unsigned)ld_off(a.nbr, ((unsigned)l * (unsigned)a.N + ud) * 4u);
     }
   };
   if (nk > 0) load_idx(0);
@@ -270,7 +274,7 @@ __device__ __forceinline__ void bond_sums(const KArgs &a, const SP &sp, const do
     }
     if (k0 + CH < nk) load_idx(k0 + CH);
 #pragma unroll
-    for (int u = 0; u < CH; ++u) bond_term<CMP, HB, HD>(a, crow, g + tps * (k0 + u), d, ds, si, sv[u], eJ, eB, eD);
+    for (int u = 0; u < CH; ++u) bond_term<LAY, HB, HD>(a, crow, g + tps * (k0 + u), d, ds, si, sv[u], eJ, eB, eD);
   }
   const int rem = nk - nfull;
   if (rem > 0) {
@@ -282,7 +286,61 @@ __device__ __forceinline__ void bond_sums(const KArgs &a, const SP &sp, const do
     }
 #pragma unroll
     for (int u = 0; u < CH; ++u)
-      if (u < rem) bond_term<CMP, HB, HD>(a, crow, g + tps * (nfull + u), d, ds, si, sv[u], eJ, eB, eD);
+      if (u < rem) bond_term<LAY, HB, HD>(a, crow, g + tps * (nfull + u), d, ds, si, sv[u], eJ, eB, eD);
+  }
+}
+
+// The bond sums of a site of geometry group sg.g over the group's bond list (one lane per site;
+// the group is the same for the whole wave).  The list is sorted by the partners' sub-cell
+// shift, so a lane wraps its sub-cell coordinates once per distinct shift (at most 8 for nearest
+// and next-nearest shells on a colouring of period 2) and a bond adds the partner group's first
+// index: about 1 + 13 x 8 / z vector instructions per partner index, against 25 when every lane
+// unpacked each slot's shift from a table in LDS.  Coefficients come as scalar loads, not LDS
+// reads.  Lists hold real bonds only, no padding.
+template <int CH, bool HB, bool HD, bool SELF>
+__device__ __forceinline__ void bond_sums_geo(const KArgs &a, const GSpins &sp, const espg::SiteGeo &sg, const Site &st,
+                                              const Proposal &p, double &eJ, double &eB, double &eD) {
+  eJ = 0.0; eB = 0.0; eD = 0.0;
+  const V3 ds = sub(p.sn, p.so);
+  const V3 si = sub(p.sn, ds);  // old spin as the reference recovers it (get_quant.F90:306,320)
+  constexpr int NC = 1 + (HB ? 1 : 0) + (HD ? 3 : 0);
+  const int n = cldi(a.gcnt, sg.g);
+  const unsigned long long *bl = a.gbond + (size_t)sg.g * a.zmax;
+  const double *crow = a.gcoef + (size_t)sg.g * a.zmax * NC;
+  const unsigned ud = (unsigned)st.d;
+  const int nfull = n - n % CH;
+  unsigned jn[CH], off = 0;
+  auto load_idx = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const unsigned long long e = cldi(bl, min(k0 + u, n - 1));
+      const unsigned q = (unsigned)(e >> 32);
+      if (q >> 31) off = (unsigned)espg::geo_shift(a.geo, sg, q);   // a new shift
+      jn[u] = off + (unsigned)e;
+    }
+  };
+  if (n > 0) load_idx(0);
+  for (int k0 = 0; k0 < nfull; k0 += CH) {
+    V3 sv[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const V3 t = sp.ld(jn[u]);
+      sv[u] = (SELF && jn[u] == ud) ? p.sn : t;
+    }
+    if (k0 + CH < n) load_idx(k0 + CH);
+#pragma unroll
+    for (int u = 0; u < CH; ++u) bond_term<LAY_IMP, HB, HD>(a, crow, k0 + u, 0, ds, si, sv[u], eJ, eB, eD);
+  }
+  if (n > nfull) {
+    V3 sv[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const V3 t = sp.ld(jn[u]);
+      sv[u] = (SELF && jn[u] == ud) ? p.sn : t;
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+      if (nfull + u < n) bond_term<LAY_IMP, HB, HD>(a, crow, nfull + u, 0, ds, si, sv[u], eJ, eB, eD);
   }
 }
 
@@ -292,28 +350,28 @@ __device__ __forceinline__ double group_sum(double v, int tps) {
   return v;
 }
 
-__device__ __forceinline__ void rej_add(unsigned long long *rej, int slot, unsigned long long n) {
-  const unsigned wv = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kRejSub - 1);
-  gadd(&rej[(size_t)slot * kRejSub + wv], n);
+__device__ __forceinline__ void rej_add(unsigned long long *rej, int R, int slot, unsigned long long n) {
+  // blocks of one replica are 8 apart (one XCD)
+  const unsigned wv = ((blockIdx.x >> 3) * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (kRejSub - 1);
+  gadd(&rej[(size_t)wv * R + slot], n);
 }
 
 // Local terms and the accept test of metropolis (get_quant.F90:166-178): reject iff
-// dE > 0 and exp(-beta dE) < u3.  Returns dE through *de.
+// dE > 0 and exp(-beta dE) < u3.  Returns dE through *de.  UNI: the basis atom b is the same for
+// the whole wave (scalar loads).
+template <bool UNI = false>
 __device__ __forceinline__ bool decide(const KArgs &a, int b, const Proposal &p, double eJ,
                                        double eB, double eD, double beta, double *de_out) {
   const V3 ds = sub(p.sn, p.so);
   const V3 si = sub(p.sn, ds);
   double de = eJ;
+  auto ld4 = [&](const double *t, int k) { return UNI ? cldi(t, 4 * (size_t)b + k) : gldi(t, 4 * (size_t)b + k); };
   if (a.has_h) {
-    const size_t q = 4 * (size_t)b;
-    const double h0 = gldi(a.h4, q), h1 = gldi(a.h4, q + 1), h2 = gldi(a.h4, q + 2),
-                 h3 = gldi(a.h4, q + 3);
+    const double h0 = ld4(a.h4, 0), h1 = ld4(a.h4, 1), h2 = ld4(a.h4, 2), h3 = ld4(a.h4, 3);
     de = de + h0 * (ds.x * h1 + ds.y * h2 + ds.z * h3);
   }
   if (a.has_si) {
-    const size_t q = 4 * (size_t)b;
-    const double k0 = gldi(a.si4, q), k1 = gldi(a.si4, q + 1), k2 = gldi(a.si4, q + 2),
-                 k3 = gldi(a.si4, q + 3);
+    const double k0 = ld4(a.si4, 0), k1 = ld4(a.si4, 1), k2 = ld4(a.si4, 2), k3 = ld4(a.si4, 3);
     const double sa = si.x * k1 + si.y * k2 + si.z * k3;
     const double dsa = ds.x * k1 + ds.y * k2 + ds.z * k3;
     de = de + k0 * (dsa * dsa + 2.0 * sa * dsa);
@@ -325,109 +383,91 @@ __device__ __forceinline__ bool decide(const KArgs &a, int b, const Proposal &p,
 }
 
 __device__ __forceinline__ void decode_block(const KArgs &a, int &r, int &b) {
-  const int L = blockIdx.x;
-  if (a.xcd_remap) {  // blocks go round-robin over the 8 XCDs: keep a replica on one XCD/L2
-    const int x = L & 7, q = L >> 3;
-    r = x + 8 * (q / a.nblk);
-    b = q % a.nblk;
-  } else {
-    r = L / a.nblk;
-    b = L % a.nblk;
-  }
+  // blocks go round-robin over the 8 XCDs: keep a replica on one XCD/L2
+  const unsigned L = blockIdx.x, q = a.xcd_remap ? L >> 3 : L, w = espg::fdiv(q, a.dnblk);
+  b = (int)(q - w * a.dnblk.d);
+  r = (int)(a.xcd_remap ? (L & 7u) + 8u * w : w);
 }
 
-// Sum over the 64 lanes of a wave with DPP lane moves (no LDS traffic): pairs, quads, half
-// rows, rows, then rows 0+1 into row 1 and rows 0..2 into row 3; lane 63 ends with the total,
-// which readlane makes wave-uniform.  Every lane must be active.  The order of the additions
-// is fixed, so the result is reproducible.
-template <int CTRL, int ROW_MASK>
+// Lane moves of a double without LDS traffic: DPP within a row of 16 lanes, and the sum of a
+// value with its neighbour row's / half wave's (v_permlane16_swap, v_permlane32_swap).
+template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
   const int2 h = __builtin_bit_cast(int2, v);
-  int2 r;
-  r.x = __builtin_amdgcn_update_dpp(0, h.x, CTRL, ROW_MASK, 0xf, false);
-  r.y = __builtin_amdgcn_update_dpp(0, h.y, CTRL, ROW_MASK, 0xf, false);
-  return __builtin_bit_cast(double, r);
+  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_mov_dpp(h.x, CTRL, 0xf, 0xf, true),
+                                              __builtin_amdgcn_mov_dpp(h.y, CTRL, 0xf, 0xf, true)));
 }
-__device__ __forceinline__ double wave_total(double v) {
-  v += dpp_f64<0xb1, 0xf>(v);    // quad_perm [1,0,3,2]
-  v += dpp_f64<0x4e, 0xf>(v);    // quad_perm [2,3,0,1]
-  v += dpp_f64<0x141, 0xf>(v);   // row_half_mirror
-  v += dpp_f64<0x140, 0xf>(v);   // row_mirror
-  v += dpp_f64<0x142, 0xa>(v);   // row_bcast:15 into rows 1, 3
-  v += dpp_f64<0x143, 0xc>(v);   // row_bcast:31 into rows 2, 3
+__device__ __forceinline__ double add_rows(double v) {
   const int2 h = __builtin_bit_cast(int2, v);
-  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(h.x, 63),
-                                              __builtin_amdgcn_readlane(h.y, 63)));
+  const auto x = __builtin_amdgcn_permlane16_swap(h.x, h.x, false, false);
+  const auto y = __builtin_amdgcn_permlane16_swap(h.y, h.y, false, false);
+  return __builtin_bit_cast(double, make_int2(x[0], y[0])) + __builtin_bit_cast(double, make_int2(x[1], y[1]));
+}
+__device__ __forceinline__ double add_halves(double v) {
+  const int2 h = __builtin_bit_cast(int2, v);
+  const auto x = __builtin_amdgcn_permlane32_swap(h.x, h.x, false, false);
+  const auto y = __builtin_amdgcn_permlane32_swap(h.y, h.y, false, false);
+  return __builtin_bit_cast(double, make_int2(x[0], y[0])) + __builtin_bit_cast(double, make_int2(x[1], y[1]));
+}
+
+// Sums of four values over the 64 lanes of a wave (every lane active): lane l returns the total
+// of value {w, x, y, z}[l & 3].  The first two steps halve the number of values a lane carries
+// (it keeps one half and hands the other to its neighbour), so the whole takes 7 additions
+// instead of 24 -- with one butterfly per value the reduction was a seventh of a colour phase's
+// vector instructions.  The order of the additions is fixed, so the result is reproducible.
+__device__ __forceinline__ double wave_total4(double w, double x, double y, double z) {
+  const bool odd = threadIdx.x & 1, hi = threadIdx.x & 2;
+  const double p = (odd ? x : w) + dpp_f64<0xb1>(odd ? w : x);   // quad_perm [1,0,3,2]
+  const double q = (odd ? z : y) + dpp_f64<0xb1>(odd ? y : z);
+  double v = (hi ? q : p) + dpp_f64<0x4e>(hi ? p : q);           // quad_perm [2,3,0,1]
+  v += dpp_f64<0x124>(v);                                        // row_ror:4
+  v += dpp_f64<0x128>(v);                                        // row_ror:8
+  return add_halves(add_rows(v));
 }
 
 // Per-wave sums of one colour phase: the accepted dE (added to the wave's accumulator, which
 // the running energy sums) and the spins after the phase (stored; a site changes only in its
 // own colour phase, so after a sweep these add up to the replica's magnetisation and the
-// measurement reads them instead of every spin).  Fixed butterflies, one writer per entry.
-// The dE sum is added with a no-return atomic (one per wave and phase, so the order of the
-// additions to an entry is that of the launches): the wave does not wait for a read.
-__device__ __forceinline__ void wave_sums(const KArgs &a, int r, int b, bool owner, bool rej, double de,
-                                          const Proposal &p, int tps) {
-  double w = owner && !rej ? de : 0.0;
+// measurement reads them instead of every spin).  Fixed butterflies, one writer per entry: the
+// wave loads its accumulator at its start (wave_old, latency hidden) and stores the sum.
+// e: the wave's entry of its colour; a wave without an entry (past the colour's last lane) passes
+// own = false.
+__device__ __forceinline__ double wave_old(const KArgs &a, int r, int e, bool own) {
+  return own ? gldi(a.w, ((size_t)r * a.ncol + a.col) * a.mpart_nw + e) : 0.0;
+}
+__device__ __forceinline__ void wave_sums(const KArgs &a, int r, int e, bool own, bool owner, bool rej, double de,
+                                          const Proposal &p, double wold) {
   V3 sf = {0.0, 0.0, 0.0};
   if (owner) sf = rej ? p.so : p.sn;
-  w = wave_total(w);
-  if (a.mpart) {
-    sf.x = wave_total(sf.x);
-    sf.y = wave_total(sf.y);
-    sf.z = wave_total(sf.z);
-  }
-  // waves past the colour's last lane own no entry (mpart_nw counts the colour's waves)
-  const int wave = (b * kBlock + threadIdx.x) >> 6;
-  if ((threadIdx.x & 63) == 0 && wave * 64 < a.c_count * tps) {
-    const size_t e = ((size_t)r * a.ncol + a.col) * a.mpart_nw + wave;
-    if (w != 0.0) gadd(a.w + e, w);
-    if (a.mpart) {
-      gsti(a.mpart, e * 3, sf.x); gsti(a.mpart, e * 3 + 1, sf.y); gsti(a.mpart, e * 3 + 2, sf.z);
+  const double t = wave_total4(owner && !rej ? de : 0.0, sf.x, sf.y, sf.z);
+  const int lane = threadIdx.x & 63;
+  if (own && lane < 4) {
+    const size_t i = ((size_t)r * a.ncol + a.col) * a.mpart_nw + e;
+    if (lane == 0) {
+      gsti(a.w, i, wold + t);
+    } else if (a.mpart) {
+      gsti(a.mpart, i * 3 + (lane - 1), t);
     }
   }
 }
 
-// Coefficient layouts of the colour phases: per-bond tables, per-(basis, slot) table in LDS,
-// or the per-(basis, slot) table plus the implicit geometry (no per-site tables read).
-enum { LAY_BOND = 0, LAY_CMP = 1, LAY_IMP = 2 };
-
-// Dynamic LDS of a colour-phase block: [coefficient table][group rows][group records].
-__host__ __device__ inline size_t phase_lds_bytes(int lay, int nb, int zmax, int rows_max) {
-  size_t n = lay >= LAY_CMP ? (size_t)nb * zmax * 5 * sizeof(double) : 0;
-  if (lay == LAY_IMP) n += (size_t)rows_max * zmax * 2 * sizeof(int) + (size_t)rows_max * sizeof(int);
-  return n;
+// Dynamic LDS of a colour-phase block: the coefficient table.
+__host__ __device__ inline size_t phase_lds_bytes(int lay, int nb, int zmax) {
+  return lay == LAY_CMP ? (size_t)nb * zmax * 5 * sizeof(double) : 0;
 }
 
-// Block b of colour phase (a.c_begin, a.c_count) of replica r (global-memory path);
+// Block b of colour phase (a.c_begin, a.c_count) of replica r (global-memory path, tables);
 // a.tps lanes per site.  Shared by the single-context and the batched kernels.
-template <int MODE, int LAY, bool HB, bool HD, bool SELF, int CH = kChunk>
-__device__ __forceinline__ void phase_body(const KArgs &a, int r, int b, double *s_ctab) {
-  constexpr bool CMP = LAY >= LAY_CMP, IMP = LAY == LAY_IMP;
+template <int MODE, bool CMP, bool HB, bool HD, bool SELF, int CH>
+__device__ __forceinline__ void phase_tab(const KArgs &a, int r, int b, double *s_ctab) {
   const int tps = a.tps;
-  const int per = kBlock / tps;                        // sites of this block
-  int g0 = 0;
-  int *s_gs = nullptr, *s_grp = nullptr;
   if (CMP) {
     const int n = a.nb * a.zmax * 5;
-    for (int k = threadIdx.x; k < n; k += kBlock) s_ctab[k] = gldi(a.ctab, k);
+    for (int k = threadIdx.x; k < n; k += kPhaseBlock) s_ctab[k] = gldi(a.ctab, k);
+    __syncthreads();
   }
-  if (IMP) {   // (group, slot) rows and group records of the groups this block's sites lie in
-    const int first = a.c_begin + b * per;
-    const int last = min(a.c_begin + a.c_count, first + per) - 1;
-    const int mt = (int)a.geo.mt.d;
-    g0 = first / mt;
-    const int nrow = last / mt - g0 + 1;
-    s_gs = reinterpret_cast<int *>(s_ctab + a.nb * a.zmax * 5);
-    s_grp = s_gs + 2 * a.rows_max * a.zmax;
-    const int n = 2 * nrow * a.zmax;
-    const int *src = a.gslot + (size_t)2 * g0 * a.zmax;
-    for (int k = threadIdx.x; k < n; k += kBlock) s_gs[k] = gldi(src, k);
-    for (int k = threadIdx.x; k < nrow; k += kBlock) s_grp[k] = gldi(a.grp, g0 + k);
-  }
-  if (CMP) __syncthreads();
   const int g = threadIdx.x & (tps - 1);
-  const int k = (b * kBlock + threadIdx.x) / tps;
+  const int k = (b * kPhaseBlock + threadIdx.x) / tps;
   const bool active = k < a.c_count;
   const int d = a.c_begin + (active ? k : 0);
   const int slot = gldi(a.rep_slot, r);
@@ -435,12 +475,14 @@ __device__ __forceinline__ void phase_body(const KArgs &a, int r, int b, double 
   const unsigned long long sweep = gldi(&a.clock->sweep, 0) + (unsigned long long)a.sweep_off;
   double *base = a.sp + (size_t)r * 3 * a.Ns;
   const GSpins sp{base, base + a.Ns, base + 2 * a.Ns};
-  // inactive lanes of a block sit on its first site, which lies in row g0
-  const Site st = site_info<IMP>(a, active ? d : a.c_begin + b * per, s_grp, g0);
+  const Site st = site_info(a, d);
+  const int wave = (b * kPhaseBlock + threadIdx.x) >> 6;
+  const bool own = wave * 64 < a.c_count * tps;
+  const double wold = wave_old(a, r, wave, own);
   Proposal p{};
   if (active) p = propose<MODE>(a, sp, st, r, sweep);
   double eJ, eB, eD;
-  bond_sums<CH, CMP, HB, HD, SELF, IMP>(a, sp, s_ctab, st, s_gs, g0, active, g, p, eJ, eB, eD);
+  bond_sums<CH, CMP, HB, HD, SELF>(a, sp, s_ctab, st, active, g, p, eJ, eB, eD);
   eJ = group_sum(eJ, tps);
   if (HB) eB = group_sum(eB, tps);
   if (HD) eD = group_sum(eD, tps);
@@ -454,13 +496,65 @@ __device__ __forceinline__ void phase_body(const KArgs &a, int r, int b, double 
     }
   }
   const unsigned long long m = __ballot(rej && g == 0);
-  if ((threadIdx.x & 63) == 0 && m) rej_add(a.rej, slot, (unsigned long long)__popcll(m));
-  wave_sums(a, r, b, active && g == 0, rej, de, p, tps);
+  if ((threadIdx.x & 63) == 0 && m) rej_add(a.rej, a.R, slot, (unsigned long long)__popcll(m));
+  wave_sums(a, r, wave, own, active && g == 0, rej, de, p, wold);
+}
+
+// The same for a model with the implicit geometry, one lane per site: every wave takes one tile
+// of at most 64 sites of one geometry group, so the group, its bond list, coefficients, basis
+// atom, moment and local terms are wave-uniform (scalar loads) and nothing goes through LDS.
+// The waves of a block take a run of up to `run` consecutive tiles of one group (their partners
+// overlap in L1), consecutive runs the same place of the colour's next group, which is the same
+// region of the lattice (its lines are in the XCD's L2).
+// FCC 32^3 J1-J2 + B x 64 replicas (1 M updates per launch): 50 us with shifts and coefficients in
+// LDS, 42 us so (25 G updates/s, 5.4 TB/s of minimal colour-phase traffic from the memory-side
+// cache, which bounds it); SC 64^3 J + B + DM x 32 (4.2 M): 117 -> 76 us (55 G/s).
+template <int MODE, bool HB, bool HD, bool SELF, int CH>
+__device__ __forceinline__ void phase_geo(const KArgs &a, int r, int b) {
+  const int t = __builtin_amdgcn_readfirstlane(b * (kPhaseBlock / 64) + (int)(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int mt = (int)a.geo.mt.d;
+  const int q = (int)espg::fdiv((uint32_t)t, a.drun), cb = (int)espg::fdiv((uint32_t)q, a.dngc);
+  const int gi = q - cb * (int)a.dngc.d;
+  const int ch = cb * a.run + (t - q * a.run);              // tile of group gi of the colour
+  if (ch >= a.tseg) return;                                 // a spare wave of a run
+  const int first = a.c_begin + gi * mt;                    // the group's first site
+  const int gg = (int)espg::fdiv((uint32_t)first, a.geo.mt);
+  const int k = ch * a.spt + lane;                          // place inside the group
+  const bool active = lane < a.spt && k < mt;
+  const int slot = cldi(a.rep_slot, r);
+  const double beta = cldi(a.beta_slot, slot);
+  const unsigned long long sweep = cldi(&a.clock->sweep, 0) + (unsigned long long)a.sweep_off;
+  double *base = a.sp + (size_t)r * 3 * a.Ns;
+  const GSpins sp{base, base + a.Ns, base + 2 * a.Ns};
+  const espg::SiteGeo sg = espg::geo_place(a.geo, cldi(a.grp, gg), gg, active ? k : ch * a.spt);
+  const Site st{first + (active ? k : ch * a.spt), sg.ir, sg.a, cldi(a.mag, first)};
+  const double wold = wave_old(a, r, gi * a.tseg + ch, true);
+  Proposal p{};
+  bool rej = false;
+  double de = 0.0;
+  if (active) {
+    p = propose<MODE>(a, sp, st, r, sweep);
+    double eJ, eB, eD;
+    bond_sums_geo<CH, HB, HD, SELF>(a, sp, sg, st, p, eJ, eB, eD);
+    rej = decide<true>(a, st.a, p, eJ, eB, eD, beta, &de);
+    if (MODE == M_HOSTFED) gsti(a.accepted, (size_t)r * a.N + st.ir, (uint8_t)(rej ? 0 : 1));
+    if (!rej) sp.st(st.d, p.sn);
+  }
+  const unsigned long long m = __ballot(rej);
+  if (lane == 0 && m) rej_add(a.rej, a.R, slot, (unsigned long long)__popcll(m));
+  wave_sums(a, r, gi * a.tseg + ch, true, active, rej, de, p, wold);
+}
+
+template <int MODE, int LAY, bool HB, bool HD, bool SELF, int CH = kChunk>
+__device__ __forceinline__ void phase_body(const KArgs &a, int r, int b, double *s_ctab) {
+  if (LAY == LAY_IMP) phase_geo<MODE, HB, HD, SELF, CH>(a, r, b);
+  else phase_tab<MODE, LAY == LAY_CMP, HB, HD, SELF, CH>(a, r, b, s_ctab);
 }
 
 // One colour phase over every replica of one context.
 template <int MODE, int LAY, bool HB, bool HD, bool SELF, int CH>
-__global__ __launch_bounds__(kBlock) ESP_PHASE_ATTR void k_phase(KArgs a) {
+__global__ __launch_bounds__(kPhaseBlock) ESP_PHASE_ATTR void k_phase(KArgs a) {
   extern __shared__ double s_ctab[];
   int r, b;
   decode_block(a, r, b);
@@ -524,11 +618,11 @@ __device__ __forceinline__ void lds_body(const KArgs &a, int r, int nsweeps, con
         const int d0 = base + threadIdx.x / tps;
         const bool active = d0 < end;
         const int d = active ? d0 : beg;
-        const Site st = site_info<false>(a, d, nullptr, 0);
+        const Site st = site_info(a, d);
         Proposal p{};
         if (active) p = propose<MODE>(a, sp, st, r, sweep);
         double eJ, eB, eD;
-        bond_sums<kChunkLds, CMP, HB, HD, SELF, false>(a, sp, ctab, st, nullptr, 0, active, g, p, eJ, eB, eD);
+        bond_sums<kChunkLds, CMP, HB, HD, SELF>(a, sp, ctab, st, active, g, p, eJ, eB, eD);
         eJ = group_sum(eJ, tps);
         if (HB) eB = group_sum(eB, tps);
         if (HD) eD = group_sum(eD, tps);
@@ -588,7 +682,7 @@ __device__ __forceinline__ void lds_body(const KArgs &a, int r, int nsweeps, con
   }
   unsigned long long v = nrej;
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  if ((threadIdx.x & 63) == 0 && v) rej_add(a.rej, slot, v);
+  if ((threadIdx.x & 63) == 0 && v) rej_add(a.rej, a.R, slot, v);
 }
 
 template <int MODE, bool CMP, bool HB, bool HD, bool SELF>
@@ -853,13 +947,48 @@ __global__ void k_fill(double *p, size_t n, double v) {
   if (t < n) p[t] = v;
 }
 
-// Per-slot totals of the rejection sub-counters rej[slot][kRejSub] (host side).
+// Per-slot totals of the rejection sub-counters rej[kRejSub][R] (host side).
 inline void sum_rej_sub(const std::vector<int64_t> &sub, int R, int64_t *out) {
   for (int s = 0; s < R; ++s) {
     int64_t t = 0;
-    for (int k = 0; k < kRejSub; ++k) t += sub[(size_t)s * kRejSub + k];
+    for (int k = 0; k < kRejSub; ++k) t += sub[(size_t)k * R + s];
     out[s] = t;
   }
+}
+
+// Geometry-group tiles of a colour (host): a group's sites in tseg tiles of at most 64, evenly.
+// Worth it from 16 sites per group; below, most lanes of a tile would idle and the tables win.
+constexpr int kGeoMinSites = 16;
+inline bool geo_tiles(const esp::HostModel &m, int tps) {
+  return m.implicit && m.compressed && tps == 1 && (int)m.geo.mt.d >= kGeoMinSites;
+}
+inline int geo_tseg(const esp::HostModel &m) { return ((int)m.geo.mt.d + 63) / 64; }
+inline void geo_args(KArgs &a, const esp::HostModel &m) {
+  constexpr int kW = kPhaseBlock / 64;
+  a.tseg = geo_tseg(m);
+  a.spt = ((int)m.geo.mt.d + a.tseg - 1) / a.tseg;
+  const int runs = (a.tseg + kW - 1) / kW;
+  a.run = (a.tseg + runs - 1) / runs;
+  a.drun = espg::make_fastdiv((uint32_t)a.run);
+}
+inline espg::FastDiv geo_ngc(const esp::HostModel &m, int col) {   // groups of the colour
+  return espg::make_fastdiv((uint32_t)((m.col_off[col + 1] - m.col_off[col]) / (int)m.geo.mt.d));
+}
+// Entries of the per-wave sums of one colour phase of one replica.
+inline int colour_waves(const esp::HostModel &m, int col, int tps, bool geo) {
+  const int n = m.col_off[col + 1] - m.col_off[col];
+  return geo ? n / (int)m.geo.mt.d * geo_tseg(m) : (n * tps + 63) / 64;
+}
+// Its blocks.
+inline int colour_blocks(const esp::HostModel &m, int col, int tps, bool geo) {
+  constexpr int kW = kPhaseBlock / 64;
+  int waves = colour_waves(m, col, tps, geo);
+  if (geo) {
+    KArgs a{};
+    geo_args(a, m);
+    waves = waves / a.tseg * ((a.tseg + a.run - 1) / a.run) * a.run;
+  }
+  return (waves + kW - 1) / kW;
 }
 
 }  // namespace

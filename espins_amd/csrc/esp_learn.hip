@@ -483,6 +483,9 @@ __global__ __launch_bounds__(kBlock) ESP_LEARN_ATTR void k_phase_learned(KArgs a
   const unsigned long long sweep = a.clock->sweep + (unsigned long long)a.sweep_off;
   double *base = a.sp + (size_t)r * 3 * a.Ns;
   const GSpins sp{base, base + a.Ns, base + 2 * a.Ns};
+  const int wave = (b * kBlock + threadIdx.x) >> 6;
+  const bool own = wave * 64 < a.c_count;
+  const double wold = wave_old(a, r, wave, own);
   V3 G;
   double QB[6];
   local_env<CMP, HB, HD>(a, sp, ctab, d, G, QB);
@@ -528,10 +531,10 @@ __global__ __launch_bounds__(kBlock) ESP_LEARN_ATTR void k_phase_learned(KArgs a
     sp.x[d] = sn.x; sp.y[d] = sn.y; sp.z[d] = sn.z;
   }
   const unsigned long long m = __ballot(active && !acc);
-  if ((threadIdx.x & 63) == 0 && m) rej_add(a.rej, slot, (unsigned long long)__popcll(m));
+  if ((threadIdx.x & 63) == 0 && m) rej_add(a.rej, a.R, slot, (unsigned long long)__popcll(m));
   Proposal pr;
   pr.so = so; pr.sn = sn; pr.u3 = 0.0;
-  wave_sums(a, r, b, active, !acc, dE, pr, 1);   // accepted dE into the wave's accumulator
+  wave_sums(a, r, wave, own, active, !acc, dE, pr, wold);   // accepted dE into the wave's accumulator
 }
 
 // Records of local conditionals: n random (replica, site) pairs of the current state.
@@ -869,6 +872,7 @@ int learn_enqueue_sweeps(esp_ctx *c, uint64_t seed, int nsweeps, int off0, hipEv
       a.c_count = m.col_off[col + 1] - m.col_off[col];
       if (a.c_count == 0) continue;
       a.nblk = (a.c_count + kBlock - 1) / kBlock;
+      a.dnblk = espg::make_fastdiv((uint32_t)a.nblk);
       a.xcd_remap = (c->R % 8 == 0) ? 1 : 0;
       a.sweep_off = off0 + s;
       if (ev)

@@ -409,8 +409,6 @@ void build_implicit(HostModel &hm, const int L[3], const int P[3], const double 
       if (espg::geo_partner(G, sg, e[0], e[1]) != hm.nbr[(size_t)l * N + d]) return;
     }
   }
-  // groups touched by the sites of one 256-lane block (one lane per site at most)
-  hm.rows_max = (int)std::min<long>(ngroups, (256 - 1) / mt + 2);
   hm.implicit = true;
 }
 }  // namespace
@@ -597,6 +595,38 @@ std::string prepare_model(HostModel &hm, int N, int nb, const double *mag, int z
     build_implicit(hm, Lc, P, mb.data());
   }
   return "";
+}
+
+SegTables segment_tables(const HostModel &hm) {
+  const int ng = hm.geo.ngroups, zp = hm.zmax, nc = 1 + (hm.has_B ? 1 : 0) + (hm.has_D ? 3 : 0);
+  SegTables t;
+  t.cnt.assign(ng, 0);
+  t.bond.assign((size_t)ng * zp, 0);
+  t.coef.assign((size_t)ng * zp * nc, 0.0);
+  std::vector<int> order;
+  for (int g = 0; g < ng; ++g) {
+    const int *gs = &hm.gslot[(size_t)g * zp * 2];
+    order.clear();
+    for (int l = 0; l < zp; ++l)
+      if (gs[2 * l] >= 0) order.push_back(l);
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return gs[2 * x + 1] < gs[2 * y + 1]; });
+    t.cnt[g] = (int)order.size();
+    for (size_t k = 0; k < order.size(); ++k) {
+      const int l = order[k];
+      const bool fresh = k == 0 || gs[2 * order[k - 1] + 1] != gs[2 * l + 1];
+      t.bond[(size_t)g * zp + k] = (unsigned long long)(unsigned)gs[2 * l] |
+                                   (unsigned long long)(unsigned)gs[2 * l + 1] << 32 |
+                                   (fresh ? 1ull << 63 : 0ull);
+      const double *c = &hm.ctab[((size_t)(hm.grp[g] & 0xff) * zp + l) * kCoef];
+      double *o = &t.coef[((size_t)g * zp + k) * nc];
+      int at = 0;
+      o[at++] = c[0];
+      if (hm.has_B) o[at++] = c[1];
+      if (hm.has_D)
+        for (int q = 2; q < 5; ++q) o[at++] = c[q];
+    }
+  }
+  return t;
 }
 
 uint64_t structure_hash(int N, int nb, int zJ, const int *j_cnt, const int *j_nbr, int zB,

@@ -42,8 +42,17 @@ struct HostModel {
   std::vector<int> grp;         // [ngroups] packed basis atom and residue
   std::vector<int> gslot;       // [ngroups][zmax][2]: partner group start, packed shift
   std::vector<double> magb;     // [nb] moment of each basis atom
-  int rows_max = 0;             // groups one 256-lane block of a colour phase can touch
 };
+
+// Bond lists of the geometry groups as the colour phases read them: per group its real bonds,
+// sorted by the partners' sub-cell shift (slot order inside a shift).
+struct SegTables {
+  std::vector<int> cnt;                 // [ngroups]
+  std::vector<unsigned long long> bond; // [ngroups][zmax]: first device index of the partner group,
+                                        // shift << 32, bit 63 where the shift differs from the one before
+  std::vector<double> coef;             // [ngroups][zmax][1 + has_B + 3 has_D]
+};
+SegTables segment_tables(const HostModel &hm);
 
 // Build the device-ready model from reference-layout tables.  Returns "" on success,
 // else an error message.
