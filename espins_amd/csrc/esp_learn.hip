@@ -35,7 +35,6 @@ constexpr int oW1 = 0, oB1 = oW1 + kH * kIn, oW2 = oB1 + kH, oB2 = oW2 + kH * kH
               oB3 = oW3 + kH * kH, oW4 = oB3 + kH, oB4 = oW4 + kOut * kH, kNP = oB4 + kOut;
 static_assert(kNP == ESP_LEARN_NPARAMS, "parameter count");
 constexpr int kRec = 16;   // record: x[5], kappa0, ghat[3], axis[3], s[3], pad
-constexpr int kTrainBlock = 128;
 constexpr double kPi = 3.14159265358979323846;
 // Weight of a fixed uniform-sphere component beside the two network components: the density
 // of any direction stays >= kUniform / (4 pi), so a poorly fitted network slows the chain by
@@ -572,64 +571,123 @@ __global__ __launch_bounds__(kBlock) void k_collect(KArgs a, int n, uint32_t s0,
   rec[15] = (float)((size_t)r * a.N + a.dev2ref[d]);  // replica * N + site (exact below 2^24)
 }
 
-// Per-block gradient of the mean negative log-likelihood over records [off, off + n):
-// each thread runs one record forward and backward; the block then sums the parameter
-// gradients over its records in a fixed order (deterministic).
 // Unit vector stored at rec[o..o+2] (records hold FP32; renormalised in FP64).
 __device__ __forceinline__ V3 rec_vec(const float *rec, int o) {
   return vnorm(V3{(double)rec[o], (double)rec[o + 1], (double)rec[o + 2]});
 }
 
-__global__ __launch_bounds__(kTrainBlock) void k_train_block(const float *w, const float *recs, int n,
-                                                             const int *perm, int off, float *part_grad,
-                                                             double *part_loss) {
-  extern __shared__ float s_tr[];
-  // per record (one thread): a0[5] a1[32] a2[32] a3[32] | g4[6] d3[32] d2[32] d1[32]; the
-  // delta slots hold the pre-activations z_l until the backward pass overwrites them
-  constexpr int kA = kIn + 3 * kH, kD = kOut + 3 * kH, kS = kA + kD;
-  float *my = s_tr + threadIdx.x * kS;  // odd stride: lanes hit distinct banks
-  float *a0 = my, *a1 = a0 + kIn, *a2 = a1 + kH, *a3 = a2 + kH;
-  float *g4 = my + kA, *d3 = g4 + kOut, *d2 = d3 + kH, *d1 = d2 + kH;
-  __shared__ double s_loss[kTrainBlock];
-  const int i = blockIdx.x * kTrainBlock + threadIdx.x;
+// ---- training: gradient of the mean negative log-likelihood ------------------------------------
+// One wave takes tiles of 32 records through the network on the matrix cores in FP32
+// (v_mfma_f32_32x32x2_f32): a 32 x 32 layer of 32 records is 16 instructions.  Operand layouts
+// (lane l, half h = l / 32): A[i = l % 32][k = h], B[k = h][j = l % 32], D register v =
+// D[8 (v / 4) + 4 h + v % 4][l % 32].  The order of the products in k is free, so step (q, r) =
+// v pairs k = 8 q + r (half 0) with k = 8 q + 4 + r (half 1): the B operand of a layer is then the
+// lane's own D register v of the layer before (forward and backward alike), with no exchange, and
+// the weights' A operand is W[l % 32][8 q + 4 h + r] (forward) or W[8 q + 4 h + r][l % 32]
+// (backward).  The weight gradients, sums over records of delta x activation, take both factors
+// with lane = unit and register = record, through a transposition in LDS, and accumulate in D
+// registers over the wave's tiles.  One thread per record and a sum over the records of a
+// block per parameter took 185 us for a minibatch of 2048 (16 blocks, a serial chain of 7200
+// multiply-adds per thread through LDS); 20 us so.
+constexpr int kTile = 32;             // records of a tile
+constexpr int kTrainWaves = 512;      // waves of a gradient at most (more tiles: several per wave)
+constexpr int kTrow = kTile + 1;      // LDS row of one unit's values over the tile's records
+
+__device__ __forceinline__ int d_unit(int v, int h) { return 8 * (v >> 2) + 4 * h + (v & 3); }
+
+// D = W B + C over 32 units with A = w[16] and B = b (D layout).
+__device__ __forceinline__ floatx16 mat32(const float (&w)[16], const floatx16 &b, floatx16 c) {
+#pragma unroll
+  for (int v = 0; v < 16; ++v) c = __builtin_amdgcn_mfma_f32_32x32x2f32(w[v], b[v], c, 0, 0, 0);
+  return c;
+}
+
+// x (D layout: lane = record) into LDS rows [unit][record].
+__device__ __forceinline__ void put_rows(float *t, const floatx16 &x, int l, int h) {
+#pragma unroll
+  for (int v = 0; v < 16; ++v) t[d_unit(v, h) * kTrow + l] = x[v];
+}
+
+// C += sum over the tile's records of left[unit i][rec] right[unit c][rec], both LDS rows; *bias
+// += this lane's half of sum over records of left[l].
+__device__ __forceinline__ floatx16 outer32(const float *left, const float *right, int l, int h, floatx16 c, float *bias) {
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    const float x = left[l * kTrow + 2 * s + h], y = right[l * kTrow + 2 * s + h];
+    if (bias) *bias += x;
+    c = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, c, 0, 0, 0);
+  }
+  return c;
+}
+
+__global__ __launch_bounds__(64) void k_train_tiles(const float *w, const float *recs, int n, const int *perm, int off,
+                                                    float *part_grad, double *part_loss) {
+  __shared__ float s_w4[kOut * kH + kOut];
+  __shared__ float s_l[kH * kTrow], s_r[kH * kTrow];
+  const int lane = threadIdx.x, l = lane & 31, h = lane >> 5;
+  for (int k = lane; k < kOut * kH + kOut; k += 64) s_w4[k] = w[oW4 + k];
+  float w1[3], w2[16], w3[16], w2t[16], w3t[16];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) w1[s] = 2 * s + h < kIn ? w[oW1 + l * kIn + 2 * s + h] : 0.f;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int k = d_unit(v, h);
+    w2[v] = w[oW2 + l * kH + k];
+    w3[v] = w[oW3 + l * kH + k];
+    w2t[v] = w[oW2 + k * kH + l];
+    w3t[v] = w[oW3 + k * kH + l];
+  }
+  floatx16 dw1{}, dw2{}, dw3{}, dw4{};
+  float db2 = 0.f, db3 = 0.f, db4 = 0.f;
   double loss = 0.0;
-  if (i < n) {
-    const float *rec = recs + (size_t)(perm ? perm[off + i] : off + i) * kRec;
-    for (int k = 0; k < kIn; ++k) a0[k] = rec[k];
-    for (int q = 0; q < kH; ++q) {
-      float z = w[oB1 + q];
-      for (int k = 0; k < kIn; ++k) z += w[oW1 + q * kIn + k] * a0[k];
-      d1[q] = z;
-      a1[q] = act(z);
-    }
-    for (int q = 0; q < kH; ++q) {
-      float z = w[oB2 + q];
-      for (int k = 0; k < kH; ++k) z += w[oW2 + q * kH + k] * a1[k];
-      d2[q] = z;
-      a2[q] = act(z);
-    }
-    for (int q = 0; q < kH; ++q) {
-      float z = w[oB3 + q];
-      for (int k = 0; k < kH; ++k) z += w[oW3 + q * kH + k] * a2[k];
-      d3[q] = z;
-      a3[q] = act(z);
-    }
-    float o[kOut];
-    for (int q = 0; q < kOut; ++q) {
-      float z = w[oB4 + q];
-      for (int k = 0; k < kH; ++k) z += w[oW4 + q * kH + k] * a3[k];
-      o[q] = z;
+  __syncthreads();
+  const int tiles = (n + kTile - 1) / kTile;
+  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const int i = t * kTile + l;
+    const bool on = i < n;
+    const float *rec = recs + (size_t)(perm ? perm[off + (on ? i : 0)] : off + (on ? i : 0)) * kRec;
+    float x[kIn + 1];
+#pragma unroll
+    for (int k = 0; k < kIn; ++k) x[k] = rec[k];
+    x[kIn] = 0.f;
+    floatx16 z, a1, a2, a3, g1, g2, g3;   // activations and their derivatives
+#pragma unroll
+    for (int v = 0; v < 16; ++v) z[v] = w[oB1 + d_unit(v, h)];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+      z = __builtin_amdgcn_mfma_f32_32x32x2f32(w1[s], h ? x[2 * s + 1] : x[2 * s], z, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) { a1[v] = act(z[v]); g1[v] = act_d(z[v]); }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) z[v] = w[oB2 + d_unit(v, h)];
+    z = mat32(w2, a1, z);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) { a2[v] = act(z[v]); g2[v] = act_d(z[v]); }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) z[v] = w[oB3 + d_unit(v, h)];
+    z = mat32(w3, a2, z);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) { a3[v] = act(z[v]); g3[v] = act_d(z[v]); }
+    float o[kOut], g4[kOut];
+#pragma unroll
+    for (int q = 0; q < kOut; ++q) {      // this half's units, then the partner's
+      float acc = 0.f;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc += s_w4[q * kH + d_unit(v, h)] * a3[v];
+      o[q] = s_w4[kOut * kH + q] + (acc + __shfl_xor(acc, 32, 64));
     }
     const V3 ghat = rec_vec(rec, 6), ax = rec_vec(rec, 9), s = rec_vec(rec, 12);
     const Mix m = make_mix(o, rec[5], ghat, ax);
     double lv[2];
+#pragma unroll
     for (int k = 0; k < 2; ++k) lv[k] = m.logw[k] + log_vmf(m, k, s);
     const double mx = fmax(fmax(lv[0], lv[1]), kLogUni);
     const double lse = mx + log(exp(lv[0] - mx) + exp(lv[1] - mx) + exp(kLogUni - mx));
-    loss = -lse;
+    if (on && h == 0) loss -= lse;
     const double rnet = exp(lv[0] - lse) + exp(lv[1] - lse);  // responsibility of the network part
     // d loss / d outputs
     const V3 e = tilt_frame(ghat, ax);
+#pragma unroll
     for (int k = 0; k < 2; ++k) {
       const double rk = exp(lv[k] - lse);      // responsibility of component k
       const double kap = m.kappa[k];
@@ -638,93 +696,129 @@ __global__ __launch_bounds__(kTrainBlock) void k_train_block(const float *w, con
       const double dks = (sraw > -8.0 && sraw < 8.0) ? (kap - 1e-6) : 0.0;              // d kappa / d o
       g4[3 * k] = (float)(-rk * dlk * dks);
       g4[3 * k + 1] = (float)(exp(m.logw[k] - kLog1mU) * rnet - rk);
-      const double t = m.t[k];
-      const double th = t / (0.5 * kPi);
-      const V3 dmu = {-sin(t) * ghat.x + cos(t) * e.x, -sin(t) * ghat.y + cos(t) * e.y,
-                      -sin(t) * ghat.z + cos(t) * e.z};
+      const double tt = m.t[k];
+      const double th = tt / (0.5 * kPi);
+      const V3 dmu = {-sin(tt) * ghat.x + cos(tt) * e.x, -sin(tt) * ghat.y + cos(tt) * e.y,
+                      -sin(tt) * ghat.z + cos(tt) * e.z};
       g4[3 * k + 2] = (float)(-rk * kap * dot(dmu, s) * 0.5 * kPi * (1.0 - th * th));
     }
-    for (int k = 0; k < kH; ++k) {
+#pragma unroll
+    for (int q = 0; q < kOut; ++q) g4[q] = on ? g4[q] : 0.f;   // spare records add nothing
+    floatx16 d3, d2, d1;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
       float acc = 0.f;
-      for (int q = 0; q < kOut; ++q) acc += w[oW4 + q * kH + k] * g4[q];
-      d3[k] = acc * act_d(d3[k]);
+#pragma unroll
+      for (int q = 0; q < kOut; ++q) acc += s_w4[q * kH + d_unit(v, h)] * g4[q];
+      d3[v] = acc * g3[v];
     }
-    for (int k = 0; k < kH; ++k) {
-      float acc = 0.f;
-      for (int q = 0; q < kH; ++q) acc += w[oW3 + q * kH + k] * d3[q];
-      d2[k] = acc * act_d(d2[k]);
+    d2 = mat32(w3t, d3, floatx16{});
+#pragma unroll
+    for (int v = 0; v < 16; ++v) d2[v] *= g2[v];
+    d1 = mat32(w2t, d2, floatx16{});
+#pragma unroll
+    for (int v = 0; v < 16; ++v) d1[v] *= g1[v];
+    // weight gradients; rows of the right factor past its units are zero (one wave: LDS
+    // operations are in order, the barriers only keep the compiler from moving them)
+    auto rows = [&](const floatx16 &left, const floatx16 &right) {
+      __syncthreads();
+      put_rows(s_l, left, l, h);
+      put_rows(s_r, right, l, h);
+      __syncthreads();
+    };
+    rows(d3, a2);
+    dw3 = outer32(s_l, s_r, l, h, dw3, &db3);
+    rows(d2, a1);
+    dw2 = outer32(s_l, s_r, l, h, dw2, &db2);
+    __syncthreads();
+    put_rows(s_l, d1, l, h);
+    if (h == 0) {
+#pragma unroll
+      for (int k = 0; k < kIn; ++k) s_r[k * kTrow + l] = x[k];
+      s_r[kIn * kTrow + l] = 1.f;                               // column kIn: the bias
+    } else {
+      for (int k = kIn + 1; k < kH; ++k) s_r[k * kTrow + l] = 0.f;
     }
-    for (int k = 0; k < kH; ++k) {
-      float acc = 0.f;
-      for (int q = 0; q < kH; ++q) acc += w[oW2 + q * kH + k] * d2[q];
-      d1[k] = acc * act_d(d1[k]);
+    __syncthreads();
+    dw1 = outer32(s_l, s_r, l, h, dw1, nullptr);
+    __syncthreads();
+    put_rows(s_r, a3, l, h);
+    if (h == 0) {
+#pragma unroll
+      for (int q = 0; q < kOut; ++q) s_l[q * kTrow + l] = g4[q];
+    } else {
+      for (int q = kOut; q < kH; ++q) s_l[q * kTrow + l] = 0.f;
     }
-  } else {
-    for (int k = 0; k < kS; ++k) my[k] = 0.f;
+    __syncthreads();
+    dw4 = outer32(s_l, s_r, l, h, dw4, &db4);
   }
-  s_loss[threadIdx.x] = loss;
-  __syncthreads();
-  // parameter gradients: sum over the block's records in record order
-  for (int p = threadIdx.x; p < kNP; p += kTrainBlock) {
-    // layer l: weight gradient = delta_out[row] * act_in[col], bias gradient = delta_out[row]
-    int dout_off, ain_off, row, col = 0;
-    bool bias = false;
-    if (p < oB1) { row = p / kIn; col = p % kIn; dout_off = kA + kOut + 2 * kH; ain_off = 0; }
-    else if (p < oW2) { row = p - oB1; dout_off = kA + kOut + 2 * kH; ain_off = 0; bias = true; }
-    else if (p < oB2) { row = (p - oW2) / kH; col = (p - oW2) % kH; dout_off = kA + kOut + kH; ain_off = kIn; }
-    else if (p < oW3) { row = p - oB2; dout_off = kA + kOut + kH; ain_off = 0; bias = true; }
-    else if (p < oB3) { row = (p - oW3) / kH; col = (p - oW3) % kH; dout_off = kA + kOut; ain_off = kIn + kH; }
-    else if (p < oW4) { row = p - oB3; dout_off = kA + kOut; ain_off = 0; bias = true; }
-    else if (p < oB4) { row = (p - oW4) / kH; col = (p - oW4) % kH; dout_off = kA; ain_off = kIn + 2 * kH; }
-    else { row = p - oB4; dout_off = kA; ain_off = 0; bias = true; }
-    float g = 0.f;
-    for (int q = 0; q < kTrainBlock; ++q) {
-      const float *rq = s_tr + q * kS;
-      const float dq = rq[dout_off + row];
-      g += bias ? dq : dq * rq[ain_off + col];
-    }
-    part_grad[(size_t)blockIdx.x * kNP + p] = g;
+  db2 += __shfl_xor(db2, 32, 64);
+  db3 += __shfl_xor(db3, 32, 64);
+  db4 += __shfl_xor(db4, 32, 64);
+  float *g = part_grad + (size_t)blockIdx.x * kNP;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int i = d_unit(v, h);
+    g[oW2 + i * kH + l] = dw2[v];
+    g[oW3 + i * kH + l] = dw3[v];
+    if (l < kIn) g[oW1 + i * kIn + l] = dw1[v];
+    else if (l == kIn) g[oB1 + i] = dw1[v];
+    if (i < kOut) g[oW4 + i * kH + l] = dw4[v];
   }
-  if (threadIdx.x == 0) {
-    double sl = 0.0;
-    for (int q = 0; q < kTrainBlock; ++q) sl += s_loss[q];
-    part_loss[blockIdx.x] = sl;
+  if (h == 0) {
+    g[oB2 + l] = db2;
+    g[oB3 + l] = db3;
+    if (l < kOut) g[oB4 + l] = db4;
   }
-}
-
-__global__ void k_train_reduce(const float *part_grad, const double *part_loss, int nblk, int n,
-                               float *grad, double *loss) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < kNP) {
-    float g = 0.f;
-    for (int b = 0; b < nblk; ++b) g += part_grad[(size_t)b * kNP + p];
-    grad[p] = g / (float)n;
-  }
-  if (p == 0) {
-    double l = 0.0;
-    for (int b = 0; b < nblk; ++b) l += part_loss[b];
-    *loss = l / (double)n;
-  }
+  for (int q = 16; q > 0; q >>= 1) loss += __shfl_xor(loss, q, 64);   // lanes of half 1 hold zeros
+  if (lane == 0) part_loss[blockIdx.x] = loss;
 }
 
 // Adam on the FP32 master weights; writes the BF16 copy used by the sweep.
-__global__ void k_adam(float *w, float *mom, float *vel, const float *g, float lr, float b1, float b2,
-                       float eps, int t, uint16_t *wbf16) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= kNP) return;
-  const float gp = g[p];
-  const float m = b1 * mom[p] + (1.f - b1) * gp;
-  const float v = b2 * vel[p] + (1.f - b2) * gp * gp;
-  mom[p] = m;
-  vel[p] = v;
-  const float mh = m / (1.f - powf(b1, (float)t));
-  const float vh = v / (1.f - powf(b2, (float)t));
-  const float nw = w[p] - lr * mh / (sqrtf(vh) + eps);
-  w[p] = nw;
+struct AdamArgs {
+  float *w, *mom, *vel;
+  uint16_t *wbf16;
+  float lr, b1, b2, eps;
+  int t;                              // step, from 1; 0: gradient only
+};
+
+// Mean gradient and loss from the waves' partial sums (64 parameters per block, the partials in
+// four slices summed in order), then the Adam step of these parameters in the same launch.
+__global__ __launch_bounds__(256) void k_train_reduce(const float *part_grad, const double *part_loss, int nw, int n,
+                                                      float *grad, double *loss, AdamArgs ad) {
+  __shared__ float s[256];
+  const int p = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
+  float g = 0.f;
+  if (p < kNP) {
+    const int b0 = nw * slice / 4, b1 = nw * (slice + 1) / 4;
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) g += part_grad[(size_t)b * kNP + p];
+  }
+  s[threadIdx.x] = g;
+  __syncthreads();
+  if (blockIdx.x == 0 && threadIdx.x >= 64 && threadIdx.x < 128) {
+    double v = 0.0;
+    for (int b = threadIdx.x - 64; b < nw; b += 64) v += part_loss[b];
+    for (int q = 32; q > 0; q >>= 1) v += __shfl_xor(v, q, 64);
+    if (threadIdx.x == 64) *loss = v / (double)n;
+  }
+  if (slice != 0 || p >= kNP) return;
+  const int q = threadIdx.x;
+  const float gp = (s[q] + s[64 + q] + s[128 + q] + s[192 + q]) / (float)n;
+  grad[p] = gp;
+  if (ad.t == 0) return;
+  const float m = ad.b1 * ad.mom[p] + (1.f - ad.b1) * gp;
+  const float v = ad.b2 * ad.vel[p] + (1.f - ad.b2) * gp * gp;
+  ad.mom[p] = m;
+  ad.vel[p] = v;
+  const float mh = m / (1.f - powf(ad.b1, (float)ad.t));
+  const float vh = v / (1.f - powf(ad.b2, (float)ad.t));
+  const float nw_ = ad.w[p] - ad.lr * mh / (sqrtf(vh) + ad.eps);
+  ad.w[p] = nw_;
   // round to nearest even BF16
-  const uint32_t u = __float_as_uint(nw);
+  const uint32_t u = __float_as_uint(nw_);
   const uint32_t rb = ((u >> 16) & 1u) + 0x7FFFu;
-  wbf16[p] = (uint16_t)((u + rb) >> 16);
+  ad.wbf16[p] = (uint16_t)((u + rb) >> 16);
 }
 
 __global__ void k_to_bf16(const float *w, uint16_t *wbf16) {
@@ -817,33 +911,34 @@ int ensure_records(esp_ctx *c, int need) {
   return ESP_OK;
 }
 
-// Dynamic LDS of k_train_block: activations and deltas of every record of the block.
-constexpr size_t train_shmem() { return (size_t)kTrainBlock * (kIn + 3 * kH + kOut + 3 * kH) * sizeof(float); }
+// Waves of a gradient over n records.
+int train_waves(int n) { return std::min((n + kTile - 1) / kTile, kTrainWaves); }
 
 // Gradient scratch for minibatches of up to n records and up to nsteps losses.
 int ensure_grad_scratch(esp_ctx *c, int n, int nsteps) {
-  const int nblk = (n + kTrainBlock - 1) / kTrainBlock;
+  const int nw = train_waves(n);
   int rc;
-  if (nblk > c->pgrad_cap) {
-    if ((rc = dalloc(c, c->d_pgrad, (size_t)nblk * kNP)) || (rc = dalloc(c, c->d_ploss, nblk))) return rc;
-    c->pgrad_cap = nblk;
+  if (nw > c->pgrad_cap) {
+    c->pgrad_cap = 0;
+    if ((rc = dalloc(c, c->d_pgrad, (size_t)nw * kNP)) || (rc = dalloc(c, c->d_ploss, nw))) return rc;
+    c->pgrad_cap = nw;
   }
   if (nsteps > c->loss_cap) {
+    c->loss_cap = 0;
     if ((rc = dalloc(c, c->d_loss, nsteps))) return rc;
     c->loss_cap = nsteps;
   }
-  HIPCHK(c, hipFuncSetAttribute((const void *)k_train_block, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)train_shmem()));
   return ESP_OK;
 }
 
-// Gradient of the mean loss over records (perm ? perm[off + i] : off + i), i < n; loss to d_loss[k].
-int enqueue_grad(esp_ctx *c, const int *perm, int off, int n, int k) {
-  const int nblk = (n + kTrainBlock - 1) / kTrainBlock;
-  hipLaunchKernelGGL(k_train_block, dim3(nblk), dim3(kTrainBlock), train_shmem(), c->stream,
-                     (const float *)c->d_lw, (const float *)c->d_recs, n, perm, off, c->d_pgrad, c->d_ploss);
-  hipLaunchKernelGGL(k_train_reduce, dim3((kNP + 255) / 256), dim3(256), 0, c->stream, (const float *)c->d_pgrad,
-                     (const double *)c->d_ploss, nblk, n, c->d_grad, c->d_loss + k);
+// Gradient of the mean loss over records (perm ? perm[off + i] : off + i), i < n; loss to d_loss[k];
+// with ad.t > 0 also the Adam step.
+int enqueue_grad(esp_ctx *c, const int *perm, int off, int n, int k, const AdamArgs &ad) {
+  const int nw = train_waves(n);
+  hipLaunchKernelGGL(k_train_tiles, dim3(nw), dim3(64), 0, c->stream, (const float *)c->d_lw, (const float *)c->d_recs, n,
+                     perm, off, c->d_pgrad, c->d_ploss);
+  hipLaunchKernelGGL(k_train_reduce, dim3((kNP + 63) / 64), dim3(256), 0, c->stream, (const float *)c->d_pgrad,
+                     (const double *)c->d_ploss, nw, n, c->d_grad, c->d_loss + k, ad);
   HIPCHK(c, hipGetLastError());
   return ESP_OK;
 }
@@ -987,7 +1082,7 @@ int esp_learn_grad(esp_ctx *c, int first, int n, float *grad, double *loss) {
   if (!c->have_learn) return fail(c, ESP_ESTATE, "no proposal weights");
   if (!grad || !loss || first < 0 || n <= 0 || first + n > c->nrec) return fail(c, ESP_EINVAL, "record range");
   if ((rc = ensure_grad_scratch(c, n, 1))) return rc;
-  if ((rc = enqueue_grad(c, nullptr, first, n, 0))) return rc;
+  if ((rc = enqueue_grad(c, nullptr, first, n, 0, AdamArgs{}))) return rc;
   HIPCHK(c, hipMemcpyAsync(grad, c->d_grad, sizeof(float) * kNP, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(loss, c->d_loss, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1022,10 +1117,9 @@ int esp_learn_train(esp_ctx *c, int epochs, int batch, float lr, uint64_t seed, 
     HIPCHK(c, hipMemcpyAsync(c->d_perm, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
     for (int b = 0; b < nb; ++b) {
       const int off = b * batch, cnt = std::min(batch, n - off);
-      if ((rc = enqueue_grad(c, c->d_perm, off, cnt, b))) return rc;
       c->adam_t += 1;
-      hipLaunchKernelGGL(k_adam, dim3((kNP + 255) / 256), dim3(256), 0, c->stream, c->d_lw, c->d_lm, c->d_lv,
-                         (const float *)c->d_grad, lr, 0.9f, 0.999f, 1e-8f, c->adam_t, c->d_lbf);
+      const AdamArgs ad{c->d_lw, c->d_lm, c->d_lv, c->d_lbf, lr, 0.9f, 0.999f, 1e-8f, c->adam_t};
+      if ((rc = enqueue_grad(c, c->d_perm, off, cnt, b, ad))) return rc;
     }
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(losses.data(), c->d_loss, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
