@@ -13,11 +13,14 @@
 using espk::Clock;
 using espk::KArgs;
 
+struct esp_cluster;              // esp_cluster.hip
+
 struct esp_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
   size_t lds_max = 65536;
+  int num_cu = 0;
   int Lhint[3] = {0, 0, 0};       // supercell size for the periodic colouring
   int path = 0;                   // 0 auto, 1 global-memory phases, 2 LDS-resident
   uint32_t stream_base = 0;       // Philox stream of replica r: stream_base + r
@@ -51,6 +54,11 @@ struct esp_ctx {
   Clock *d_clock = nullptr;
   unsigned *d_done = nullptr;    // blocks of k_reduce_fin done this step (the last one resets it)
   std::vector<double> tems;
+  // replicas shared by clusters of blocks (esp_cluster.hip): tables, or null where clusters do not
+  // serve; decided for cluster_R replicas (0: not yet)
+  esp_cluster *cluster = nullptr;
+  int cluster_R = 0;
+  bool w_dirty = false;           // d_w may hold sums (the launch-per-colour path ran since a fold)
   // host-fed staging
   double *d_prop = nullptr, *d_unif = nullptr;
   uint8_t *d_accd = nullptr;
@@ -120,6 +128,14 @@ struct esp_ctx {
   std::string gkey;
 };
 
+namespace esp {
+// Clusters (esp_cluster.hip): decide and build tables once per (model, replicas); run; free.
+int cluster_prepare(esp_ctx *c);
+int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, int M, bool measure, bool exchange,
+                int round, int *ran);
+void cluster_free(esp_ctx *c);
+}  // namespace esp
+
 namespace {
 
 int fail(esp_ctx *c, int code, const std::string &msg) {
@@ -172,6 +188,7 @@ void free_replicas(esp_ctx *c) {
   dfree(c->d_nswap); dfree(c->d_nmeas); dfree(c->d_prop); dfree(c->d_unif); dfree(c->d_accd);
   dfree(c->d_trace);
   c->trace_cap = 0;
+  c->w_dirty = false;
   dfree(c->d_mpart);
   c->mpart_nw = 0;
   c->mpart_valid = false;
@@ -180,6 +197,7 @@ void free_replicas(esp_ctx *c) {
 }
 
 void free_model(esp_ctx *c) {
+  esp::cluster_free(c);
   dfree(c->d_nbr); dfree(c->d_dev2ref); dfree(c->d_ref2dev); dfree(c->d_col_off);
   dfree(c->d_cJ); dfree(c->d_cB); dfree(c->d_cD); dfree(c->d_ctab); dfree(c->d_mag);
   dfree(c->d_si4); dfree(c->d_h4); dfree(c->d_basis);

@@ -199,6 +199,7 @@ void set_colour(KArgs &a, const esp::HostModel &m, int col, int lay) {
 
 // Enqueue `nsweeps` sweeps starting at clock->sweep + off0 (global-memory path).
 int enqueue_phase_sweeps(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsweeps, int off0) {
+  c->w_dirty = true;
   if (mode == ESP_MODE_LEARNED) {
     c->mpart_valid = false;
     return esp::learn_enqueue_sweeps(c, seed, nsweeps, off0);
@@ -314,6 +315,7 @@ int rebase(esp_ctx *c) {
   if ((rc = enqueue_energy(c, c->d_ebase))) return rc;
   const size_t n = (size_t)c->R * c->hm.ncol * c->mpart_nw;
   hipLaunchKernelGGL(k_fill, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, c->d_w, n, 0.0);
+  c->w_dirty = false;
   c->mpart_valid = false;
   HIPCHK(c, hipMemcpyAsync(c->d_erun, c->d_ebase, sizeof(double) * c->R, hipMemcpyDeviceToDevice,
                            c->stream));
@@ -325,6 +327,31 @@ int rebase(esp_ctx *c) {
 // is recorded; learned proposals and traced runs use the global-memory path.
 bool lds_sweeps(const esp_ctx *c, int mode) {
   return c->use_lds && mode != ESP_MODE_LEARNED && !c->d_trace && !c->obs.flags;
+}
+
+// Clusters of blocks serve the plain proposals of the automatic path.  Replicas that one block
+// holds (k_lds) go to a cluster from kClusterMinSites sites per colour: below, a block's threads
+// all have one site anyway and the flags between blocks only add.
+constexpr int kClusterMinSites = 384;
+bool cluster_sweeps(const esp_ctx *c, int mode) {
+  if (c->path != 0 || c->tps_user || (mode != ESP_MODE_RANDOM && mode != ESP_MODE_CONST) || c->obs.flags) return false;
+  return !lds_sweeps(c, mode) || c->hm.N / std::max(1, c->hm.ncol) >= kClusterMinSites;
+}
+
+// The steps of a run on clusters, as far as they serve it: *ran of nsteps (from the device clock).
+int run_clusters(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, int M, bool measure, bool exchange,
+                 int round, int *ran) {
+  *ran = 0;
+  if (!cluster_sweeps(c, mode)) return ESP_OK;
+  int rc = esp::cluster_prepare(c);
+  if (rc || !c->cluster) return rc;
+  if (c->w_dirty) {          // the clusters count their accepted dE on top of e_base
+    hipLaunchKernelGGL(k_fold_w, dim3((c->R + 255) / 256), dim3(256), 0, c->stream, c->d_w,
+                       c->hm.ncol * c->mpart_nw, c->R, c->d_ebase);
+    HIPCHK(c, hipGetLastError());
+    c->w_dirty = false;
+  }
+  return esp::cluster_run(c, mode, tilt, seed, nsteps, M, measure, exchange, round, ran);
 }
 
 // One MC "round": steps x (M sweeps [+ measure]) [+ exchange]; advances the clock.
@@ -384,7 +411,10 @@ int esp_create(esp_ctx **out, int device) {
     return ESP_EHIP;
   }
   hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->lds_max = prop.sharedMemPerBlock;
+  if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
+    c->lds_max = prop.sharedMemPerBlock;
+    c->num_cu = prop.multiProcessorCount;
+  }
   if (hipMalloc((void **)&c->d_clock, sizeof(Clock)) != hipSuccess ||
       hipMalloc((void **)&c->d_done, sizeof(unsigned)) != hipSuccess ||
       hipMemset(c->d_done, 0, sizeof(unsigned)) != hipSuccess) {
@@ -641,6 +671,7 @@ int esp_set_replicas(esp_ctx *c, int R, const double *tems, const double *spins)
   HIPCHK(c, hipMemsetAsync(c->d_nswap, 0, sizeof(unsigned long long) * 2 * R, c->stream));
   HIPCHK(c, hipMemsetAsync(c->d_nmeas, 0, sizeof(unsigned long long), c->stream));
   if ((rc = esp::obs_resize(c))) return rc;
+  if (cluster_sweeps(c, ESP_MODE_RANDOM) && (rc = esp::cluster_prepare(c))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return esp_put_spins(c, spins);
 }
@@ -726,6 +757,9 @@ int esp_sweep(esp_ctx *c, int nsweeps, int mode, double tilt, uint64_t seed, uin
     return fail(c, ESP_EINVAL, "bad nsweeps / mode");
   if (nsweeps == 0) return ESP_OK;
   if ((rc = set_clock(c, sweep0, 0, 1))) return rc;
+  int ran = 0;
+  if ((rc = run_clusters(c, mode, tilt, seed, nsweeps, 1, false, false, 1, &ran))) return rc;
+  if ((nsweeps -= ran) == 0) return ESP_OK;      // (the device clock has moved on by ran)
   if (lds_sweeps(c, mode)) rc = enqueue_lds_sweeps(c, mode, tilt, seed, nsweeps, 0);
   else rc = enqueue_phase_sweeps(c, mode, tilt, seed, nsweeps, 0);
   if (rc) return rc;
@@ -749,6 +783,7 @@ int esp_sweep_hostfed(esp_ctx *c, const double *prop, const double *unif, uint8_
   KArgs a = base_args(c);   // one lane per site here: no per-wave sums
   a.prop = c->d_prop; a.unif = c->d_unif; a.accepted = c->d_accd;
   c->mpart_valid = false;
+  c->w_dirty = true;
   PhaseFn fn = phase_fn(M_HOSTFED, c, launch_lanes(c));
   if ((rc = set_clock(c, 0, 0, 1))) return rc;
   a.tps = 1;
@@ -796,6 +831,18 @@ int esp_run(esp_ctx *c, int n_rounds, int steps_per_round, int steps_measure, in
     return fail(c, ESP_EINVAL, "bad esp_run arguments");
   if (n_rounds == 0) return ESP_OK;
   if ((rc = set_clock(c, sweep0, step0, start_parity))) return rc;
+  if ((int64_t)n_rounds * steps_per_round < (1ll << 30)) {
+    int ran = 0;
+    if ((rc = run_clusters(c, mode, tilt, seed, n_rounds * steps_per_round, steps_measure, do_measure, do_exchange,
+                           do_exchange ? steps_per_round : 1, &ran)))
+      return rc;
+    if (ran == n_rounds * steps_per_round) return ESP_OK;
+    if (ran % steps_per_round) {     // (no exchanges: finish the round step by step)
+      for (; ran % steps_per_round; ++ran)
+        if ((rc = enqueue_round(c, 1, steps_measure, do_measure, false, mode, tilt, seed))) return rc;
+    }
+    n_rounds -= ran / steps_per_round;
+  }
   if (!use_graph) {
     for (int k = 0; k < n_rounds; ++k) {
       rc = enqueue_round(c, steps_per_round, steps_measure, do_measure, do_exchange, mode, tilt, seed);
@@ -823,6 +870,7 @@ int esp_run(esp_ctx *c, int n_rounds, int steps_per_round, int steps_measure, in
     }
     c->gkey = key;
   }
+  c->w_dirty = true;
   for (int k = 0; k < n_rounds; ++k) HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return ESP_OK;
@@ -838,6 +886,7 @@ int esp_time_sweeps(esp_ctx *c, int nsweeps, int mode, double tilt, uint64_t see
   if ((rc = set_clock(c, sweep0, 0, 1))) return rc;
   const esp::HostModel &m = c->hm;
   const bool lds = lds_sweeps(c, mode);
+  c->w_dirty = true;
   // one event pair around every sweep-kernel launch, on the context's stream
   const int per = lds ? 1 : nsweeps * m.ncol;
   std::vector<hipEvent_t> ev(2 * per, nullptr);
