@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <vector>
 
 #include "esp_ctx.h"
@@ -37,6 +38,7 @@ constexpr int kSfRep = 8;             // replicas per structure-factor wave (sin
 constexpr int kSfRepLat = 4;          // replicas per structure-factor wave (lattice path)
 constexpr int kSfWaves = 4096;        // structure-factor waves aimed at (site chunks fill up to it)
 constexpr int kSfMaxChunks = 64;
+constexpr size_t kSfPlaneBytes = size_t(256) << 20;   // plane sums held at a time (lattice path)
 constexpr int kPmLdsBins = 12288;     // P(m) bins counted in LDS (48 KiB); more use global atomics
 
 struct ObsArgs {
@@ -63,8 +65,11 @@ struct ObsArgs {
   double *sfspin, *sfpart;
   int sf_chunk, sf_nchunk;
   // lattice positions r = B_a + x0 A0 + x1 A1 + x2 A2 (reference order ((x2 L1 + x1) L0 + x0) nb
-  // + a): phase tables exp(i q.x0 A0), exp(i q.x1 A1), exp(i q.x2 A2), exp(i q.B_a), [k][q] each
+  // + a): phase tables exp(i q.x0 A0), exp(i q.x1 A1) by distinct pair (q.A0, q.A1), [x][pair], and
+  // exp(i q.x2 A2), exp(i q.B_a), [k][q]; sfpair: the pair of each q-point
   int sf_lat, sfL[3], sf_rep;         // sf_rep: replicas per group of the packed spins
+  int npq, sf_g0;                     // pairs; first replica group of the launch
+  const int *sfpair;
   const double2 *sfex, *sfey, *sfez, *sfeb;
   double *sf;
   unsigned long long *sfn;
@@ -108,14 +113,24 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_cells(ObsArgs o) {
     if (c >= o.ncell) break;
     V3 m = {0.0, 0.0, 0.0}, st = {0.0, 0.0, 0.0};
     double op = 0.0;
-    for (int a = 0; a < o.nb; ++a) {
-      const int d = gldi(o.cdev, (size_t)a * o.ncell + c);
-      const V3 s = spin_at(o, r, d);
-      m.x += s.x; m.y += s.y; m.z += s.z;
-      if (OP) op += s.x * gldi(o.axes, 3 * a) + s.y * gldi(o.axes, 3 * a + 1) + s.z * gldi(o.axes, 3 * a + 2);
-      if (SM) {
-        const double w = gldi(o.coeff, a);
-        st.x += w * s.x; st.y += w * s.y; st.z += w * s.z;
+    for (int a0 = 0; a0 < o.nb; a0 += 4) {       // four atoms' loads in flight together
+      int d[4];
+      V3 sp[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d[k] = gldi(o.cdev, (size_t)min(a0 + k, o.nb - 1) * o.ncell + c);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) sp[k] = spin_at(o, r, d[k]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int a = a0 + k;
+        if (a >= o.nb) break;
+        const V3 s = sp[k];
+        m.x += s.x; m.y += s.y; m.z += s.z;
+        if (OP) op += s.x * cldi(o.axes, 3 * a) + s.y * cldi(o.axes, 3 * a + 1) + s.z * cldi(o.axes, 3 * a + 2);
+        if (SM) {
+          const double w = cldi(o.coeff, a);
+          st.x += w * s.x; st.y += w * s.y; st.z += w * s.z;
+        }
       }
     }
     v[0] += op; v[1] += st.x; v[2] += st.y; v[3] += st.z;
@@ -151,8 +166,10 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_cells(ObsArgs o) {
 // j (device index, its kind in the top two bits) and the weights of i -> j and, when the
 // shell is symmetric, of j -> i (both directions of the bond from one gather); shell s has
 // rows soff[s] .. soff[s+1]-1.  A bond costs coalesced table loads shared by the REP
-// replicas and one spin gather per replica.  (Keeping a replica group on one
+// replicas and one spin gather per replica; rows go in groups of kRows, whose table loads and then
+// gathers are in flight together (one round trip per group instead of per row).  (Keeping a replica group on one
 // XCD, as the sweep does, measured slower here: 468 against 404 us on FCC 32^3 x 64.)
+constexpr int kRows = 3;
 template <int NS, int REP>
 __global__ __launch_bounds__(kObsBlock) void k_obs_spincorr(ObsArgs o) {
   constexpr int NV = 2 * NS * NS * REP;
@@ -179,23 +196,36 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_spincorr(ObsArgs o) {
 #pragma unroll
       for (int y = 0; y < NS; ++y) { v[u][0][y] = v[u][1][y] = vr[u][0][y] = vr[u][1][y] = 0.0; }
     const int l1 = gldi(o.soff, s + 1);
-    for (int l = gldi(o.soff, s); l < l1; ++l) {
-      const unsigned e = gldi(o.sbond, (size_t)l * o.N + d);
-      const double w = gldi(o.sw, (size_t)l * o.N + d);
-      const double wr = NS > 1 ? gldi(o.sw, ((size_t)o.srows + l) * o.N + d) : 0.0;
-      const int dj = (int)(e & kBondIdx);
-      const int kj = NS > 1 ? (int)(e >> kBondKindShift) : 0;
+    for (int l0 = gldi(o.soff, s); l0 < l1; l0 += kRows) {
+      unsigned e[kRows];
+      double w[kRows], wr[kRows];
+      V3 sj[kRows][REP];
 #pragma unroll
-      for (int u = 0; u < REP; ++u) {
-        const V3 sj = spin_at(o, ru[u], dj);
-        const double x = si[u].x * sj.x + si[u].y * sj.y + si[u].z * sj.z;
-        const double t = x * w, ta = fabs(x) * w;
+      for (int k = 0; k < kRows; ++k) {          // rows past the shell repeat its last, weight 0
+        const int l = min(l0 + k, l1 - 1);
+        e[k] = gldi(o.sbond, (size_t)l * o.N + d);
+        w[k] = gldi(o.sw, (size_t)l * o.N + d);
+        wr[k] = NS > 1 ? gldi(o.sw, ((size_t)o.srows + l) * o.N + d) : 0.0;
+        if (l0 + k >= l1) { w[k] = 0.0; wr[k] = 0.0; }
+      }
 #pragma unroll
-        for (int y = 0; y < NS; ++y)
-          if (y == kj) {
-            v[u][0][y] += t; v[u][1][y] += ta;
-            if (NS > 1) { vr[u][0][y] += x * wr; vr[u][1][y] += fabs(x) * wr; }
-          }
+      for (int k = 0; k < kRows; ++k)
+#pragma unroll
+        for (int u = 0; u < REP; ++u) sj[k][u] = spin_at(o, ru[u], (int)(e[k] & kBondIdx));
+#pragma unroll
+      for (int k = 0; k < kRows; ++k) {
+        const int kj = NS > 1 ? (int)(e[k] >> kBondKindShift) : 0;
+#pragma unroll
+        for (int u = 0; u < REP; ++u) {
+          const double x = si[u].x * sj[k][u].x + si[u].y * sj[k][u].y + si[u].z * sj[k][u].z;
+          const double t = x * w[k], ta = fabs(x) * w[k];
+#pragma unroll
+          for (int y = 0; y < NS; ++y)
+            if (y == kj) {
+              v[u][0][y] += t; v[u][1][y] += ta;
+              if (NS > 1) { vr[u][0][y] += x * wr[k]; vr[u][1][y] += fabs(x) * wr[k]; }
+            }
+        }
       }
     }
     double f[NV];
@@ -221,11 +251,11 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_spincorr(ObsArgs o) {
 }
 
 // The structure factor F0(q) = sum_j S_j exp(i q.r_j) of every replica is a product of the
-// phase matrix [q][site] with the spin matrix [site][replica, component]; a phase is computed
-// once per (q, site) and kSfRep replicas.  Three launches, each a no-op unless this
-// measurement is one that evaluates S(q) (uniform over the grid):
-//   k_sf_pack   the spins, site-major in groups of kSfRep replicas: [group][site][kSfRep][3]
-//               (device order; for lattice positions reference order and groups of kSfRepLat);
+// phase matrix [q][site] with the spin matrix [site][replica, component].  Launches, each a no-op
+// unless this measurement is one that evaluates S(q) (uniform over the grid):
+//   k_sf_pack   the spins, site-major in groups of replicas: [group][site][replica][3]
+//               (device order, kSfRep replicas; for lattice positions by planes, kSfRepLat);
+// and, for positions that are not a lattice,
 //   k_sf_main   one wave per (64 q-points, replica group, site chunk): lane = q-point, the
 //               site's position and its kSfRep x 3 spins are wave-uniform loads (SGPRs),
 //               one sincos per site serves kSfRep x 6 FMAs (the wave is bound by its FP64
@@ -241,9 +271,13 @@ __device__ __forceinline__ bool sf_due(const ObsArgs &o) {
 
 __global__ __launch_bounds__(kObsBlock) void k_sf_pack(ObsArgs o) {
   if (!sf_due(o)) return;
-  const int j = blockIdx.x * kObsBlock + threadIdx.x;    // device site, or reference site (lattice)
+  const int j = blockIdx.x * kObsBlock + threadIdx.x;    // device site, or place ((x2 nb + a) L1 + x1) L0 + x0
   if (j >= o.N) return;
-  const int d = o.sf_lat ? gldi(o.ref2dev, j) : j;
+  int d = j;
+  if (o.sf_lat) {
+    const int L0 = o.sfL[0], L1 = o.sfL[1], x0 = j % L0, x1 = j / L0 % L1, pl = j / (L0 * L1);
+    d = gldi(o.ref2dev, (((pl / o.nb) * L1 + x1) * L0 + x0) * o.nb + pl % o.nb);
+  }
   const int g = blockIdx.y;
   double *out = o.sfspin + ((size_t)g * o.N + j) * (o.sf_rep * 3);
 #pragma unroll
@@ -295,75 +329,111 @@ __global__ __launch_bounds__(kSfQ) void k_sf_main(ObsArgs o) {
   }
 }
 
-// k_sf_main for lattice positions: the phase of site (x0, x1, x2, a) is the product of four
-// table entries (exp(i q.x0 A0) exp(i q.x1 A1) exp(i q.x2 A2) exp(i q.B_a)): per site one
-// complex product instead of a sincos.  A chunk is a range of (x1, x2) rows, sites in
-// reference order inside a row.
-__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
+// Lattice positions r = B_a + x0 A0 + x1 A1 + x2 A2: F0 is summed axis by axis,
+//   F0(q) = sum_a e^{i q.B_a} sum_x2 e^{i q.A2 x2} Y,   Y(q.A0, q.A1; x2, a) =
+//           sum_x1 e^{i q.A1 x1} sum_x0 e^{i q.A0 x0} S(x0, x1, x2, a),
+// and Y is computed once per distinct pair (q.A0, q.A1) of the q-points -- 51 of the 2601 points of
+// the default mesh -- so a site costs one phase product per pair instead of one per q-point.  Even
+// for q-points that share no pair a site costs its spin's products alone, without the product of
+// phases.
+//   k_sf_plane  one wave per (64 pairs, kSfRepLat replicas, plane x2, a): lane = pair, spins
+//               wave-uniform (scalar loads), 24 FP64 FMAs per site;
+//   k_sf_q      one thread per (q, replica): the planes' sums, then as k_sf_fin.
+// FCC 16^3 x 32, 2601 q: 530 us per evaluation with a phase per q-point and site, 120 us so.
 __device__ __forceinline__ double2 ld2(const double2 *p, size_t i) {
   const double *d = reinterpret_cast<const double *>(p);
   return make_double2(gldi(d, 2 * i), gldi(d, 2 * i + 1));
 }
 
-__global__ __launch_bounds__(kSfQ) void k_sf_lat(ObsArgs o) {
+__global__ __launch_bounds__(kSfQ) void k_sf_plane(ObsArgs o) {
   constexpr int RV = kSfRepLat * 3;                 // spin values of one site and group
   if (!sf_due(o)) return;
-  const int iq0 = blockIdx.x * kSfQ + threadIdx.x;
-  const int iq = min(iq0, o.nq - 1);                 // lanes past nq compute q nq-1, store nothing
-  const int g = blockIdx.y, ch = blockIdx.z;
-  const int L0 = o.sfL[0], L1 = o.sfL[1], nb = o.nb;
-  const int rows = L1 * o.sfL[2];
-  const int w0 = ch * o.sf_chunk, w1 = min(rows, w0 + o.sf_chunk);
-  double fr[kSfRepLat][3], fi[kSfRepLat][3];
+  const int u0 = blockIdx.x * kSfQ + threadIdx.x;
+  const int u = min(u0, o.npq - 1);                  // lanes past npq repeat the last pair, store nothing
+  const int g = o.sf_g0 + blockIdx.y, pl = blockIdx.z;
+  const int L0 = o.sfL[0], L1 = o.sfL[1];
+  const double *sv = o.sfspin + ((size_t)g * o.N + (size_t)pl * L0 * L1) * RV;
+  double yr[RV], yi[RV];
 #pragma unroll
-  for (int u = 0; u < kSfRepLat; ++u)
+  for (int k = 0; k < RV; ++k) { yr[k] = 0.0; yi[k] = 0.0; }
+  for (int x1 = 0; x1 < L1; ++x1) {
+    double xr[RV], xi[RV];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) { fr[u][k] = 0.0; fi[u][k] = 0.0; }
-  auto add = [&](const double (&v)[RV], double2 ph) {
+    for (int k = 0; k < RV; ++k) { xr[k] = 0.0; xi[k] = 0.0; }
+    int x0 = 0;
+    for (; x0 + 1 < L0; x0 += 2, sv += 2 * RV) {     // two sites per wait on the scalar loads
+      double v0[RV], v1[RV];
 #pragma unroll
-    for (int u = 0; u < kSfRepLat; ++u)
+      for (int k = 0; k < RV; ++k) { v0[k] = cldi(sv, k); v1[k] = cldi(sv, RV + k); }
+      const double2 p0 = ld2(o.sfex, (size_t)x0 * o.npq + u), p1 = ld2(o.sfex, (size_t)(x0 + 1) * o.npq + u);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        fr[u][k] += v[3 * u + k] * ph.x;
-        fi[u][k] += v[3 * u + k] * ph.y;
-      }
-  };
-  const double *spg = o.sfspin + (size_t)g * o.N * RV;
-  for (int w = w0; w < w1; ++w) {
-    const double2 byz = cmul(ld2(o.sfey, (size_t)(w % L1) * o.nq + iq), ld2(o.sfez, (size_t)(w / L1) * o.nq + iq));
-    for (int x0 = 0; x0 < L0; ++x0) {
-      const double2 bx = cmul(ld2(o.sfex, (size_t)x0 * o.nq + iq), byz);
-      const double *sv0 = spg + ((size_t)w * L0 + x0) * nb * RV;
-      int a = 0;
-      for (; a + 1 < nb; a += 2) {     // two sites per wait on the (out-of-order) scalar loads
-        double v0[RV], v1[RV];
-#pragma unroll
-        for (int k = 0; k < RV; ++k) { v0[k] = sv0[(size_t)a * RV + k]; v1[k] = sv0[(size_t)(a + 1) * RV + k]; }
-        add(v0, cmul(bx, ld2(o.sfeb, (size_t)a * o.nq + iq)));
-        add(v1, cmul(bx, ld2(o.sfeb, (size_t)(a + 1) * o.nq + iq)));
-      }
-      if (a < nb) {
-        double v0[RV];
-#pragma unroll
-        for (int k = 0; k < RV; ++k) v0[k] = sv0[(size_t)a * RV + k];
-        add(v0, cmul(bx, ld2(o.sfeb, (size_t)a * o.nq + iq)));
+      for (int k = 0; k < RV; ++k) {
+        xr[k] += v0[k] * p0.x; xi[k] += v0[k] * p0.y;
+        xr[k] += v1[k] * p1.x; xi[k] += v1[k] * p1.y;
       }
     }
-  }
-  if (iq0 >= o.nq) return;
+    if (x0 < L0) {
+      const double2 p0 = ld2(o.sfex, (size_t)x0 * o.npq + u);
 #pragma unroll
-  for (int u = 0; u < kSfRepLat; ++u) {
-    const int r = g * kSfRepLat + u;
+      for (int k = 0; k < RV; ++k) {
+        const double v = cldi(sv, k);
+        xr[k] += v * p0.x; xi[k] += v * p0.y;
+      }
+      sv += RV;
+    }
+    const double2 p = ld2(o.sfey, (size_t)x1 * o.npq + u);
+#pragma unroll
+    for (int k = 0; k < RV; ++k) {
+      yr[k] += xr[k] * p.x - xi[k] * p.y;
+      yi[k] += xr[k] * p.y + xi[k] * p.x;
+    }
+  }
+  if (u0 >= o.npq) return;
+#pragma unroll
+  for (int t = 0; t < kSfRepLat; ++t) {
+    const int r = g * kSfRepLat + t;
     if (r >= o.R) break;
-    double *out = o.sfpart + ((size_t)ch * o.R + r) * 6 * o.nq + iq;
+    double *out = o.sfpart + (((size_t)(r - o.sf_g0 * kSfRepLat) * gridDim.z + pl) * 6) * o.npq + u;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      gsti(out, (size_t)k * o.nq, fr[u][k]);
-      gsti(out, (size_t)(3 + k) * o.nq, fi[u][k]);
+      gsti(out, (size_t)k * o.npq, yr[3 * t + k]);
+      gsti(out, (size_t)(3 + k) * o.npq, yi[3 * t + k]);
     }
   }
+}
+
+__device__ __forceinline__ void sf_accumulate(const ObsArgs &o, int iq, int r, const double (&fr)[3], const double (&fi)[3]);
+
+__global__ __launch_bounds__(kObsBlock) void k_sf_q(ObsArgs o) {
+  if (!sf_due(o)) return;
+  const int iq = blockIdx.x * kObsBlock + threadIdx.x;
+  const int rl = blockIdx.y, r = o.sf_g0 * kSfRepLat + rl;
+  if (iq >= o.nq) return;
+  const int nb = o.nb, L2 = o.sfL[2], npl = L2 * nb;
+  const int u = gldi(o.sfpair, iq);
+  const double *y = o.sfpart + (size_t)rl * npl * 6 * o.npq + u;
+  double fr[3] = {0.0, 0.0, 0.0}, fi[3] = {0.0, 0.0, 0.0};
+  for (int a = 0; a < nb; ++a) {
+    double zr[3] = {0.0, 0.0, 0.0}, zi[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int x2 = 0; x2 < L2; ++x2) {
+      const double2 p = ld2(o.sfez, (size_t)x2 * o.nq + iq);
+      const double *t = y + (size_t)(x2 * nb + a) * 6 * o.npq;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double re = gldi(t, (size_t)k * o.npq), im = gldi(t, (size_t)(3 + k) * o.npq);
+        zr[k] += re * p.x - im * p.y;
+        zi[k] += re * p.y + im * p.x;
+      }
+    }
+    const double2 p = ld2(o.sfeb, (size_t)a * o.nq + iq);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      fr[k] += zr[k] * p.x - zi[k] * p.y;
+      fi[k] += zr[k] * p.y + zi[k] * p.x;
+    }
+  }
+  sf_accumulate(o, iq, r, fr, fi);
 }
 
 __global__ __launch_bounds__(kObsBlock) void k_sf_fin(ObsArgs o) {
@@ -371,9 +441,6 @@ __global__ __launch_bounds__(kObsBlock) void k_sf_fin(ObsArgs o) {
   const int iq = blockIdx.x * kObsBlock + threadIdx.x;
   const int r = blockIdx.y;
   if (iq >= o.nq) return;
-  const double qx = gldi(o.q, 3 * iq), qy = gldi(o.q, 3 * iq + 1), qz = gldi(o.q, 3 * iq + 2);
-  const double q2 = qx * qx + qy * qy + qz * qz;
-  if (q2 == 0.0) return;
   double fr[3] = {0.0, 0.0, 0.0}, fi[3] = {0.0, 0.0, 0.0};
   for (int ch = 0; ch < o.sf_nchunk; ++ch) {
     const double *p = o.sfpart + ((size_t)ch * o.R + r) * 6 * o.nq + iq;
@@ -383,6 +450,14 @@ __global__ __launch_bounds__(kObsBlock) void k_sf_fin(ObsArgs o) {
       fi[k] += gldi(p, (size_t)(3 + k) * o.nq);
     }
   }
+  sf_accumulate(o, iq, r, fr, fi);
+}
+
+// F0(q) of replica r into its slot's sums; q = 0 adds nothing.
+__device__ __forceinline__ void sf_accumulate(const ObsArgs &o, int iq, int r, const double (&fr)[3], const double (&fi)[3]) {
+  const double qx = gldi(o.q, 3 * iq), qy = gldi(o.q, 3 * iq + 1), qz = gldi(o.q, 3 * iq + 2);
+  const double q2 = qx * qx + qy * qy + qz * qz;
+  if (q2 == 0.0) return;
   const double pn = o.have_polar ? sqrt(o.polar[0] * o.polar[0] + o.polar[1] * o.polar[1] +
                                         o.polar[2] * o.polar[2]) : 1.0;
   // perpendicular part: F - (F . q / q^2) q (real and imaginary parts separately)
@@ -484,8 +559,9 @@ ObsArgs obs_args(esp_ctx *c) {
   o.sf_rep = b.sf_lat ? kSfRepLat : kSfRep;
   for (int k = 0; k < 3; ++k) o.sfL[k] = b.sfL[k];
   o.sfex = b.d_sftab;
-  o.sfey = o.sfex ? o.sfex + (size_t)b.sfL[0] * b.nq : nullptr;
-  o.sfez = o.sfey ? o.sfey + (size_t)b.sfL[1] * b.nq : nullptr;
+  o.npq = b.npq; o.sfpair = b.d_sfpair;
+  o.sfey = o.sfex ? o.sfex + (size_t)b.sfL[0] * b.npq : nullptr;
+  o.sfez = o.sfey ? o.sfey + (size_t)b.sfL[1] * b.npq : nullptr;
   o.sfeb = o.sfez ? o.sfez + (size_t)b.sfL[2] * b.nq : nullptr;
   o.sf = b.d_sf; o.sfn = b.d_sfn;
   o.acc = b.d_acc; o.trace = b.d_trace; o.trace_cap = c->trace_cap;
@@ -514,7 +590,7 @@ void obs_free(esp_ctx *c) {
   dfree(b.d_axes); dfree(b.d_coeff); dfree(b.d_acc); dfree(b.d_part); dfree(b.d_pm);
   dfree(b.d_skind); dfree(b.d_soff); dfree(b.d_sbond); dfree(b.d_sw); dfree(b.d_sc);
   dfree(b.d_scpart); dfree(b.d_q); dfree(b.d_pos); dfree(b.d_sf); dfree(b.d_sfn); dfree(b.d_trace);
-  dfree(b.d_sfspin); dfree(b.d_sfpart); dfree(b.d_sftab); dfree(b.d_cdev);
+  dfree(b.d_sfspin); dfree(b.d_sfpart); dfree(b.d_sftab); dfree(b.d_sfpair); dfree(b.d_cdev);
   b = esp_ctx::Obs{};
 }
 
@@ -552,17 +628,26 @@ int obs_resize(esp_ctx *c) {
   if (b.flags & ESP_OBS_SFACTOR) {
     if ((rc = dalloc(c, b.d_sf, (size_t)R * 3 * b.nq))) return rc;
     if ((rc = dalloc(c, b.d_sfn, 1))) return rc;
-    // site chunks (lattice: chunks of (x1, x2) rows): enough waves to fill the chip, at least
-    // 64 sites each
     const int srep = b.sf_lat ? kSfRepLat : kSfRep;
-    const int ng = (R + srep - 1) / srep, nqb = (b.nq + kSfQ - 1) / kSfQ;
-    const int units = b.sf_lat ? b.sfL[1] * b.sfL[2] : N;
-    int nch = (kSfWaves + ng * nqb - 1) / (ng * nqb);
-    nch = std::max(1, std::min({nch, kSfMaxChunks, units, (N + 63) / 64}));
-    b.sf_chunk = (units + nch - 1) / nch;
-    b.sf_nchunk = (units + b.sf_chunk - 1) / b.sf_chunk;
+    const int ng = (R + srep - 1) / srep;
+    size_t npart;
+    if (b.sf_lat) {
+      // plane sums of as many replica groups at a time as kSfPlaneBytes hold
+      const size_t per = (size_t)srep * b.sfL[2] * nb * 6 * b.npq;
+      b.sf_chunk = (int)std::max<size_t>(1, std::min<size_t>(ng, kSfPlaneBytes / (per * sizeof(double))));
+      b.sf_nchunk = (ng + b.sf_chunk - 1) / b.sf_chunk;
+      npart = per * b.sf_chunk;
+    } else {
+      // site chunks: enough waves to fill the chip, at least 64 sites each
+      const int nqb = (b.nq + kSfQ - 1) / kSfQ;
+      int nch = (kSfWaves + ng * nqb - 1) / (ng * nqb);
+      nch = std::max(1, std::min({nch, kSfMaxChunks, N, (N + 63) / 64}));
+      b.sf_chunk = (N + nch - 1) / nch;
+      b.sf_nchunk = (N + b.sf_chunk - 1) / b.sf_chunk;
+      npart = (size_t)b.sf_nchunk * R * 6 * b.nq;
+    }
     if ((rc = dalloc(c, b.d_sfspin, (size_t)ng * N * srep * 3))) return rc;
-    if ((rc = dalloc(c, b.d_sfpart, (size_t)b.sf_nchunk * R * 6 * b.nq))) return rc;
+    if ((rc = dalloc(c, b.d_sfpart, npart))) return rc;
   }
   if (c->trace_cap > 0 && (b.flags & (ESP_OBS_ORDER | ESP_OBS_STAGGERED)))
     if ((rc = dalloc(c, b.d_trace, (size_t)c->trace_cap * R * 2))) return rc;
@@ -607,11 +692,18 @@ int obs_enqueue(esp_ctx *c) {
     const int srep = b.sf_lat ? kSfRepLat : kSfRep;
     const int ng = (c->R + srep - 1) / srep;
     hipLaunchKernelGGL(k_sf_pack, dim3((o.N + kObsBlock - 1) / kObsBlock, ng), dim3(kObsBlock), 0, c->stream, o);
-    if (b.sf_lat)
-      hipLaunchKernelGGL(k_sf_lat, dim3((b.nq + kSfQ - 1) / kSfQ, ng, b.sf_nchunk), dim3(kSfQ), 0, c->stream, o);
-    else
+    if (b.sf_lat) {
+      ObsArgs p = o;
+      for (int g0 = 0; g0 < ng; g0 += b.sf_chunk) {
+        const int n = std::min(b.sf_chunk, ng - g0), nr = std::min(c->R - g0 * srep, n * srep);
+        p.sf_g0 = g0;
+        hipLaunchKernelGGL(k_sf_plane, dim3((b.npq + kSfQ - 1) / kSfQ, n, b.sfL[2] * o.nb), dim3(kSfQ), 0, c->stream, p);
+        hipLaunchKernelGGL(k_sf_q, dim3((b.nq + kObsBlock - 1) / kObsBlock, nr), dim3(kObsBlock), 0, c->stream, p);
+      }
+    } else {
       hipLaunchKernelGGL(k_sf_main, dim3((b.nq + kSfQ - 1) / kSfQ, ng, b.sf_nchunk), dim3(kSfQ), 0, c->stream, o);
-    hipLaunchKernelGGL(k_sf_fin, dim3((b.nq + kObsBlock - 1) / kObsBlock, c->R), dim3(kObsBlock), 0, c->stream, o);
+      hipLaunchKernelGGL(k_sf_fin, dim3((b.nq + kObsBlock - 1) / kObsBlock, c->R), dim3(kObsBlock), 0, c->stream, o);
+    }
   }
   hipLaunchKernelGGL(k_obs_final, dim3(c->R), dim3(kObsBlock), 0, c->stream, o);
   HIPCHK(c, hipGetLastError());
@@ -842,7 +934,7 @@ int esp_set_sfactor(esp_ctx *c, int nq, const double *q, const double *pos, cons
   int rc = need_model(c);
   if (rc) return rc;
   auto &b = c->obs;
-  dfree(b.d_q); dfree(b.d_pos); dfree(b.d_sftab);
+  dfree(b.d_q); dfree(b.d_pos); dfree(b.d_sftab); dfree(b.d_sfpair);
   b.flags &= ~ESP_OBS_SFACTOR;
   b.nq = 0;
   b.sf_lat = 0;
@@ -886,22 +978,35 @@ int esp_set_sfactor(esp_ctx *c, int nq, const double *q, const double *pos, cons
               if (std::fabs(at(x0, x1, x2, a)[m] - r) > tol) { lat = false; break; }
             }
     if (lat) {
-      std::vector<double2> tab((size_t)(L[0] + L[1] + L[2] + nb) * nq);
-      size_t row = 0;
+      // distinct pairs (q.A0, q.A1)
+      auto along = [&](int iq, int k) {
+        const double *qq = q + 3 * (size_t)iq;
+        return qq[0] * A[k][0] + qq[1] * A[k][1] + qq[2] * A[k][2];
+      };
+      std::map<std::pair<double, double>, int> pairs;
+      std::vector<int> pair(nq), first;
+      for (int iq = 0; iq < nq; ++iq) {
+        const auto it = pairs.insert({{along(iq, 0), along(iq, 1)}, (int)first.size()});
+        if (it.second) first.push_back(iq);
+        pair[iq] = it.first->second;
+      }
+      const int np = (int)first.size();
+      std::vector<double2> tab((size_t)(L[0] + L[1]) * np + (size_t)(L[2] + nb) * nq);
+      size_t at0 = 0;
+      auto phase = [&](int iq, double x, double y, double z) {
+        const double *qq = q + 3 * (size_t)iq;
+        const double ph = qq[0] * x + qq[1] * y + qq[2] * z;
+        tab[at0++] = make_double2(std::cos(ph), std::sin(ph));
+      };
       for (int k = 0; k < 3; ++k)
-        for (int x = 0; x < L[k]; ++x, ++row)
-          for (int iq = 0; iq < nq; ++iq) {
-            const double *qq = q + 3 * (size_t)iq;
-            const double ph = qq[0] * (x * A[k][0]) + qq[1] * (x * A[k][1]) + qq[2] * (x * A[k][2]);
-            tab[row * nq + iq] = make_double2(std::cos(ph), std::sin(ph));
-          }
-      for (int a = 0; a < nb; ++a, ++row)
-        for (int iq = 0; iq < nq; ++iq) {
-          const double *qq = q + 3 * (size_t)iq, *ba = pos + 3 * (size_t)a;
-          const double ph = qq[0] * ba[0] + qq[1] * ba[1] + qq[2] * ba[2];
-          tab[row * nq + iq] = make_double2(std::cos(ph), std::sin(ph));
-        }
-      if ((rc = upload(c, b.d_sftab, tab))) return rc;
+        for (int x = 0; x < L[k]; ++x)
+          for (int i = 0; i < (k < 2 ? np : nq); ++i)
+            phase(k < 2 ? first[i] : i, x * A[k][0], x * A[k][1], x * A[k][2]);
+      for (int a = 0; a < nb; ++a)
+        for (int iq = 0; iq < nq; ++iq) phase(iq, pos[3 * (size_t)a], pos[3 * (size_t)a + 1], pos[3 * (size_t)a + 2]);
+      if ((rc = upload(c, b.d_sftab, tab)) || (rc = upload(c, b.d_sfpair, pair))) return rc;
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+      b.npq = np;
       b.sf_lat = 1;
       for (int k = 0; k < 3; ++k) b.sfL[k] = L[k];
     }
