@@ -243,15 +243,6 @@ __device__ __forceinline__ void net_forward_mfma(const float *wl, const NetA &na
   }
 }
 
-struct Mix {
-  double logw[2];   // log of (1 - kUniform) w_k
-  double kappa[2];
-  double lnorm[2];  // log of kappa / (2 pi (1 - e^{-2 kappa})): vMF density = exp(lnorm + kappa (mu.x - 1))
-  double e2k[2];    // e^{-2 kappa}
-  double t[2];      // tilt angle of mu_k from ghat
-  V3 mu[2];
-};
-
 __device__ __forceinline__ V3 vnorm(V3 v) {
   const double r = rsqrt(dot(v, v));
   return {v.x * r, v.y * r, v.z * r};
@@ -269,34 +260,43 @@ __device__ __forceinline__ V3 tilt_frame(const V3 &ghat, const V3 &ax) {
 
 __device__ __forceinline__ float softplusf(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
 
-// Mixture from the network outputs and the local frame (ghat, pole axis).
-__device__ __forceinline__ Mix make_mix(const float o[kOut], float kappa0, const V3 &ghat, const V3 &ax) {
-  Mix m;
-  const V3 e = tilt_frame(ghat, ax);
-  const float d = o[4] - o[1];                 // log softmax of the two weight logits
-  m.logw[0] = (double)(-softplusf(d)) + kLog1mU;
-  m.logw[1] = (double)(-softplusf(-d)) + kLog1mU;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const float sc = fminf(fmaxf(o[3 * k], -8.0f), 8.0f);
-    const double kap = (double)(kappa0 * expf(sc)) + 1e-6;
-    m.kappa[k] = kap;
-    const double em1 = expm1(-2.0 * kap);
-    m.e2k[k] = 1.0 + em1;
-    m.lnorm[k] = log(kap / -em1) - kLog2Pi;
-    const float th = tanhf(o[3 * k + 2]);
-    float sn, cs;
-    sincospif(0.5f * th, &sn, &cs);
-    m.t[k] = 0.5 * kPi * (double)th;
-    m.mu[k] = vnorm(V3{cs * ghat.x + sn * e.x, cs * ghat.y + sn * e.y, cs * ghat.z + sn * e.z});
-  }
+// One component of the mixture in the log domain, from its outputs (o0: concentration, o1: weight
+// logit, o2: tilt), the other component's weight logit p1 and the local frame (ghat, e).
+struct Comp {
+  double logw;      // log of (1 - kUniform) w_k
+  double kappa;
+  double lnorm;     // log of kappa / (2 pi (1 - e^{-2 kappa})): vMF density = exp(lnorm + kappa (mu.x - 1))
+  double t;         // tilt angle of mu_k from ghat
+  V3 mu;
+};
+__device__ __forceinline__ Comp make_comp(float o0, float o1, float o2, float p1, float kappa0, const V3 &ghat,
+                                          const V3 &e) {
+  Comp m;
+  m.logw = (double)(-softplusf(p1 - o1)) + kLog1mU;   // log softmax of the two weight logits
+  const float sc = fminf(fmaxf(o0, -8.0f), 8.0f);
+  m.kappa = (double)(kappa0 * expf(sc)) + 1e-6;
+  m.lnorm = log(m.kappa / -expm1(-2.0 * m.kappa)) - kLog2Pi;
+  const float th = tanhf(o2);
+  float sn, cs;
+  sincospif(0.5f * th, &sn, &cs);
+  m.t = 0.5 * kPi * (double)th;
+  m.mu = vnorm(V3{cs * ghat.x + sn * e.x, cs * ghat.y + sn * e.y, cs * ghat.z + sn * e.z});
   return m;
+}
+// log of (1 - kUniform) w_k vMF_k(x), log vMF(x) = lnorm + kappa (mu . x - 1)
+__device__ __forceinline__ double log_part(const Comp &m, const V3 &x) {
+  return m.logw + (m.lnorm + m.kappa * (dot(m.mu, x) - 1.0));
+}
+// Log density of the mixture from its two components' parts.
+__device__ __forceinline__ double log_mix(double l0, double l1) {
+  const double mx = fmax(fmax(l0, l1), kLogUni);
+  return mx + log(exp(l0 - mx) + exp(l1 - mx) + exp(kLogUni - mx));
 }
 
 // The mixture as the sweep uses it, without logarithms: selection weights ws_k = (1 - kUniform)
 // w_k, concentrations, e^{-2 kappa_k} and density prefactors c_k = ws_k kappa_k / (2 pi (1 -
 // e^{-2 kappa_k})), so that q(x) = sum_k c_k exp(kappa_k (mu_k . x - 1)) + kUniform / (4 pi).
-// Sampling and density use the same ws_k, kappa_k and mu_k (the log-domain Mix of training
+// Sampling and density use the same ws_k, kappa_k and mu_k (the log-domain mixture of training
 // differs from it only by rounding, which no sweep quantity depends on).
 struct MixS {
   double ws0;       // selection weight of component 0 (component 1: 1 - kUniform - ws0)
@@ -324,18 +324,6 @@ __device__ __forceinline__ MixS make_mix_sweep(const float o[kOut], float kappa0
     m.mu[k] = vnorm(V3{cs * ghat.x + sn * e.x, cs * ghat.y + sn * e.y, cs * ghat.z + sn * e.z});
   }
   return m;
-}
-
-// log vMF_k(x) = lnorm_k + kappa_k (mu_k . x - 1)
-__device__ __forceinline__ double log_vmf(const Mix &m, int k, const V3 &x) {
-  return m.lnorm[k] + m.kappa[k] * (dot(m.mu[k], x) - 1.0);
-}
-
-__device__ __forceinline__ double log_q(const Mix &m, const V3 &x) {
-  const double l0 = m.logw[0] + log_vmf(m, 0, x);
-  const double l1 = m.logw[1] + log_vmf(m, 1, x);
-  const double mx = fmax(fmax(l0, l1), kLogUni);
-  return mx + log(exp(l0 - mx) + exp(l1 - mx) + exp(kLogUni - mx));
 }
 
 // Wood (1994) for S^2: w = 1 + log(v + (1 - v) e^{-2 kappa}) / kappa, azimuth 2 pi u; kappa = 0
@@ -577,201 +565,208 @@ __device__ __forceinline__ V3 rec_vec(const float *rec, int o) {
 }
 
 // ---- training: gradient of the mean negative log-likelihood ------------------------------------
-// One wave takes tiles of 32 records through the network on the matrix cores in FP32
-// (v_mfma_f32_32x32x2_f32): a 32 x 32 layer of 32 records is 16 instructions.  Operand layouts
-// (lane l, half h = l / 32): A[i = l % 32][k = h], B[k = h][j = l % 32], D register v =
-// D[8 (v / 4) + 4 h + v % 4][l % 32].  The order of the products in k is free, so step (q, r) =
-// v pairs k = 8 q + r (half 0) with k = 8 q + 4 + r (half 1): the B operand of a layer is then the
-// lane's own D register v of the layer before (forward and backward alike), with no exchange, and
-// the weights' A operand is W[l % 32][8 q + 4 h + r] (forward) or W[8 q + 4 h + r][l % 32]
-// (backward).  The weight gradients, sums over records of delta x activation, take both factors
-// with lane = unit and register = record, through a transposition in LDS, and accumulate in D
-// registers over the wave's tiles.  One thread per record and a sum over the records of a
-// block per parameter took 185 us for a minibatch of 2048 (16 blocks, a serial chain of 7200
-// multiply-adds per thread through LDS); 20 us so.
-constexpr int kTile = 32;             // records of a tile
-constexpr int kTrainWaves = 512;      // waves of a gradient at most (more tiles: several per wave)
-constexpr int kTrow = kTile + 1;      // LDS row of one unit's values over the tile's records
-
-__device__ __forceinline__ int d_unit(int v, int h) { return 8 * (v >> 2) + 4 * h + (v & 3); }
-
-// D = W B + C over 32 units with A = w[16] and B = b (D layout).
-__device__ __forceinline__ floatx16 mat32(const float (&w)[16], const floatx16 &b, floatx16 c) {
-#pragma unroll
-  for (int v = 0; v < 16; ++v) c = __builtin_amdgcn_mfma_f32_32x32x2f32(w[v], b[v], c, 0, 0, 0);
-  return c;
+// One block per 128 records, one wave per 16 of them from the first layer to the last delta: a
+// layer is a 32 x 32 by 32 x 16 product on the FP32 matrix instructions (16 x 16 x 4, two unit
+// tiles), which round like a chain of FMAs over the inputs in order.  Weights lie in LDS; a
+// layer's values go through LDS rows [unit][record], where a wave reads only what it wrote (no
+// block barrier between layers) and where the parameter gradients are summed from, up to
+// five entries per thread, over the block's records in order.  Every sum has a fixed order -- inputs,
+// records, blocks ascending -- and products enter the gradient sums rounded: Adam divides a
+// gradient by its own size, so a changed rounding of an entry near zero changes its sign and the
+// weight by a whole step (summing gradients on the matrix cores too moved epoch losses by 3e-7).
+// A minibatch of 2048 records is 16 blocks, so the time is one block's chain of layers: 185 us
+// with a record per thread and rows [record][unit] in LDS, 25 us on FMAs with scalar weights
+// (whose loads it waited for), 18 us so -- the mixture's FP64 and the gradients' LDS reads.
+constexpr int kTrainRec = 128;        // records of a block
+constexpr int kTrainThreads = 512;    // 16 records a wave
+constexpr int kTrow = kTrainRec + 4;  // LDS row of one unit's values over the block's records
+constexpr int kWrow = kH + 4;         // LDS row of a weight matrix: 16 rows x 4 columns on 64 banks
+struct TrainLds {
+  float x[kIn][kTrow], g4[kOut][kTrow], one[kTrow];
+  float a1[kH][kTrow], a2[kH][kTrow], a3[kH][kTrow], d1[kH][kTrow], d2[kH][kTrow], d3[kH][kTrow];
+  float w1[kH][8], w2[kH][kWrow], w3[kH][kWrow], w4[16][kWrow];   // w1's columns and w4's rows padded with 0
+  float b1[kH], b2[kH], b3[kH], b4[16];
+  double loss[kTrainRec];
+};
+using F4 = float __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ F4 mfma4(float a, float b, F4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-
-// x (D layout: lane = record) into LDS rows [unit][record].
-__device__ __forceinline__ void put_rows(float *t, const floatx16 &x, int l, int h) {
-#pragma unroll
-  for (int v = 0; v < 16; ++v) t[d_unit(v, h) * kTrow + l] = x[v];
+// LDS written by a wave's lanes, read by others of the same wave.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
-
-// C += sum over the tile's records of left[unit i][rec] right[unit c][rec], both LDS rows; *bias
-// += this lane's half of sum over records of left[l].
-__device__ __forceinline__ floatx16 outer32(const float *left, const float *right, int l, int h, floatx16 c, float *bias) {
+// z += W in for one wave's records; lane (h, c): record i of column c, units 16 t + 4 h + r in
+// z[t][r].  TR: W transposed.
+template <bool TR>
+__device__ __forceinline__ void layer_mfma(const float (&w)[kH][kWrow], const float (&in)[kH][kTrow], int i, int h,
+                                           int c, F4 (&z)[2]) {
 #pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    const float x = left[l * kTrow + 2 * s + h], y = right[l * kTrow + 2 * s + h];
-    if (bias) *bias += x;
-    c = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, c, 0, 0, 0);
+  for (int s = 0; s < kH / 4; ++s) {
+    const float b = in[4 * s + h][i];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) z[t] = mfma4(TR ? w[4 * s + h][16 * t + c] : w[16 * t + c][4 * s + h], b, z[t]);
   }
-  return c;
+}
+__device__ __forceinline__ void bias4(const float (&b)[kH], int h, F4 (&z)[2]) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t) z[t] = *reinterpret_cast<const F4 *>(&b[16 * t + 4 * h]);
+}
+// A gradient term: the product is rounded before it is added.
+__device__ __forceinline__ float mad(float s, float d, float a) {
+#pragma clang fp contract(off)
+  const float p = d * a;
+  return s + p;
 }
 
-__global__ __launch_bounds__(64) void k_train_tiles(const float *w, const float *recs, int n, const int *perm, int off,
-                                                    float *part_grad, double *part_loss) {
-  __shared__ float s_w4[kOut * kH + kOut];
-  __shared__ float s_l[kH * kTrow], s_r[kH * kTrow];
-  const int lane = threadIdx.x, l = lane & 31, h = lane >> 5;
-  for (int k = lane; k < kOut * kH + kOut; k += 64) s_w4[k] = w[oW4 + k];
-  float w1[3], w2[16], w3[16], w2t[16], w3t[16];
+__global__ __launch_bounds__(kTrainThreads) void k_train_block(const float *w, const float *recs, int n,
+                                                               const int *perm, int off, float *part_grad,
+                                                               double *part_loss) {
+  extern __shared__ double s_tr[];
+  TrainLds &t = *reinterpret_cast<TrainLds *>(s_tr);
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 4, c = lane & 15;
+  const int i = 16 * (tid >> 6) + c, ir = blockIdx.x * kTrainRec + i;
+  const bool on = ir < n;                         // rows of records past n hold zeros: they add nothing
+  const float *rec = recs + (size_t)(perm ? perm[off + (on ? ir : 0)] : off + (on ? ir : 0)) * kRec;
+  const float x0 = rec[h], x1 = h ? 0.f : rec[4];  // inputs h and 4 + h (kIn = 5)
+  float rv[10];                                   // kappa_0, ghat, axis, spin
 #pragma unroll
-  for (int s = 0; s < 3; ++s) w1[s] = 2 * s + h < kIn ? w[oW1 + l * kIn + 2 * s + h] : 0.f;
+  for (int k = 0; k < 10; ++k) rv[k] = rec[5 + k];
+  for (int e = tid; e < kH * 8; e += kTrainThreads) t.w1[e >> 3][e & 7] = (e & 7) < kIn ? w[oW1 + (e >> 3) * kIn + (e & 7)] : 0.f;
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int k = d_unit(v, h);
-    w2[v] = w[oW2 + l * kH + k];
-    w3[v] = w[oW3 + l * kH + k];
-    w2t[v] = w[oW2 + k * kH + l];
-    w3t[v] = w[oW3 + k * kH + l];
+  for (int e = tid; e < kH * kH; e += kTrainThreads) {
+    t.w2[e >> 5][e & 31] = w[oW2 + e];
+    t.w3[e >> 5][e & 31] = w[oW3 + e];
   }
-  floatx16 dw1{}, dw2{}, dw3{}, dw4{};
-  float db2 = 0.f, db3 = 0.f, db4 = 0.f;
-  double loss = 0.0;
+  if (tid < 16 * kH) t.w4[tid >> 5][tid & 31] = tid < kOut * kH ? w[oW4 + tid] : 0.f;
+  if (tid < kH) { t.b1[tid] = w[oB1 + tid]; t.b2[tid] = w[oB2 + tid]; t.b3[tid] = w[oB3 + tid]; }
+  if (tid < 16) t.b4[tid] = tid < kOut ? w[oB4 + tid] : 0.f;
+  if (tid < kTrainRec) t.one[tid] = 1.f;
+  t.x[h][i] = on ? x0 : 0.f;
+  if (h == 0) t.x[4][i] = on ? x1 : 0.f;
   __syncthreads();
-  const int tiles = (n + kTile - 1) / kTile;
-  for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
-    const int i = t * kTile + l;
-    const bool on = i < n;
-    const float *rec = recs + (size_t)(perm ? perm[off + (on ? i : 0)] : off + (on ? i : 0)) * kRec;
-    float x[kIn + 1];
+
+  F4 z[2], g1[2], g2[2], g3[2];                   // g: derivatives of the activations
+  auto put = [&](float (&a)[kH][kTrow], F4 (&g)[2]) {
 #pragma unroll
-    for (int k = 0; k < kIn; ++k) x[k] = rec[k];
-    x[kIn] = 0.f;
-    floatx16 z, a1, a2, a3, g1, g2, g3;   // activations and their derivatives
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) z[v] = w[oB1 + d_unit(v, h)];
+      for (int r = 0; r < 4; ++r) {
+        a[16 * m + 4 * h + r][i] = on ? act(z[m][r]) : 0.f;
+        g[m][r] = act_d(z[m][r]);
+      }
+    wave_lds_sync();
+  };
+  bias4(t.b1, h, z);
 #pragma unroll
-    for (int s = 0; s < 3; ++s)
-      z = __builtin_amdgcn_mfma_f32_32x32x2f32(w1[s], h ? x[2 * s + 1] : x[2 * s], z, 0, 0, 0);
+  for (int m = 0; m < 2; ++m) z[m] = mfma4(t.w1[16 * m + c][4 + h], x1, mfma4(t.w1[16 * m + c][h], x0, z[m]));
+  put(t.a1, g1);
+  bias4(t.b2, h, z);
+  layer_mfma<false>(t.w2, t.a1, i, h, c, z);
+  put(t.a2, g2);
+  bias4(t.b3, h, z);
+  layer_mfma<false>(t.w3, t.a2, i, h, c, z);
+  put(t.a3, g3);
+  F4 zo = *reinterpret_cast<const F4 *>(&t.b4[4 * h]);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) { a1[v] = act(z[v]); g1[v] = act_d(z[v]); }
+  for (int s = 0; s < kH / 4; ++s) zo = mfma4(t.w4[c][4 * s + h], t.a3[4 * s + h][i], zo);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) z[v] = w[oB2 + d_unit(v, h)];
-    z = mat32(w2, a1, z);
-#pragma unroll
-    for (int v = 0; v < 16; ++v) { a2[v] = act(z[v]); g2[v] = act_d(z[v]); }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) z[v] = w[oB3 + d_unit(v, h)];
-    z = mat32(w3, a2, z);
-#pragma unroll
-    for (int v = 0; v < 16; ++v) { a3[v] = act(z[v]); g3[v] = act_d(z[v]); }
-    float o[kOut], g4[kOut];
-#pragma unroll
-    for (int q = 0; q < kOut; ++q) {      // this half's units, then the partner's
-      float acc = 0.f;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc += s_w4[q * kH + d_unit(v, h)] * a3[v];
-      o[q] = s_w4[kOut * kH + q] + (acc + __shfl_xor(acc, 32, 64));
-    }
-    const V3 ghat = rec_vec(rec, 6), ax = rec_vec(rec, 9), s = rec_vec(rec, 12);
-    const Mix m = make_mix(o, rec[5], ghat, ax);
-    double lv[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) lv[k] = m.logw[k] + log_vmf(m, k, s);
-    const double mx = fmax(fmax(lv[0], lv[1]), kLogUni);
-    const double lse = mx + log(exp(lv[0] - mx) + exp(lv[1] - mx) + exp(kLogUni - mx));
-    if (on && h == 0) loss -= lse;
-    const double rnet = exp(lv[0] - lse) + exp(lv[1] - lse);  // responsibility of the network part
-    // d loss / d outputs
+  for (int r = 0; r < 4; ++r)
+    if (4 * h + r < kOut) t.g4[4 * h + r][i] = zo[r];
+  wave_lds_sync();
+  {   // mixture, loss and d loss / d outputs in FP64: the lane's component k = h & 1, the other by a shuffle
+    const int k = h & 1;
+    const float o0 = t.g4[3 * k][i], o1 = t.g4[3 * k + 1][i], o2 = t.g4[3 * k + 2][i], p1 = t.g4[4 - 3 * k][i];
+    wave_lds_sync();
+    const V3 ghat = rec_vec(rv, 1), ax = rec_vec(rv, 4), sp = rec_vec(rv, 7);
     const V3 e = tilt_frame(ghat, ax);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const double rk = exp(lv[k] - lse);      // responsibility of component k
-      const double kap = m.kappa[k];
-      const double dlk = 1.0 / kap - 2.0 / expm1(2.0 * kap) + (dot(m.mu[k], s) - 1.0);  // d log f / d kappa
-      const double sraw = (double)o[3 * k];
-      const double dks = (sraw > -8.0 && sraw < 8.0) ? (kap - 1e-6) : 0.0;              // d kappa / d o
-      g4[3 * k] = (float)(-rk * dlk * dks);
-      g4[3 * k + 1] = (float)(exp(m.logw[k] - kLog1mU) * rnet - rk);
-      const double tt = m.t[k];
-      const double th = tt / (0.5 * kPi);
-      const V3 dmu = {-sin(tt) * ghat.x + cos(tt) * e.x, -sin(tt) * ghat.y + cos(tt) * e.y,
-                      -sin(tt) * ghat.z + cos(tt) * e.z};
-      g4[3 * k + 2] = (float)(-rk * kap * dot(dmu, s) * 0.5 * kPi * (1.0 - th * th));
+    const Comp m = make_comp(o0, o1, o2, p1, rv[0], ghat, e);
+    const double lv = log_part(m, sp), lse = log_mix(lv, __shfl_xor(lv, 16));
+    if (h == 0) t.loss[i] = on ? -lse : 0.0;
+    const double rk = exp(lv - lse);             // responsibility of the component
+    const double rnet = rk + __shfl_xor(rk, 16); // ... of the network part
+    const double dlk = 1.0 / m.kappa - 2.0 / expm1(2.0 * m.kappa) + (dot(m.mu, sp) - 1.0);  // d log f / d kappa
+    const double sraw = (double)o0;
+    const double dks = (sraw > -8.0 && sraw < 8.0) ? (m.kappa - 1e-6) : 0.0;                // d kappa / d o
+    const double th = m.t / (0.5 * kPi);
+    double sn, cs;
+    sincos(m.t, &sn, &cs);
+    const V3 dmu = {-sn * ghat.x + cs * e.x, -sn * ghat.y + cs * e.y, -sn * ghat.z + cs * e.z};
+    if (h < 2) {
+      t.g4[3 * k][i] = on ? (float)(-rk * dlk * dks) : 0.f;
+      t.g4[3 * k + 1][i] = on ? (float)(exp(m.logw - kLog1mU) * rnet - rk) : 0.f;
+      t.g4[3 * k + 2][i] = on ? (float)(-rk * m.kappa * dot(dmu, sp) * 0.5 * kPi * (1.0 - th * th)) : 0.f;
     }
-#pragma unroll
-    for (int q = 0; q < kOut; ++q) g4[q] = on ? g4[q] : 0.f;   // spare records add nothing
-    floatx16 d3, d2, d1;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      float acc = 0.f;
-#pragma unroll
-      for (int q = 0; q < kOut; ++q) acc += s_w4[q * kH + d_unit(v, h)] * g4[q];
-      d3[v] = acc * g3[v];
-    }
-    d2 = mat32(w3t, d3, floatx16{});
-#pragma unroll
-    for (int v = 0; v < 16; ++v) d2[v] *= g2[v];
-    d1 = mat32(w2t, d2, floatx16{});
-#pragma unroll
-    for (int v = 0; v < 16; ++v) d1[v] *= g1[v];
-    // weight gradients; rows of the right factor past its units are zero (one wave: LDS
-    // operations are in order, the barriers only keep the compiler from moving them)
-    auto rows = [&](const floatx16 &left, const floatx16 &right) {
-      __syncthreads();
-      put_rows(s_l, left, l, h);
-      put_rows(s_r, right, l, h);
-      __syncthreads();
-    };
-    rows(d3, a2);
-    dw3 = outer32(s_l, s_r, l, h, dw3, &db3);
-    rows(d2, a1);
-    dw2 = outer32(s_l, s_r, l, h, dw2, &db2);
-    __syncthreads();
-    put_rows(s_l, d1, l, h);
-    if (h == 0) {
-#pragma unroll
-      for (int k = 0; k < kIn; ++k) s_r[k * kTrow + l] = x[k];
-      s_r[kIn * kTrow + l] = 1.f;                               // column kIn: the bias
-    } else {
-      for (int k = kIn + 1; k < kH; ++k) s_r[k * kTrow + l] = 0.f;
-    }
-    __syncthreads();
-    dw1 = outer32(s_l, s_r, l, h, dw1, nullptr);
-    __syncthreads();
-    put_rows(s_r, a3, l, h);
-    if (h == 0) {
-#pragma unroll
-      for (int q = 0; q < kOut; ++q) s_l[q * kTrow + l] = g4[q];
-    } else {
-      for (int q = kOut; q < kH; ++q) s_l[q * kTrow + l] = 0.f;
-    }
-    __syncthreads();
-    dw4 = outer32(s_l, s_r, l, h, dw4, &db4);
+    wave_lds_sync();
   }
-  db2 += __shfl_xor(db2, 32, 64);
-  db3 += __shfl_xor(db3, 32, 64);
-  db4 += __shfl_xor(db4, 32, 64);
+  auto back = [&](float (&d)[kH][kTrow], const F4 (&g)[2]) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d[16 * m + 4 * h + r][i] = z[m][r] * g[m][r];
+    wave_lds_sync();
+  };
+  const float q0 = t.g4[h][i], q1 = h < 2 ? t.g4[4 + (h & 1)][i] : 0.f;   // output deltas h and 4 + h
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+    z[m] = mfma4(t.w4[4 + h][16 * m + c], q1, mfma4(t.w4[h][16 * m + c], q0, F4{0.f, 0.f, 0.f, 0.f}));
+  back(t.d3, g3);
+  z[0] = z[1] = F4{0.f, 0.f, 0.f, 0.f};
+  layer_mfma<true>(t.w3, t.d3, i, h, c, z);
+  back(t.d2, g2);
+  z[0] = z[1] = F4{0.f, 0.f, 0.f, 0.f};
+  layer_mfma<true>(t.w2, t.d2, i, h, c, z);
+  back(t.d1, g1);
+  __syncthreads();
+
   float *g = part_grad + (size_t)blockIdx.x * kNP;
+  auto mad4 = [](float s, const float4 &d, const float4 &a) {
+    return mad(mad(mad(mad(s, d.x, a.x), d.y, a.y), d.z, a.z), d.w, a.w);
+  };
+  auto ld4 = [](const float *p) { return *reinterpret_cast<const float4 *>(p); };
+  {   // 2 x 2 entries of a square layer, the third by waves 0-3, the second by waves 4-7
+    const bool third = tid < kTrainThreads / 2;
+    const int e = tid & (kTrainThreads / 2 - 1), r = 2 * (e / (kH / 2)), k = 2 * (e % (kH / 2));
+    const float *d = third ? t.d3[r] : t.d2[r], *a = third ? t.a2[k] : t.a1[k];
+    float s[2][2] = {};
+#pragma unroll 4
+    for (int q = 0; q < kTrainRec; q += 4) {
+      const float4 p[2] = {ld4(d + q), ld4(d + kTrow + q)}, v[2] = {ld4(a + q), ld4(a + kTrow + q)};
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int i = d_unit(v, h);
-    g[oW2 + i * kH + l] = dw2[v];
-    g[oW3 + i * kH + l] = dw3[v];
-    if (l < kIn) g[oW1 + i * kIn + l] = dw1[v];
-    else if (l == kIn) g[oB1 + i] = dw1[v];
-    if (i < kOut) g[oW4 + i * kH + l] = dw4[v];
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int l = 0; l < 2; ++l) s[m][l] = mad4(s[m][l], p[m], v[l]);
+    }
+    float *go = g + (third ? oW3 : oW2) + r * kH + k;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int l = 0; l < 2; ++l) go[m * kH + l] = s[m][l];
   }
-  if (h == 0) {
-    g[oB2 + l] = db2;
-    g[oB3 + l] = db3;
-    if (l < kOut) g[oB4 + l] = db4;
+  // first and output layers, biases (delta times 1): one entry of a list per thread
+  constexpr int nW1 = kH * kIn, nW4 = kOut * kH, nB = 3 * kH + kOut;
+  static_assert(nW1 + nW4 + nB < kTrainThreads, "one entry per thread, the last thread sums the losses");
+  if (tid < nW1 + nW4 + nB) {
+    const float *d, *a = t.one;
+    int p = tid, o;
+    if (p < nW1) { d = t.d1[p / kIn]; a = t.x[p % kIn]; o = oW1 + p; }
+    else if ((p -= nW1) < nW4) { d = t.g4[p / kH]; a = t.a3[p % kH]; o = oW4 + p; }
+    else if ((p -= nW4) < kH) { d = t.d1[p]; o = oB1 + p; }
+    else if ((p -= kH) < kH) { d = t.d2[p]; o = oB2 + p; }
+    else if ((p -= kH) < kH) { d = t.d3[p]; o = oB3 + p; }
+    else { p -= kH; d = t.g4[p]; o = oB4 + p; }
+    float s = 0.f;
+#pragma unroll 4
+    for (int q = 0; q < kTrainRec; q += 4) s = mad4(s, ld4(d + q), ld4(a + q));
+    g[o] = s;
   }
-  for (int q = 16; q > 0; q >>= 1) loss += __shfl_xor(loss, q, 64);   // lanes of half 1 hold zeros
-  if (lane == 0) part_loss[blockIdx.x] = loss;
+  if (tid == kTrainThreads - 1) {
+    double l = 0.0;
+#pragma unroll 16
+    for (int q = 0; q < kTrainRec; ++q) l += t.loss[q];
+    part_loss[blockIdx.x] = l;
+  }
 }
 
 // Adam on the FP32 master weights; writes the BF16 copy used by the sweep.
@@ -782,29 +777,22 @@ struct AdamArgs {
   int t;                              // step, from 1; 0: gradient only
 };
 
-// Mean gradient and loss from the waves' partial sums (64 parameters per block, the partials in
-// four slices summed in order), then the Adam step of these parameters in the same launch.
-__global__ __launch_bounds__(256) void k_train_reduce(const float *part_grad, const double *part_loss, int nw, int n,
-                                                      float *grad, double *loss, AdamArgs ad) {
-  __shared__ float s[256];
-  const int p = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
-  float g = 0.f;
-  if (p < kNP) {
-    const int b0 = nw * slice / 4, b1 = nw * (slice + 1) / 4;
+// Mean gradient and loss from the blocks' partial sums, block after block, then the Adam step in
+// the same launch (one thread per parameter; the last thread sums the losses).
+__global__ __launch_bounds__(64) void k_train_reduce(const float *part_grad, const double *part_loss, int nblk, int n,
+                                                     float *grad, double *loss, AdamArgs ad) {
+  const int p = blockIdx.x * 64 + threadIdx.x;
+  if (p == kNP) {
+    double l = 0.0;
 #pragma unroll 8
-    for (int b = b0; b < b1; ++b) g += part_grad[(size_t)b * kNP + p];
+    for (int b = 0; b < nblk; ++b) l += part_loss[b];
+    *loss = l / (double)n;
   }
-  s[threadIdx.x] = g;
-  __syncthreads();
-  if (blockIdx.x == 0 && threadIdx.x >= 64 && threadIdx.x < 128) {
-    double v = 0.0;
-    for (int b = threadIdx.x - 64; b < nw; b += 64) v += part_loss[b];
-    for (int q = 32; q > 0; q >>= 1) v += __shfl_xor(v, q, 64);
-    if (threadIdx.x == 64) *loss = v / (double)n;
-  }
-  if (slice != 0 || p >= kNP) return;
-  const int q = threadIdx.x;
-  const float gp = (s[q] + s[64 + q] + s[128 + q] + s[192 + q]) / (float)n;
+  if (p >= kNP) return;
+  float g = 0.f;
+#pragma unroll 16
+  for (int b = 0; b < nblk; ++b) g += part_grad[(size_t)b * kNP + p];
+  const float gp = g / (float)n;
   grad[p] = gp;
   if (ad.t == 0) return;
   const float m = ad.b1 * ad.mom[p] + (1.f - ad.b1) * gp;
@@ -851,13 +839,15 @@ __global__ __launch_bounds__(kEvalBlock) void k_eval(const float *w, const uint1
   }
   if (i >= n) return;
   const V3 ghat = rec_vec(rec, 6), ax = rec_vec(rec, 9), s = rec_vec(rec, 12);
-  const Mix m = make_mix(o, rec[5], ghat, ax);
+  const V3 e = tilt_frame(ghat, ax);
+  const Comp m0 = make_comp(o[0], o[1], o[2], o[4], rec[5], ghat, e);
+  const Comp m1 = make_comp(o[3], o[4], o[5], o[1], rec[5], ghat, e);
   double *q = out + (size_t)i * 10;
   for (int k = 0; k < kOut; ++k) q[k] = o[k];
-  q[6] = m.kappa[0];
-  q[7] = m.kappa[1];
-  q[8] = log_q(m, s);
-  q[9] = exp(m.logw[0] - kLog1mU);
+  q[6] = m0.kappa;
+  q[7] = m1.kappa;
+  q[8] = log_mix(log_part(m0, s), log_part(m1, s));
+  q[9] = exp(m0.logw - kLog1mU);
 }
 
 using LearnFn = void (*)(KArgs, const uint16_t *);
@@ -911,34 +901,35 @@ int ensure_records(esp_ctx *c, int need) {
   return ESP_OK;
 }
 
-// Waves of a gradient over n records.
-int train_waves(int n) { return std::min((n + kTile - 1) / kTile, kTrainWaves); }
+int train_blocks(int n) { return (n + kTrainRec - 1) / kTrainRec; }
 
 // Gradient scratch for minibatches of up to n records and up to nsteps losses.
 int ensure_grad_scratch(esp_ctx *c, int n, int nsteps) {
-  const int nw = train_waves(n);
+  const int nblk = train_blocks(n);
   int rc;
-  if (nw > c->pgrad_cap) {
+  if (nblk > c->pgrad_cap) {
     c->pgrad_cap = 0;
-    if ((rc = dalloc(c, c->d_pgrad, (size_t)nw * kNP)) || (rc = dalloc(c, c->d_ploss, nw))) return rc;
-    c->pgrad_cap = nw;
+    if ((rc = dalloc(c, c->d_pgrad, (size_t)nblk * kNP)) || (rc = dalloc(c, c->d_ploss, nblk))) return rc;
+    c->pgrad_cap = nblk;
   }
   if (nsteps > c->loss_cap) {
     c->loss_cap = 0;
     if ((rc = dalloc(c, c->d_loss, nsteps))) return rc;
     c->loss_cap = nsteps;
   }
+  HIPCHK(c, hipFuncSetAttribute((const void *)k_train_block, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)sizeof(TrainLds)));
   return ESP_OK;
 }
 
 // Gradient of the mean loss over records (perm ? perm[off + i] : off + i), i < n; loss to d_loss[k];
 // with ad.t > 0 also the Adam step.
 int enqueue_grad(esp_ctx *c, const int *perm, int off, int n, int k, const AdamArgs &ad) {
-  const int nw = train_waves(n);
-  hipLaunchKernelGGL(k_train_tiles, dim3(nw), dim3(64), 0, c->stream, (const float *)c->d_lw, (const float *)c->d_recs, n,
-                     perm, off, c->d_pgrad, c->d_ploss);
-  hipLaunchKernelGGL(k_train_reduce, dim3((kNP + 63) / 64), dim3(256), 0, c->stream, (const float *)c->d_pgrad,
-                     (const double *)c->d_ploss, nw, n, c->d_grad, c->d_loss + k, ad);
+  const int nblk = train_blocks(n);
+  hipLaunchKernelGGL(k_train_block, dim3(nblk), dim3(kTrainThreads), sizeof(TrainLds), c->stream, (const float *)c->d_lw,
+                     (const float *)c->d_recs, n, perm, off, c->d_pgrad, c->d_ploss);
+  hipLaunchKernelGGL(k_train_reduce, dim3(kNP / 64 + 1), dim3(64), 0, c->stream, (const float *)c->d_pgrad,
+                     (const double *)c->d_ploss, nblk, n, c->d_grad, c->d_loss + k, ad);
   HIPCHK(c, hipGetLastError());
   return ESP_OK;
 }

@@ -1,8 +1,8 @@
-"""The training gradient on tiles of 32 records against the oracle's FP64 gradient: one record,
-the edges of a tile, and more tiles than waves (several per wave, the last one partial).
+"""The training gradient against the oracle's FP64 gradient: one record, the edges of a wave's
+records (16) and of a block's (128), and many blocks, the last one partial.
 
 FP32 throughout: a unit's pre-activation sums 32 products and a gradient entry the records of a
-tile (then FP32 partial sums over waves), so entries are off by about sqrt(32) 2^-24 per layer
+block (then FP32 partial sums over blocks), so entries are off by about sqrt(32) 2^-24 per layer
 through seven layers of forward and backward, 3e-6 of the largest entry; the bound is 1e-4 of it
 (the oracle's mixture terms are FP64, the kernel's kappa and tilt FP32: 1e-6 relative on factors
 that reach beta |G| ~ 50)."""
@@ -16,7 +16,7 @@ from tests.test_learn_oracle import random_records
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 31, 32, 33, 512 * 32 + 33])
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 127, 128, 129, 512 * 32 + 33])
 def test_gradient_at_tile_edges(n):
     from espins_amd.engine import Engine
     print("records", n, flush=True)
