@@ -19,6 +19,7 @@
 #include "../../include/espins_hip.h"
 #include "esp_kernels.h"
 #include "esp_model.h"
+#include "esp_xfer.h"
 
 using namespace espd;
 using namespace espk;
@@ -220,6 +221,10 @@ struct esp_batch {
   std::vector<Var> vars;
   hipGraphExec_t gexec = nullptr;
   std::string gkey;
+  double *d_eout = nullptr;                 // energies of a chain on their way to the caller
+  int eout_cap = 0;
+  espx::Xfer xfer;
+  std::mutex read_mu;                       // read-outs share the buffers
 };
 
 namespace {
@@ -529,6 +534,7 @@ int esp_batch_create(esp_batch **out, int device) {
     return ESP_EHIP;
   }
   (void)hipMemset(b->d_done, 0, sizeof(unsigned));
+  espx::xfer_open(b->xfer, device);
   *out = b;
   return ESP_OK;
 }
@@ -540,6 +546,8 @@ int esp_batch_destroy(esp_batch *b) {
   (void)hipStreamSynchronize(b->side);
   drop_plan(b);
   for (auto &c : b->chains) free_chain(c);
+  bfree(b->d_eout);
+  espx::xfer_close(b->xfer);
   bfree(b->d_clock);
   bfree(b->d_done);
   (void)hipEventDestroy(b->fork);
@@ -734,9 +742,8 @@ int esp_batch_run(esp_batch *b, int n_rounds, int steps_per_round, int steps_mea
   if (b->gkey != key) {
     if ((rc = build_plan(b, tilt, seed))) return rc;
   }
-  Clock h{sweep0, step0, start_parity, 0};
-  BCHK(b, hipMemcpyAsync(b->d_clock, &h, sizeof(Clock), hipMemcpyHostToDevice, b->stream));
-  BCHK(b, hipStreamSynchronize(b->stream));
+  hipLaunchKernelGGL(k_set_clock, dim3(1), dim3(1), 0, b->stream, b->d_clock, Clock{sweep0, step0, start_parity, 0});
+  BCHK(b, hipGetLastError());
   if (!use_graph) {
     for (int k = 0; k < n_rounds; ++k)
       if ((rc = enqueue_round(b, steps_per_round, steps_measure, do_measure, do_exchange, mode))) return rc;
@@ -1045,6 +1052,8 @@ int esp_batch_get_stats(esp_batch *b, int k, double *acc, int64_t *rejected, dou
   int rc = check_chain(b, k);
   if (rc) return rc;
   Chain &c = b->chains[k];
+  std::lock_guard<std::mutex> lk(b->read_mu);
+  espx::SmallRead rd(b->xfer, b->stream);
   if (e_run) {
     // fresh running energies: partial sums over the replica, e_base + sum w
     KArgs a = chain_args(c, k);
@@ -1058,14 +1067,13 @@ int esp_batch_get_stats(esp_batch *b, int k, double *acc, int64_t *rejected, dou
     f.clock = b->d_clock;
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, b->stream, f);
     BCHK(b, hipGetLastError());
-    BCHK(b, hipMemcpyAsync(e_run, c.erun, sizeof(double) * c.R, hipMemcpyDeviceToHost, b->stream));
+    rd.add(e_run, c.erun, sizeof(double) * c.R);
   }
-  if (acc) BCHK(b, hipMemcpyAsync(acc, c.acc, sizeof(double) * 6 * c.R, hipMemcpyDeviceToHost, b->stream));
+  if (acc) rd.add(acc, c.acc, sizeof(double) * 6 * c.R);
   std::vector<int64_t> rsub(rejected ? (size_t)kRejSub * c.R : 0);
-  if (rejected)
-    BCHK(b, hipMemcpyAsync(rsub.data(), c.rej, sizeof(int64_t) * rsub.size(), hipMemcpyDeviceToHost, b->stream));
-  if (nmeas) BCHK(b, hipMemcpyAsync(nmeas, c.nmeas, sizeof(int64_t), hipMemcpyDeviceToHost, b->stream));
-  BCHK(b, hipStreamSynchronize(b->stream));
+  if (rejected) rd.add(rsub.data(), c.rej, sizeof(int64_t) * rsub.size());
+  if (nmeas) rd.add(nmeas, c.nmeas, sizeof(int64_t));
+  BCHK(b, rd.finish());
   if (rejected) sum_rej_sub(rsub, c.R, rejected);
   return ESP_OK;
 }
@@ -1075,9 +1083,11 @@ int esp_batch_get_map(esp_batch *b, int k, int *slot_rep, int64_t *nswap) {
   if (rc) return rc;
   Chain &c = b->chains[k];
   std::vector<int> sr(c.R);
-  BCHK(b, hipMemcpyAsync(sr.data(), c.slot_rep, sizeof(int) * c.R, hipMemcpyDeviceToHost, b->stream));
-  if (nswap) BCHK(b, hipMemcpyAsync(nswap, c.nswap, sizeof(int64_t) * 2 * c.R, hipMemcpyDeviceToHost, b->stream));
-  BCHK(b, hipStreamSynchronize(b->stream));
+  std::lock_guard<std::mutex> lk(b->read_mu);
+  espx::SmallRead rd(b->xfer, b->stream);
+  rd.add(sr.data(), c.slot_rep, sizeof(int) * c.R);
+  if (nswap) rd.add(nswap, c.nswap, sizeof(int64_t) * 2 * c.R);
+  BCHK(b, rd.finish());
   if (slot_rep)
     for (int t = 0; t < c.R; ++t) slot_rep[t] = sr[t] + 1;
   return ESP_OK;
@@ -1089,16 +1099,9 @@ int esp_batch_get_spins(esp_batch *b, int k, int by_slot, double *spins) {
   if (!spins) return bfail(b, ESP_EINVAL, "spins is NULL");
   Chain &c = b->chains[k];
   const int N = c.hm.N, R = c.R;
-  double *d_out = nullptr;
-  if ((rc = balloc(b, d_out, (size_t)3 * N * R))) return rc;
-  const size_t n = (size_t)N * R;
-  hipLaunchKernelGGL(k_get_spins, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, b->stream,
-                     (const double *)c.sp, (const int *)c.ref2dev,
-                     by_slot ? (const int *)c.slot_rep : (const int *)nullptr, N, c.Ns, R, d_out);
-  BCHK(b, hipGetLastError());
-  BCHK(b, hipMemcpyAsync(spins, d_out, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, b->stream));
-  BCHK(b, hipStreamSynchronize(b->stream));
-  bfree(d_out);
+  std::lock_guard<std::mutex> lk(b->read_mu);
+  BCHK(b, espx::xfer_spins(k_get_spins, b->xfer, b->device, b->stream, c.sp, c.ref2dev,
+                           by_slot ? c.slot_rep : nullptr, N, c.Ns, R, spins));
   return ESP_OK;
 }
 
@@ -1107,12 +1110,16 @@ int esp_batch_energy(esp_batch *b, int k, double *E) {
   if (rc) return rc;
   if (!E) return bfail(b, ESP_EINVAL, "E is NULL");
   Chain &c = b->chains[k];
-  double *d_e = nullptr;
-  if ((rc = balloc(b, d_e, c.R))) return rc;
-  if ((rc = chain_energy(b, k, d_e))) return rc;
-  BCHK(b, hipMemcpyAsync(E, d_e, sizeof(double) * c.R, hipMemcpyDeviceToHost, b->stream));
-  BCHK(b, hipStreamSynchronize(b->stream));
-  bfree(d_e);
+  std::lock_guard<std::mutex> lk(b->read_mu);
+  if (c.R > b->eout_cap) {
+    b->eout_cap = 0;
+    if ((rc = balloc(b, b->d_eout, c.R))) return rc;
+    b->eout_cap = c.R;
+  }
+  if ((rc = chain_energy(b, k, b->d_eout))) return rc;
+  espx::SmallRead rd(b->xfer, b->stream);
+  rd.add(E, b->d_eout, sizeof(double) * c.R);
+  BCHK(b, rd.finish());
   return ESP_OK;
 }
 
@@ -1120,13 +1127,10 @@ int esp_batch_reset_stats(esp_batch *b) {
   if (!b) return ESP_EINVAL;
   if (!b->committed) return bfail(b, ESP_ESTATE, "batch not committed");
   BCHK(b, hipSetDevice(b->device));
-  for (auto &c : b->chains) {
-    BCHK(b, hipMemsetAsync(c.acc, 0, sizeof(double) * 6 * c.R, b->stream));
-    BCHK(b, hipMemsetAsync(c.rej, 0, sizeof(unsigned long long) * kRejSub * c.R, b->stream));
-    BCHK(b, hipMemsetAsync(c.nswap, 0, sizeof(unsigned long long) * 2 * c.R, b->stream));
-    BCHK(b, hipMemsetAsync(c.nmeas, 0, sizeof(unsigned long long), b->stream));
-  }
-  BCHK(b, hipStreamSynchronize(b->stream));
+  for (auto &c : b->chains)
+    hipLaunchKernelGGL(k_zero_stats, dim3((kRejSub * c.R + 255) / 256), dim3(256), 0, b->stream, c.acc, c.rej, c.nswap,
+                       c.nmeas, c.R);
+  BCHK(b, hipGetLastError());
   return ESP_OK;
 }
 

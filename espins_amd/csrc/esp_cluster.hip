@@ -642,8 +642,12 @@ int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, in
     hipLaunchKernelGGL(fn, dim3(c->R * q->k), dim3(kCBlock), shm, c->stream, x);
     HIPCHK(c, hipGetLastError());
     Ctl h{};
-    HIPCHK(c, hipMemcpyAsync(&h, q->ctl, sizeof h, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    {
+      std::lock_guard<std::mutex> lk(c->read_mu);
+      espx::SmallRead rd(c->xfer, c->stream);
+      rd.add(&h, q->ctl, sizeof h);
+      HIPCHK(c, rd.finish());
+    }
     if (h.failed) return fail(c, ESP_EHIP, "cluster sweep: a block stopped making progress");
     if (h.decided != kGo) return ESP_OK;     // *ran: steps finished so far
     c->mpart_valid = false;

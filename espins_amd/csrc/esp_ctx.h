@@ -9,6 +9,7 @@
 #include "../../include/espins_hip.h"
 #include "esp_kernels.h"
 #include "esp_model.h"
+#include "esp_xfer.h"
 
 using espk::Clock;
 using espk::KArgs;
@@ -53,6 +54,9 @@ struct esp_ctx {
   unsigned long long *d_rej = nullptr, *d_nswap = nullptr, *d_nmeas = nullptr;
   Clock *d_clock = nullptr;
   unsigned *d_done = nullptr;    // blocks of k_reduce_fin done this step (the last one resets it)
+  double *d_eout = nullptr;      // [R] energies on their way to the caller
+  espx::Xfer xfer;
+  std::mutex read_mu;            // read-outs share the buffers
   std::vector<double> tems;
   // replicas shared by clusters of blocks (esp_cluster.hip): tables, or null where clusters do not
   // serve; decided for cluster_R replicas (0: not yet)
@@ -185,7 +189,8 @@ void drop_graph(esp_ctx *c) {
 }
 
 void free_replicas(esp_ctx *c) {
-  dfree(c->d_sp); dfree(c->d_w); dfree(c->d_beta); dfree(c->d_ebase); dfree(c->d_erun); dfree(c->d_acc);
+  dfree(c->d_sp); dfree(c->d_w); dfree(c->d_beta); dfree(c->d_ebase); dfree(c->d_erun); dfree(c->d_eout);
+  dfree(c->d_acc);
   dfree(c->d_partial); dfree(c->d_slot_rep); dfree(c->d_rep_slot); dfree(c->d_rej);
   dfree(c->d_nswap); dfree(c->d_nmeas); dfree(c->d_prop); dfree(c->d_unif); dfree(c->d_accd);
   dfree(c->d_trace);

@@ -287,9 +287,8 @@ int enqueue_reduce_finalize(esp_ctx *c, bool measure, bool exchange, int advance
 }
 
 int set_clock(esp_ctx *c, uint64_t sweep, uint64_t step, int parity) {
-  Clock h{sweep, step, parity, 0};
-  HIPCHK(c, hipMemcpyAsync(c->d_clock, &h, sizeof(Clock), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  hipLaunchKernelGGL(k_set_clock, dim3(1), dim3(1), 0, c->stream, c->d_clock, Clock{sweep, step, parity, 0});
+  HIPCHK(c, hipGetLastError());
   return ESP_OK;
 }
 
@@ -427,6 +426,7 @@ int esp_create(esp_ctx **out, int device) {
   // set-up of the allocation-free entry point on this device (its scratch address); a
   // failure here only disables esp_energy_noalloc, which then reports it
   (void)scratch_address(device);
+  espx::xfer_open(c->xfer, device);
   *out = c;
   return ESP_OK;
 }
@@ -439,6 +439,7 @@ int esp_destroy(esp_ctx *c) {
   free_model(c);
   esp::obs_free(c);
   esp::learn_free(c);
+  espx::xfer_close(c->xfer);
   dfree(c->d_clock);
   dfree(c->d_done);
   (void)hipStreamDestroy(c->stream);
@@ -652,6 +653,7 @@ int esp_set_replicas(esp_ctx *c, int R, const double *tems, const double *spins)
   if ((rc = dalloc(c, c->d_beta, R))) return rc;
   if ((rc = dalloc(c, c->d_ebase, R))) return rc;
   if ((rc = dalloc(c, c->d_erun, R))) return rc;
+  if ((rc = dalloc(c, c->d_eout, R))) return rc;
   if ((rc = dalloc(c, c->d_acc, (size_t)6 * R))) return rc;
   if ((rc = dalloc(c, c->d_partial, (size_t)4 * R * c->red_blocks))) return rc;
   if ((rc = dalloc(c, c->d_slot_rep, R))) return rc;
@@ -698,16 +700,9 @@ int esp_get_spins(esp_ctx *c, int by_slot, double *spins) {
   if (rc) return rc;
   if (!spins) return fail(c, ESP_EINVAL, "spins is NULL");
   const int N = c->hm.N, R = c->R;
-  double *d_out = nullptr;
-  if ((rc = dalloc(c, d_out, (size_t)3 * N * R))) return rc;
-  const size_t n = (size_t)N * R;
-  hipLaunchKernelGGL(k_get_spins, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream,
-                     (const double *)c->d_sp, (const int *)c->d_ref2dev,
-                     by_slot ? (const int *)c->d_slot_rep : (const int *)nullptr, N, c->Ns, R, d_out);
-  HIPCHK(c, hipGetLastError());
-  HIPCHK(c, hipMemcpyAsync(spins, d_out, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  dfree(d_out);
+  std::lock_guard<std::mutex> lk(c->read_mu);
+  HIPCHK(c, espx::xfer_spins(k_get_spins, c->xfer, c->device, c->stream, c->d_sp, c->d_ref2dev,
+                             by_slot ? c->d_slot_rep : nullptr, N, c->Ns, R, spins));
   return ESP_OK;
 }
 
@@ -715,12 +710,11 @@ int esp_energy(esp_ctx *c, double *E) {
   int rc = check_ready(c, true);
   if (rc) return rc;
   if (!E) return fail(c, ESP_EINVAL, "E is NULL");
-  double *d_e = nullptr;
-  if ((rc = dalloc(c, d_e, c->R))) return rc;
-  if ((rc = enqueue_energy(c, d_e))) return rc;
-  HIPCHK(c, hipMemcpyAsync(E, d_e, sizeof(double) * c->R, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  dfree(d_e);
+  std::lock_guard<std::mutex> lk(c->read_mu);
+  if ((rc = enqueue_energy(c, c->d_eout))) return rc;
+  espx::SmallRead rd(c->xfer, c->stream);
+  rd.add(E, c->d_eout, sizeof(double) * c->R);
+  HIPCHK(c, rd.finish());
   return ESP_OK;
 }
 
@@ -947,17 +941,18 @@ int esp_get_stats(esp_ctx *c, double *acc, int64_t *rejected, double *e_run, int
   int rc = check_ready(c, true);
   if (rc) return rc;
   const int R = c->R;
+  std::lock_guard<std::mutex> lk(c->read_mu);
+  espx::SmallRead rd(c->xfer, c->stream);
   if (e_run) {
     if ((rc = enqueue_reduce(c))) return rc;
     if ((rc = enqueue_finalize(c, true, false, false, 0, 0))) return rc;
-    HIPCHK(c, hipMemcpyAsync(e_run, c->d_erun, sizeof(double) * R, hipMemcpyDeviceToHost, c->stream));
+    rd.add(e_run, c->d_erun, sizeof(double) * R);
   }
-  if (acc) HIPCHK(c, hipMemcpyAsync(acc, c->d_acc, sizeof(double) * 6 * R, hipMemcpyDeviceToHost, c->stream));
+  if (acc) rd.add(acc, c->d_acc, sizeof(double) * 6 * R);
   std::vector<int64_t> rsub(rejected ? (size_t)kRejSub * R : 0);
-  if (rejected)
-    HIPCHK(c, hipMemcpyAsync(rsub.data(), c->d_rej, sizeof(int64_t) * rsub.size(), hipMemcpyDeviceToHost, c->stream));
-  if (nmeas) HIPCHK(c, hipMemcpyAsync(nmeas, c->d_nmeas, sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (rejected) rd.add(rsub.data(), c->d_rej, sizeof(int64_t) * rsub.size());
+  if (nmeas) rd.add(nmeas, c->d_nmeas, sizeof(int64_t));
+  HIPCHK(c, rd.finish());
   if (rejected) sum_rej_sub(rsub, R, rejected);
   return ESP_OK;
 }
@@ -967,10 +962,11 @@ int esp_get_map(esp_ctx *c, int *slot_rep, int64_t *nswap) {
   if (rc) return rc;
   const int R = c->R;
   std::vector<int> sr(R);
-  HIPCHK(c, hipMemcpyAsync(sr.data(), c->d_slot_rep, sizeof(int) * R, hipMemcpyDeviceToHost, c->stream));
-  if (nswap)
-    HIPCHK(c, hipMemcpyAsync(nswap, c->d_nswap, sizeof(int64_t) * 2 * R, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  std::lock_guard<std::mutex> lk(c->read_mu);
+  espx::SmallRead rd(c->xfer, c->stream);
+  rd.add(sr.data(), c->d_slot_rep, sizeof(int) * R);
+  if (nswap) rd.add(nswap, c->d_nswap, sizeof(int64_t) * 2 * R);
+  HIPCHK(c, rd.finish());
   if (slot_rep)
     for (int t = 0; t < R; ++t) slot_rep[t] = sr[t] + 1;
   return ESP_OK;
@@ -1012,13 +1008,10 @@ int esp_reset_stats(esp_ctx *c) {
   int rc = check_ready(c, true);
   if (rc) return rc;
   const int R = c->R;
-  HIPCHK(c, hipMemsetAsync(c->d_acc, 0, sizeof(double) * 6 * R, c->stream));
-  HIPCHK(c, hipMemsetAsync(c->d_rej, 0, sizeof(unsigned long long) * kRejSub * R, c->stream));
-  HIPCHK(c, hipMemsetAsync(c->d_nswap, 0, sizeof(unsigned long long) * 2 * R, c->stream));
-  HIPCHK(c, hipMemsetAsync(c->d_nmeas, 0, sizeof(unsigned long long), c->stream));
-  if ((rc = esp::obs_clear(c))) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  return ESP_OK;
+  hipLaunchKernelGGL(k_zero_stats, dim3((kRejSub * R + 255) / 256), dim3(256), 0, c->stream, c->d_acc, c->d_rej,
+                     c->d_nswap, c->d_nmeas, R);
+  HIPCHK(c, hipGetLastError());
+  return esp::obs_clear(c);      // (in stream order: every later call sees them cleared)
 }
 
 int esp_sync(esp_ctx *c) {

@@ -923,16 +923,30 @@ __global__ void k_put_spins(const double *in, const int *ref2dev, int N, int Ns,
   x[d] = p[0]; x[Ns + d] = p[1]; x[2 * Ns + d] = p[2];
 }
 
+// Spins out: sites t0 .. t0 + n - 1 of the [R][N] reference order.
 __global__ void k_get_spins(const double *sp, const int *ref2dev, const int *src_rep, int N, int Ns,
-                            int R, double *out) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)N * R) return;
+                            size_t t0, size_t n, double *out) {
+  const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const size_t t = t0 + k;
   const int q = (int)(t / N), i = (int)(t % N);
   const int r = src_rep ? src_rep[q] : q;
   const double *x = sp + (size_t)r * 3 * Ns;
   const int d = ref2dev[i];
-  double *p = out + 3 * t;
+  double *p = out + 3 * k;
   p[0] = x[d]; p[1] = x[Ns + d]; p[2] = x[2 * Ns + d];
+}
+
+__global__ void k_set_clock(Clock *c, Clock v) { *c = v; }
+
+// Statistics to zero: estimators, rejections, swaps, measurement count.
+__global__ void k_zero_stats(double *acc, unsigned long long *rej, unsigned long long *nswap,
+                             unsigned long long *nmeas, int R) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < 6 * R) acc[t] = 0.0;
+  if (t < kRejSub * R) rej[t] = 0;
+  if (t < 2 * R) nswap[t] = 0;
+  if (t == 0) *nmeas = 0;
 }
 
 // Plain streaming copy (grid-stride, 32 B per lane per iteration): calibrates the HBM

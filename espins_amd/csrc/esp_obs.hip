@@ -1025,42 +1025,36 @@ int esp_get_obs(esp_ctx *c, int which, double *out, int64_t *count) {
   if (!(b.flags & which) || c->R == 0) return fail(c, ESP_ESTATE, "esp_get_obs: observable not on");
   if (hipSetDevice(c->device) != hipSuccess) return fail(c, ESP_EHIP, "hipSetDevice");
   const int R = c->R;
-  if (count) {
-    unsigned long long n = 0;
-    HIPCHK(c, hipMemcpyAsync(&n, which == ESP_OBS_SFACTOR ? b.d_sfn : c->d_nmeas, sizeof n,
-                             hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    *count = (int64_t)n;
-  }
+  std::lock_guard<std::mutex> lk(c->read_mu);
+  espx::SmallRead rd(c->xfer, c->stream);
+  unsigned long long n = 0;
+  if (count) rd.add(&n, which == ESP_OBS_SFACTOR ? b.d_sfn : c->d_nmeas, sizeof n);
+  std::vector<double> a;
+  std::vector<unsigned long long> h;
   if (which == ESP_OBS_ORDER || which == ESP_OBS_STAGGERED) {
-    std::vector<double> a((size_t)R * 6);
-    HIPCHK(c, hipMemcpyAsync(a.data(), b.d_acc, sizeof(double) * a.size(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    a.resize((size_t)R * 6);
+    rd.add(a.data(), b.d_acc, sizeof(double) * a.size());
+  } else if (which == ESP_OBS_PM) {
+    h.resize((size_t)R * ndim_pm(c) * b.nfreq);
+    rd.add(h.data(), b.d_pm, sizeof(unsigned long long) * h.size());
+  } else if (which == ESP_OBS_SPINCORR) {
+    rd.add(out, b.d_sc, sizeof(double) * R * 3 * b.nshell * b.nsp * b.nsp);
+  } else if (which == ESP_OBS_SFACTOR) {
+    rd.add(out, b.d_sf, sizeof(double) * R * 3 * b.nq);
+  }
+  HIPCHK(c, rd.finish());
+  if (count) *count = (int64_t)n;
+  if (!a.empty()) {
     const int o = which == ESP_OBS_ORDER ? 0 : 3;
     for (int r = 0; r < R; ++r)
       for (int k = 0; k < 3; ++k) out[3 * r + k] = a[6 * (size_t)r + o + k];
-    return ESP_OK;
   }
-  if (which == ESP_OBS_PM) {
-    std::vector<unsigned long long> h((size_t)R * ndim_pm(c) * b.nfreq);
-    HIPCHK(c, hipMemcpyAsync(h.data(), b.d_pm, sizeof(unsigned long long) * h.size(), hipMemcpyDeviceToHost,
-                             c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (size_t k = 0; k < h.size(); ++k) out[k] = (double)h[k];
-    return ESP_OK;
-  }
-  if (which == ESP_OBS_SPINCORR) {
-    HIPCHK(c, hipMemcpyAsync(out, b.d_sc, sizeof(double) * R * 3 * b.nshell * b.nsp * b.nsp,
-                             hipMemcpyDeviceToHost, c->stream));
-  } else if (which == ESP_OBS_SFACTOR) {
-    HIPCHK(c, hipMemcpyAsync(out, b.d_sf, sizeof(double) * R * 3 * b.nq, hipMemcpyDeviceToHost, c->stream));
-  } else {
+  for (size_t k = 0; k < h.size(); ++k) out[k] = (double)h[k];
+  if (which != ESP_OBS_ORDER && which != ESP_OBS_STAGGERED && which != ESP_OBS_PM && which != ESP_OBS_SPINCORR &&
+      which != ESP_OBS_SFACTOR)
     return fail(c, ESP_EINVAL, "esp_get_obs: unknown observable");
-  }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   return ESP_OK;
 }
-
 int esp_get_obs_trace(esp_ctx *c, double *trace, int *n) {
   if (!c || !n) return ESP_EINVAL;
   auto &b = c->obs;
