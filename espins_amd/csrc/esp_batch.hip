@@ -102,6 +102,7 @@ using BLdsFn = void (*)(const KArgs *, const LdsMeas *, const int2 *, int, int);
 // variant bits: 0-1 coefficient layout (LAY_*), 2 biquadratic, 3 DM, 4 self bonds; launch
 // variants add bit 5: the wide setting of the partner gathers in flight per lane (global path)
 constexpr int kVarChunk4 = 32;
+constexpr size_t kGroupBytes = size_t(192) << 20;   // spins of a replica group
 constexpr int kNarrow = 2;   // the narrow setting, as set_chain_chunk and info name it
 template <int MODE, int LAY, bool HB, bool HD, int CH>
 BPhaseFn bp4(bool self) { return self ? k_bphase<MODE, LAY, HB, HD, true, CH> : k_bphase<MODE, LAY, HB, HD, false, CH>; }
@@ -212,13 +213,14 @@ struct esp_batch {
   // per variant: tiles per colour, LDS items
   struct Var {
     int variant = 0;
-    std::vector<int4 *> d_tiles;          // per colour
+    std::vector<int4 *> d_tiles;          // per replica group and colour
     std::vector<int> ntiles;
     int2 *d_lds = nullptr;
     int nlds = 0;
     size_t shm_phase = 0, shm_lds = 0;
   };
   std::vector<Var> vars;
+  int ngroups = 1;                          // replica groups that run their colours one after the other
   hipGraphExec_t gexec = nullptr;
   std::string gkey;
   double *d_eout = nullptr;                 // energies of a chain on their way to the caller
@@ -384,27 +386,58 @@ int build_plan(esp_batch *b, double tilt, uint64_t seed) {
       b->vars.emplace_back();
       b->vars.back().variant = launch_variant(c);
     }
+  // Replica groups: a sweep runs all colours of one group, then of the next.  A colour phase reads
+  // most of its replicas' spins, so the phases of more state than the memory-side cache (256 MB)
+  // come from HBM each time; a launch more costs about 4 us.  24 chains of 369 MB, 60 rounds, in
+  // groups of 32 / 64 / 96 / 128 / 192 MB and in one: 65 / 52 / 46 / 43 / 41 / 43 ms.
+  // Chains with as many colours stand together (a group's last colours would run a few chains).
+  std::vector<std::vector<int4>> groups;              // (chain, first replica, end)
+  {
+    std::vector<int> order;
+    for (int k = 0; k < nc; ++k)
+      if (!b->chains[k].lds) order.push_back(k);
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b->chains[x].hm.ncol > b->chains[y].hm.ncol; });
+    size_t total = 0, left = 0;
+    for (int k : order) total += sizeof(double) * 3 * b->chains[k].Ns * b->chains[k].R;
+    const size_t ng = std::max<size_t>(1, (total + kGroupBytes / 2) / kGroupBytes);
+    for (int k : order) {
+      const size_t rep = sizeof(double) * 3 * b->chains[k].Ns;
+      for (int r = 0; r < b->chains[k].R; ++r) {
+        if (groups.empty() || (left < rep / 2 && groups.size() < ng)) {
+          groups.emplace_back();
+          left += total / ng;
+        }
+        auto &g = groups.back();
+        if (g.empty() || g.back().x != k) g.push_back(make_int4(k, r, r, 0));
+        g.back().z = r + 1;
+        left -= std::min(left, rep);
+      }
+    }
+    if (groups.empty()) groups.emplace_back();
+  }
+  b->ngroups = (int)groups.size();
   for (auto &v : b->vars) {
     // Global-path tiles per colour.  Tile t runs on XCD t % 8 and all tiles of one replica share
     // an XCD (and its L2).  Replicas go, largest first, to the XCD with the fewest tiles so far:
     // dealt out in turn, the replicas of a chain differ by one between XCDs, and a few large
     // chains left XCDs idle at the end of the launch.
-    v.d_tiles.assign(b->maxcol, nullptr);
-    v.ntiles.assign(b->maxcol, 0);
-    for (int col = 0; col < b->maxcol; ++col) {
-      std::vector<std::pair<int, int>> unit;           // (blocks per replica, chain)
-      for (int k = 0; k < nc; ++k) {
-        const Chain &c = b->chains[k];
-        if (launch_variant(c) != v.variant || c.lds || col >= c.hm.ncol) continue;
+    v.d_tiles.assign((size_t)b->ngroups * b->maxcol, nullptr);
+    v.ntiles.assign((size_t)b->ngroups * b->maxcol, 0);
+    for (int slot = 0; slot < b->ngroups * b->maxcol; ++slot) {
+      const int col = slot % b->maxcol;
+      std::vector<std::pair<int, int4>> unit;          // (blocks per replica, replicas)
+      for (const int4 &u : groups[slot / b->maxcol]) {
+        const Chain &c = b->chains[u.x];
+        if (launch_variant(c) != v.variant || col >= c.hm.ncol) continue;
         // (geometry-group tiles are numbered in sub-cell order across the groups)
-        unit.push_back({colour_blocks(c.hm, col, c.tps, chain_geo(c)), k});
+        unit.push_back({colour_blocks(c.hm, col, c.tps, chain_geo(c)), u});
       }
       std::stable_sort(unit.begin(), unit.end(), [](const auto &x, const auto &y) { return x.first > y.first; });
       std::vector<std::vector<int4>> q(8);
-      for (const auto &[nblk, k] : unit)
-        for (int r = 0; r < b->chains[k].R; ++r) {
+      for (const auto &[nblk, u] : unit)
+        for (int r = u.y; r < u.z; ++r) {
           auto &x = *std::min_element(q.begin(), q.end(), [](const auto &m, const auto &n) { return m.size() < n.size(); });
-          for (int bb = 0; bb < nblk; ++bb) x.push_back(make_int4(k, r, bb, 0));
+          for (int bb = 0; bb < nblk; ++bb) x.push_back(make_int4(u.x, r, bb, 0));
         }
       size_t longest = 0;
       for (auto &x : q) longest = std::max(longest, x.size());
@@ -414,8 +447,8 @@ int build_plan(esp_batch *b, double tilt, uint64_t seed) {
           tiles.push_back(i < q[x].size() ? q[x][i] : make_int4(-1, 0, 0, 0));
       // trim trailing padding
       while (!tiles.empty() && tiles.back().x < 0) tiles.pop_back();
-      v.ntiles[col] = (int)tiles.size();
-      if (!tiles.empty() && (rc = bupload(b, v.d_tiles[col], tiles.data(), tiles.size()))) return rc;
+      v.ntiles[slot] = (int)tiles.size();
+      if (!tiles.empty() && (rc = bupload(b, v.d_tiles[slot], tiles.data(), tiles.size()))) return rc;
     }
     std::vector<int2> li;
     size_t shm_l = 0, shm_p = 0;
@@ -458,12 +491,12 @@ int enqueue_round(esp_batch *b, int steps, int M, bool measure, bool exchange, i
   }
   for (int s = 0; s < steps; ++s) {
     for (int m = 0; m < M; ++m)
-      for (int col = 0; col < b->maxcol; ++col)
+      for (int slot = 0; slot < b->ngroups * b->maxcol; ++slot)
         for (auto &v : b->vars)
-          if (v.ntiles[col] > 0)
-            hipLaunchKernelGGL(bphase_fn(mode, v.variant), dim3(v.ntiles[col]), dim3(kPhaseBlock), v.shm_phase,
-                               b->stream, (const KArgs *)b->d_chains, (const int4 *)v.d_tiles[col], col,
-                               s * M + m);
+          if (v.ntiles[slot] > 0)
+            hipLaunchKernelGGL(bphase_fn(mode, v.variant), dim3(v.ntiles[slot]), dim3(kPhaseBlock), v.shm_phase,
+                               b->stream, (const KArgs *)b->d_chains, (const int4 *)v.d_tiles[slot],
+                               slot % b->maxcol, s * M + m);
     BCHK(b, hipGetLastError());
     const bool last = s + 1 == steps;
     if (measure && b->n_red_items > 0)
@@ -1001,19 +1034,19 @@ int esp_batch_time_sweeps(esp_batch *b, int nsweeps, int mode, uint64_t seed, ui
   Clock h{sweep0, 0, 1, 0};
   BCHK(b, hipMemcpyAsync(b->d_clock, &h, sizeof(Clock), hipMemcpyHostToDevice, b->stream));
   int per = 0;
-  for (int col = 0; col < b->maxcol; ++col)
-    for (auto &v : b->vars) per += v.ntiles[col] > 0;
+  for (int slot = 0; slot < b->ngroups * b->maxcol; ++slot)
+    for (auto &v : b->vars) per += v.ntiles[slot] > 0;
   if (per == 0) return bfail(b, ESP_ESTATE, "no global-memory chains to time");
   std::vector<hipEvent_t> ev(2 * (size_t)per * nsweeps, nullptr);
   for (auto &e : ev) BCHK(b, hipEventCreate(&e));
   int k = 0;
   for (int s = 0; s < nsweeps; ++s)
-    for (int col = 0; col < b->maxcol; ++col)
+    for (int slot = 0; slot < b->ngroups * b->maxcol; ++slot)
       for (auto &v : b->vars)
-        if (v.ntiles[col] > 0) {
-          hipExtLaunchKernelGGL(bphase_fn(mode, v.variant), dim3(v.ntiles[col]), dim3(kPhaseBlock), v.shm_phase,
+        if (v.ntiles[slot] > 0) {
+          hipExtLaunchKernelGGL(bphase_fn(mode, v.variant), dim3(v.ntiles[slot]), dim3(kPhaseBlock), v.shm_phase,
                                 b->stream, ev[2 * k], ev[2 * k + 1], 0, (const KArgs *)b->d_chains,
-                                (const int4 *)v.d_tiles[col], col, s);
+                                (const int4 *)v.d_tiles[slot], slot % b->maxcol, s);
           ++k;
         }
   BCHK(b, hipGetLastError());
