@@ -86,12 +86,10 @@ __global__ __launch_bounds__(1024) void k_bfinal(const FinArgs *fa, Clock *clock
   finalize_body(f, start, step);  // (LDS chains count their measurements in their kernel)
   __syncthreads();
   if (threadIdx.x == 0) {
-    __threadfence();
-    const unsigned t = atomicAdd(done, 1u);
-    if (t == gridDim.x - 1) {
+    // (every block has read the clock above; nothing else passes between blocks, so no fence)
+    if (__hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
       advance_clock(clock, exchange, advance);
       *done = 0u;
-      __threadfence();
     }
   }
 }

@@ -73,18 +73,10 @@ struct CArgs {
   int nsteps, M, measure, exchange, round;        // exchange after every `round` steps
 };
 
-template <class T>
-__device__ __forceinline__ T ald(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-template <class T>
-__device__ __forceinline__ void ast(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
-// What blocks exchange during a launch -- spins, partial sums, slots, flags -- moves by agent-scope
-// atomic loads and stores only, which act at the GPU's coherence point, past the L1s and the
-// XCDs' L2s.  Before a block raises a flag every wave waits until its stores have been
-// acknowledged there (stores_done) and then for the block's other waves, so what a flag announces
-// is in place when the flag is; no cache needs writing back or invalidating (agent-scope release
-// and acquire fences do both, for whole caches: 10 us per colour phase, against 3).
-__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// What blocks exchange during a launch -- spins, partial sums, slots, flags -- moves by ald and ast
+// only.  Before a block raises a flag every wave waits until its stores have been acknowledged
+// (stores_done) and then for the block's other waves, so what a flag announces is in place when
+// the flag is (with release and acquire fences a colour phase took 10 us, against 3).
 
 // Waits until *p >= want; false after 60 s without it (only a lost block could cause that).
 __device__ __forceinline__ bool wait_ge(const unsigned *p, unsigned want, const Ctl *ctl) {
