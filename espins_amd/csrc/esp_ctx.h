@@ -69,10 +69,11 @@ struct esp_ctx {
   // per-wave spin sums of the colour phases: [R][ncol][mpart_nw][3]; valid while the last
   // change of the spins was a full global-path sweep (d_w has the same wave layout).  The
   // waves' layout: geometry-group tiles or not, lanes per site
-  double *d_mpart = nullptr;
+  double *d_mpart = nullptr, *d_mpart_l = nullptr;   // _l: the learned phases' own (other entries)
   int mpart_nw = 0, mpart_tps = 0;
   bool mpart_geo = false;
   bool mpart_valid = false;
+  bool mpart_learned = false;    // the valid sums are d_mpart_l
   // per-measurement trace of E and |m| by slot (global-memory path only)
   double *d_trace = nullptr;      // [trace_cap][R][2]
   int trace_cap = 0;
@@ -196,7 +197,7 @@ void free_replicas(esp_ctx *c) {
   dfree(c->d_trace);
   c->trace_cap = 0;
   c->w_dirty = false;
-  dfree(c->d_mpart);
+  dfree(c->d_mpart); dfree(c->d_mpart_l);
   c->mpart_nw = 0;
   c->mpart_valid = false;
   c->R = 0;

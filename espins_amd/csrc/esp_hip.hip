@@ -146,7 +146,9 @@ int check_ready(esp_ctx *c, bool need_replicas) {
 
 // Per-wave sums of the colour phases -- spins (mpart) and accepted dE (d_w) -- sized for the
 // current lanes per site and zeroed on (re)allocation: entries of waves a colour does not
-// have stay zero.  Before the accumulators are re-laid out their sums move into e_base.
+// have stay zero (the learned phases number their waves differently and keep sums of their own:
+// measured from the spins, 64 replicas of fcc 24^3 took 36 us a step, so 9).  Before the
+// accumulators are re-laid out their sums move into e_base.
 // Called before any capture, never inside one.
 int ensure_mpart(esp_ctx *c) {
   const esp::HostModel &m = c->hm;
@@ -154,7 +156,15 @@ int ensure_mpart(esp_ctx *c) {
   int need = 1;
   for (int col = 0; col < m.ncol; ++col)   // (host-fed sweeps take one lane per site)
     need = std::max({need, colour_waves(m, col, c->tps, geo), colour_waves(m, col, 1, phase_kernel_layout(c, 1) == LAY_IMP)});
-  if (c->d_mpart && c->d_w && need == c->mpart_nw && geo == c->mpart_geo && c->tps == c->mpart_tps) return ESP_OK;
+  if (c->d_mpart && c->d_w && need == c->mpart_nw && geo == c->mpart_geo && c->tps == c->mpart_tps) {
+    if (!c->have_learn || c->d_mpart_l) return ESP_OK;
+    const size_t bytes = 3 * sizeof(double) * c->R * m.ncol * need;   // the learned phases' sums, from now on
+    int rc = dalloc(c, c->d_mpart_l, bytes / sizeof(double));
+    if (rc) return rc;
+    HIPCHK(c, hipMemsetAsync(c->d_mpart_l, 0, bytes, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return ESP_OK;
+  }
   drop_graph(c);   // a captured round may hold the old buffers
   if (c->d_w && c->mpart_nw > 0) {
     hipLaunchKernelGGL(k_fold_w, dim3((c->R + 255) / 256), dim3(256), 0, c->stream, c->d_w,
@@ -166,6 +176,7 @@ int ensure_mpart(esp_ctx *c) {
   int rc = dalloc(c, c->d_mpart, 3 * n);
   if (rc) return rc;
   if ((rc = dalloc(c, c->d_w, n))) return rc;
+  dfree(c->d_mpart_l);
   HIPCHK(c, hipMemsetAsync(c->d_mpart, 0, 3 * n * sizeof(double), c->stream));
   HIPCHK(c, hipMemsetAsync(c->d_w, 0, n * sizeof(double), c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -173,7 +184,12 @@ int ensure_mpart(esp_ctx *c) {
   c->mpart_geo = geo;
   c->mpart_tps = c->tps;
   c->mpart_valid = false;
-  return ESP_OK;
+  return ensure_mpart(c);        // (the learned phases' sums)
+}
+
+// The valid per-wave spin sums, or null.
+const double *wave_spin_sums(const esp_ctx *c) {
+  return !c->mpart_valid ? nullptr : c->mpart_learned ? c->d_mpart_l : c->d_mpart;
 }
 
 // Kernel arguments of the colour phases, with the per-wave spin sums attached.
@@ -201,8 +217,10 @@ void set_colour(KArgs &a, const esp::HostModel &m, int col, int lay) {
 int enqueue_phase_sweeps(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsweeps, int off0) {
   c->w_dirty = true;
   if (mode == ESP_MODE_LEARNED) {
-    c->mpart_valid = false;
-    return esp::learn_enqueue_sweeps(c, seed, nsweeps, off0);
+    int rc = esp::learn_enqueue_sweeps(c, seed, nsweeps, off0);
+    c->mpart_valid = rc == ESP_OK && nsweeps > 0 && c->d_mpart_l;
+    c->mpart_learned = true;
+    return rc;
   }
   const esp::HostModel &m = c->hm;
   KArgs a = phase_args(c, tilt, seed);
@@ -217,7 +235,10 @@ int enqueue_phase_sweeps(esp_ctx *c, int mode, double tilt, uint64_t seed, int n
       hipLaunchKernelGGL(fn, dim3(a.nblk * c->R), dim3(kPhaseBlock), shm, c->stream, a);
     }
   HIPCHK(c, hipGetLastError());
-  if (nsweeps > 0) c->mpart_valid = a.mpart != nullptr;
+  if (nsweeps > 0) {
+    c->mpart_valid = a.mpart != nullptr;
+    c->mpart_learned = false;
+  }
   return ESP_OK;
 }
 
@@ -238,10 +259,10 @@ int enqueue_lds_sweeps(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsw
 // Running-energy and magnetisation sums: the spins' sums come from the colour phases'
 // per-wave sums when the last sweep left them, else from the spins.
 int enqueue_reduce(esp_ctx *c) {
-  const bool mp = c->mpart_valid;
+  const double *mp = wave_spin_sums(c);
   hipLaunchKernelGGL(k_reduce, dim3(c->red_blocks, c->R), dim3(kBlock), 0, c->stream,
                      (const double *)c->d_sp, (const double *)c->d_w, c->hm.N, c->Ns,
-                     c->red_blocks, c->d_partial, mp ? (const double *)c->d_mpart : nullptr,
+                     c->red_blocks, c->d_partial, mp,
                      c->hm.ncol * c->mpart_nw);   // ncol * mpart_nw entries of both
   HIPCHK(c, hipGetLastError());
   return ESP_OK;
@@ -267,7 +288,7 @@ int enqueue_finalize(esp_ctx *c, bool use_partials, bool measure, bool exchange,
 // enqueue_reduce + enqueue_finalize(use_partials = true) in one launch (k_reduce_fin): with the
 // colour phases' per-wave sums, one block per 4096 entries of a replica, else the spin-sum blocks.
 int enqueue_reduce_finalize(esp_ctx *c, bool measure, bool exchange, int advance, uint64_t seed) {
-  const bool mp = c->mpart_valid;
+  const double *mp = wave_spin_sums(c);
   const int ne = c->hm.ncol * c->mpart_nw;
   const int nblk = mp ? std::max(1, std::min(c->red_blocks, (ne + 4095) / 4096)) : c->red_blocks;
   FinArgs f{};
@@ -280,7 +301,7 @@ int enqueue_reduce_finalize(esp_ctx *c, bool measure, bool exchange, int advance
   f.key0 = (uint32_t)seed; f.key1 = (uint32_t)(seed >> 32); f.stream_base = c->stream_base;
   f.trace = c->d_trace; f.trace_cap = c->trace_cap;
   hipLaunchKernelGGL(k_reduce_fin, dim3(nblk, c->R), dim3(kBlock), 0, c->stream, (const double *)c->d_sp,
-                     (const double *)c->d_w, c->hm.N, c->Ns, mp ? (const double *)c->d_mpart : nullptr, ne,
+                     (const double *)c->d_w, c->hm.N, c->Ns, mp, ne,
                      c->d_partial, f, c->d_done);
   HIPCHK(c, hipGetLastError());
   return ESP_OK;
@@ -919,6 +940,7 @@ int esp_time_sweeps(esp_ctx *c, int nsweeps, int mode, double tilt, uint64_t see
     HIPCHK(c, hipGetLastError());
   }
   c->mpart_valid = !lds && mode != ESP_MODE_LEARNED;
+  c->mpart_learned = false;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   double sum = 0.0;
   for (int q = 0; q < k; ++q) {

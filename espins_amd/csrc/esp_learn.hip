@@ -946,7 +946,7 @@ int learn_enqueue_sweeps(esp_ctx *c, uint64_t seed, int nsweeps, int off0, hipEv
   const esp::HostModel &m = c->hm;
   KArgs a = base_args(c);
   a.tps = 1;
-  a.mpart = nullptr;                  // the learned phases keep no spin sums
+  a.mpart = c->d_mpart_l;             // (null before the first call after the weights were set)
   a.key0 = (uint32_t)seed; a.key1 = (uint32_t)(seed >> 32);
   LearnFn fn = learn_fn(m);
   const size_t shm = (m.compressed ? c->ctab_bytes : 0) + kNP * sizeof(float);
