@@ -349,20 +349,43 @@ bool lds_sweeps(const esp_ctx *c, int mode) {
   return c->use_lds && mode != ESP_MODE_LEARNED && !c->d_trace && !c->obs.flags;
 }
 
-// Clusters of blocks serve the plain proposals of the automatic path.  Replicas that one block
-// holds (k_lds) go to a cluster from kClusterMinSites sites per colour: below, a block's threads
-// all have one site anyway and the flags between blocks only add.
+// Clusters of blocks may serve the plain proposals of the automatic path.
+bool cluster_possible(const esp_ctx *c, int mode) {
+  return c->path == 0 && !c->tps_user && (mode == ESP_MODE_RANDOM || mode == ESP_MODE_CONST) && !c->obs.flags;
+}
+
+// Their tables are laid out with the replicas from this many sites per colour; smaller replicas
+// that one block holds (k_lds) get them in a run that is long enough to pay for it (0.6 ms).
 constexpr int kClusterMinSites = 384;
-bool cluster_sweeps(const esp_ctx *c, int mode) {
-  if (c->path != 0 || c->tps_user || (mode != ESP_MODE_RANDOM && mode != ESP_MODE_CONST) || c->obs.flags) return false;
-  return !lds_sweeps(c, mode) || c->hm.N / std::max(1, c->hm.ncol) >= kClusterMinSites;
+constexpr int kClusterLateSteps = 256;
+bool cluster_early(const esp_ctx *c, int mode) {
+  return cluster_possible(c, mode) && (!lds_sweeps(c, mode) || c->hm.N / std::max(1, c->hm.ncol) >= kClusterMinSites);
+}
+
+// Where one block holds a replica, both serve.  k_lds pays a launch and an exchange kernel per
+// exchange (14 us), a cluster the flags between its blocks in every phase and step.  us per step,
+// cluster / k_lds, with an exchange every step: sc 8^3 10.8 / 16.9, sc 12^3 12.5 / 21.0, fcc 8^3
+// 22.0 / 28.6; every 10 steps: 8.3 / 4.5, sc 14^3 12.7 / 11.8 -- the lines cross at 2 to 6 steps.
+// Without exchanges k_lds takes about 2 us per phase and pass of its threads over the colour, a
+// cluster 8 + 2.7 per phase: 11.2 / 7.4 (sc 12^3, 2 colours, 2 passes), 14.0 / 13.6 (sc 16^3, 4),
+// 18.4 / 16.4 (with second neighbours, 4 colours, 2 passes), 18.8 / 23.5 (sc 14^3, 4 and 3),
+// 28.3 / 32.6 (fcc 10^3, 8 and 2).
+bool cluster_sweeps(const esp_ctx *c, int mode, bool exchange, int round, int nsteps) {
+  if (!cluster_possible(c, mode)) return false;
+  if (!lds_sweeps(c, mode)) return true;
+  const bool early = cluster_early(c, mode);
+  if (exchange && round <= 3)
+    return early || (c->cluster && c->cluster_R == c->R) || nsteps >= kClusterLateSteps;
+  const int ncol = std::max(1, c->hm.ncol);
+  const int passes = (c->hm.N * c->tps / ncol + kLdsBlock - 1) / kLdsBlock;
+  return early && ncol * (passes - 1) > 4;
 }
 
 // The steps of a run on clusters, as far as they serve it: *ran of nsteps (from the device clock).
 int run_clusters(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, int M, bool measure, bool exchange,
                  int round, int *ran) {
   *ran = 0;
-  if (!cluster_sweeps(c, mode)) return ESP_OK;
+  if (!cluster_sweeps(c, mode, exchange, round, nsteps)) return ESP_OK;
   int rc = esp::cluster_prepare(c);
   if (rc || !c->cluster) return rc;
   if (c->w_dirty) {          // the clusters count their accepted dE on top of e_base
@@ -694,7 +717,7 @@ int esp_set_replicas(esp_ctx *c, int R, const double *tems, const double *spins)
   HIPCHK(c, hipMemsetAsync(c->d_nswap, 0, sizeof(unsigned long long) * 2 * R, c->stream));
   HIPCHK(c, hipMemsetAsync(c->d_nmeas, 0, sizeof(unsigned long long), c->stream));
   if ((rc = esp::obs_resize(c))) return rc;
-  if (cluster_sweeps(c, ESP_MODE_RANDOM) && (rc = esp::cluster_prepare(c))) return rc;
+  if (cluster_early(c, ESP_MODE_RANDOM) && (rc = esp::cluster_prepare(c))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return esp_put_spins(c, spins);
 }

@@ -52,7 +52,7 @@ constexpr int kLdsBlock = 512;   // LDS-resident kernel (8 waves per replica)
 #endif
 constexpr int kChunk = ESP_CHUNK;  // partner gathers issued together per lane
 constexpr int kChunkWide = ESP_CHUNK_WIDE;  // ... for launches too small to fill the GPU with waves
-constexpr int kChunkLds = 8;     // ... in the LDS-resident sweep
+constexpr int kChunkLds = 3;     // ... in the LDS-resident sweep
 #ifndef ESP_CHUNK_LEARN
 #define ESP_CHUNK_LEARN 8
 #endif
@@ -245,6 +245,16 @@ __device__ __forceinline__ void bond_term(const KArgs &a, const double *crow, in
                cz * (ds.x * sj.y - ds.y * sj.x));
 }
 
+// Partner indices of a site's first chunk (bond_sums).
+template <int CH>
+__device__ __forceinline__ void first_bonds(const KArgs &a, int d, int g, unsigned (&jn)[CH]) {
+  const int tps = a.tps, nk = (a.zmax - g + tps - 1) / tps;
+#pragma unroll
+  for (int u = 0; u < CH; ++u) {
+    const int l = u < nk ? g + tps * u : g;
+    jn[u] = nk > 0 ? (unsigned)ld_off(a.nbr, ((unsigned)l * (unsigned)a.N + (unsigned)d) * 4u) : 0u;
+  }
+}
 // Partial bond sums over the slots l = g, g+tps, ... of site st.  Inactive lanes return
 // zeros.  Slots go in chunks of CH: the CH partner indices of the next chunk are loaded
 // while the current chunk's CH partner gathers are in flight, so a
@@ -253,8 +263,8 @@ __device__ __forceinline__ void bond_term(const KArgs &a, const double *crow, in
 // spin (index N), so they need no test; a self bond (SELF) reads the new spin.
 template <int CH, bool CMP, bool HB, bool HD, bool SELF, class SP>
 __device__ __forceinline__ void bond_sums(const KArgs &a, const SP &sp, const double *ctab, const Site &st,
-                                          bool active, int g,
-                                          const Proposal &p, double &eJ, double &eB, double &eD) {
+                                          bool active, int g, const Proposal &p, unsigned (&jn)[CH], double &eJ,
+                                          double &eB, double &eD) {
   constexpr int LAY = CMP ? LAY_CMP : LAY_BOND;
   eJ = 0.0; eB = 0.0; eD = 0.0;
   if (!active) return;
@@ -266,7 +276,7 @@ __device__ __forceinline__ void bond_sums(const KArgs &a, const SP &sp, const do
   const int nfull = nk - nk % CH;
   const double *crow = CMP ? ctab + (size_t)st.a * a.zmax * 5 : nullptr;
   const unsigned ud = (unsigned)d;
-  unsigned jn[CH];   // partner indices of the next chunk
+  // (jn: partner indices of the next chunk; the first was loaded by first_bonds)
   auto load_idx = [&](int k0) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
@@ -274,7 +284,6 @@ __device__ __forceinline__ void bond_sums(const KArgs &a, const SP &sp, const do
       jn[u] = (unsigned)ld_off(a.nbr, ((unsigned)l * (unsigned)a.N + ud) * 4u);
     }
   };
-  if (nk > 0) load_idx(0);
   for (int k0 = 0; k0 < nfull; k0 += CH) {
     V3 sv[CH];
 #pragma unroll
@@ -492,7 +501,9 @@ __device__ __forceinline__ void phase_tab(const KArgs &a, int r, int b, double *
   Proposal p{};
   if (active) p = propose<MODE>(a, sp, st, r, sweep);
   double eJ, eB, eD;
-  bond_sums<CH, CMP, HB, HD, SELF>(a, sp, s_ctab, st, active, g, p, eJ, eB, eD);
+  unsigned jn[CH];
+  if (active) first_bonds(a, st.d, g, jn);
+  bond_sums<CH, CMP, HB, HD, SELF>(a, sp, s_ctab, st, active, g, p, jn, eJ, eB, eD);
   eJ = group_sum(eJ, tps);
   if (HB) eB = group_sum(eB, tps);
   if (HD) eD = group_sum(eD, tps);
@@ -580,6 +591,22 @@ struct LdsMeas {
   int measure_every;             // 0 = never
 };
 
+// Sums of v over the kLdsBlock threads, valid in wave 0; red: 4 values a wave.
+__device__ __forceinline__ void block_total4(double (&v)[4], double *red) {
+  constexpr int kW = kLdsBlock / 64;
+  const int lane = threadIdx.x & 63;
+  const double t = wave_total4(v[0], v[1], v[2], v[3]);
+  if (lane < 4) red[4 * (threadIdx.x >> 6) + lane] = t;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    double s = lane < 4 * kW ? red[lane] : 0.0;
+#pragma unroll
+    for (int off = 4; off < 4 * kW; off <<= 1) s += __shfl_xor(s, off);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = __shfl(s, k);
+  }
+}
+
 // All colours of nsweeps sweeps of one replica per block, spins resident in LDS,
 // measurement (mcarlo.F90:536-543) fused every measure_every sweeps.
 template <int MODE, bool CMP, bool HB, bool HD, bool SELF>
@@ -609,6 +636,33 @@ __device__ __forceinline__ void lds_body(const KArgs &a, int r, int nsweeps, con
   const int tps = a.tps;
   const int g = threadIdx.x & (tps - 1);
   const int per = kLdsBlock / tps;
+  // Colours of at most half a block: the two halves of the block (on the same SIMDs) take turns.
+  // While one finishes a phase, the other draws its proposals of the next and loads its first
+  // partner indices; a site's own spin changes only in its own phase.
+  // (16 replicas of sc 8^3, 2 colours: 5.7 us a sweep without turns, 3.2 with; bcc 6^3, z = 14,
+  // 12.2 and 7.4.  Three partner indices at a time: 6 gain 5 % for z = 6 and lose it for z = 14, 18.)
+  constexpr int kHalf = kLdsBlock / 2;
+  bool halves = a.ncol > 1;
+  for (int c = 0; c < a.ncol; ++c) {
+    const int n = gldi(a.col_off, c + 1) - gldi(a.col_off, c);
+    halves &= n > 0 && n * tps <= kHalf;
+  }
+  const int half = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kHalf);
+  struct Turn {
+    Site st;
+    Proposal p;
+    unsigned jn[kChunkLds];
+    bool active;
+  };
+  auto begin = [&](int d0, int beg, int end, unsigned long long sweep) {
+    Turn t;
+    t.active = d0 < end;
+    t.st = site_info(a, t.active ? d0 : beg);
+    first_bonds(a, t.st.d, g, t.jn);
+    t.p = Proposal{};
+    if (t.active) t.p = propose<MODE>(a, sp, t.st, r, sweep);
+    return t;
+  };
   unsigned long long nrej = 0;   // 64-bit: one launch may run many sweeps at high rejection
   // The estimator sums of this replica's slot live in thread 0's registers during the
   // launch (same additions, same order as adding to memory each time) and are stored once
@@ -620,34 +674,37 @@ __device__ __forceinline__ void lds_body(const KArgs &a, int r, int nsweeps, con
     for (int k = 0; k < 6; ++k) A[k] = gldi(m.acc, 6 * slot + k);
   const double e_base = gldi(m.e_base, r);
   double w_launch = 0.0;      // thread 0: the launch's accepted dE at the last block sum
+  auto finish = [&](Turn &t) {
+    double eJ, eB, eD;
+    bond_sums<kChunkLds, CMP, HB, HD, SELF>(a, sp, ctab, t.st, t.active, g, t.p, t.jn, eJ, eB, eD);
+    eJ = group_sum(eJ, tps);
+    if (HB) eB = group_sum(eB, tps);
+    if (HD) eD = group_sum(eD, tps);
+    if (!t.active) return;
+    double de;
+    const bool rej = decide(a, t.st.a, t.p, eJ, eB, eD, beta, &de);
+    if (g != 0) return;
+    if (rej) ++nrej;
+    else {
+      const double4 old = s_sp[t.st.d];
+      s_sp[t.st.d] = make_double4(t.p.sn.x, t.p.sn.y, t.p.sn.z, old.w + de);
+    }
+  };
+  Turn turn{};                 // (nobody's yet: inactive)
+  int whose = 1;               // the half that finishes the phase (halves)
   for (int sw = 0; sw < nsweeps; ++sw) {
-    const unsigned long long sweep = sweep0 + (unsigned long long)sw;
-    for (int c = 0; c < a.ncol; ++c) {
-      const int beg = gldi(a.col_off, c), end = gldi(a.col_off, c + 1);
-      for (int base = beg; base < end; base += per) {  // uniform trip count in the block
-        const int d0 = base + threadIdx.x / tps;
-        const bool active = d0 < end;
-        const int d = active ? d0 : beg;
-        const Site st = site_info(a, d);
-        Proposal p{};
-        if (active) p = propose<MODE>(a, sp, st, r, sweep);
-        double eJ, eB, eD;
-        bond_sums<kChunkLds, CMP, HB, HD, SELF>(a, sp, ctab, st, active, g, p, eJ, eB, eD);
-        eJ = group_sum(eJ, tps);
-        if (HB) eB = group_sum(eB, tps);
-        if (HD) eD = group_sum(eD, tps);
-        if (active) {
-          double de;
-          const bool rej = decide(a, st.a, p, eJ, eB, eD, beta, &de);
-          if (g == 0) {
-            if (rej) ++nrej;
-            else {
-              const double4 old = s_sp[d];
-              s_sp[d] = make_double4(p.sn.x, p.sn.y, p.sn.z, old.w + de);
-            }
-          }
-        }
+    // with halves, a phase -1 goes first, in which half 0 draws its proposals of phase 0
+    for (int c = halves && sw == 0 ? -1 : 0; c < a.ncol; ++c) {
+      const bool wrap = halves && c + 1 == a.ncol;
+      const int cb = wrap ? 0 : halves ? c + 1 : c;            // the colour to begin
+      const unsigned long long sweep = sweep0 + (unsigned long long)(sw + wrap);
+      const int beg = gldi(a.col_off, cb), end = gldi(a.col_off, cb + 1);
+      const int lane = halves ? (int)threadIdx.x & (kHalf - 1) : (int)threadIdx.x;
+      for (int base = beg; base < end; base += per) {          // uniform trip count in the block
+        if (!halves || half != whose) turn = begin(base + lane / tps, beg, end, sweep);
+        if (!halves || half == whose) finish(turn);
       }
+      whose ^= 1;
       __syncthreads();
     }
     const bool last = sw + 1 == nsweeps;
@@ -658,7 +715,7 @@ __device__ __forceinline__ void lds_body(const KArgs &a, int r, int nsweeps, con
         const double4 s = s_sp[d];
         v[0] += s.w; v[1] += s.x; v[2] += s.y; v[3] += s.z;
       }
-      block_sum<4>(v, red);
+      block_total4(v, red);
       if (threadIdx.x == 0) {
         const double e = e_base + wg[0] + v[0];
         w_launch = v[0];
@@ -843,7 +900,7 @@ __global__ __launch_bounds__(1024) void k_finalize(FinArgs f) {
 // -- then runs finalize_body and advances the clock.  The partial sums move past the caches (ast,
 // ald) and a block counts itself when its own are in place: with device fences, which write back
 // the XCD's whole L2 with the spins that the sweep has just changed, it took 12.0 us for 64
-// replicas of fcc 32^3 and 8.0 for 16 of fcc 16^3, without 10.8 and 6.9.
+// replicas of fcc 32^3 and 8.0 for 32 of fcc 16^3, without 10.8 and 6.9.
 __global__ __launch_bounds__(kBlock) void k_reduce_fin(const double *sp, const double *wpart, int N, int Ns,
                                                        const double *mpart, int ne, double *partial, FinArgs f,
                                                        unsigned *done) {
