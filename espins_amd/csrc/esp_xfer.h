@@ -8,9 +8,11 @@
 //    chunk is turned into reference order and copied by the GPU, the others move theirs into the
 //    destination (and take its page faults);
 //  * small results of one call are copied into one pinned page and waited for once.
-// A context or batch takes its buffers at the first read-out and gives them back when it is
-// destroyed; up to kXKeep sets wait for the next one (allocating pinned memory takes longer than
-// a small run), and the last context or batch to go frees them all.  Workers live for one call.
+// Pinned memory takes milliseconds to allocate and to free, longer than a small run, so a context
+// or batch that finds no buffers waiting allocates them only after kXFirst bytes of spins or
+// kXAsks small reads; until then it copies as it comes.  It gives its buffers back when it is
+// destroyed; up to kXKeep sets wait for the next one, and the last context or batch to go frees
+// them all.  Workers live for one call.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -26,12 +28,16 @@ namespace espx {
 constexpr size_t kXChunk = size_t(3) << 20;      // bytes per slot (a multiple of 24)
 constexpr int kXSlots = 8;
 constexpr size_t kXSmall = size_t(1) << 18;
+constexpr size_t kXFirst = size_t(64) << 20;
+constexpr int kXAsks = 32;
 
 struct Xfer {
   int device = -1;
   char *pin = nullptr, *dev = nullptr, *small = nullptr;
   hipEvent_t ev[kXSlots] = {};
   int slots = 0;                                 // slots allocated
+  size_t seen = 0;                               // bytes of spins read so far
+  int asks = 0;                                  // small reads so far
 
   void release() {
     for (auto &e : ev)
@@ -89,7 +95,7 @@ inline void xfer_take(Xfer &x) {           // buffers of an earlier owner, if an
   std::lock_guard<std::mutex> lk(p.mu);
   for (size_t i = 0; i < p.idle.size(); ++i)
     if (p.idle[i].device == x.device) {
-      x = p.idle[i];
+      x = p.idle[i];       // (its counts, too: they only grow)
       p.idle.erase(p.idle.begin() + i);
       return;
     }
@@ -118,7 +124,20 @@ hipError_t xfer_spins(K kernel, Xfer &x, int device, hipStream_t stream, const d
   const size_t chunks = (total + per - 1) / per;
   const int nt = (int)std::min<size_t>(chunks, kXSlots);
   xfer_take(x);
-  hipError_t e = x.reserve(nt);
+  x.seen += 24 * total;
+  hipError_t e;
+  if (!x.dev && x.seen < kXFirst) {
+    double *d = nullptr;
+    if ((e = hipMalloc((void **)&d, 24 * total)) != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, sp, ref2dev, src_rep, N,
+                       Ns, (size_t)0, total, d);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(out, d, 24 * total, hipMemcpyDeviceToHost, stream);
+    const hipError_t q = hipStreamSynchronize(stream);
+    (void)hipFree(d);
+    return e == hipSuccess ? q : e;
+  }
+  e = x.reserve(nt);
   if (e != hipSuccess) return e;
   std::atomic<int> err{hipSuccess};
   auto work = [&](int t) {
@@ -155,7 +174,7 @@ class SmallRead {
  public:
   SmallRead(Xfer &x, hipStream_t s) : x_(x), s_(s) {
     xfer_take(x_);
-    if (!x_.small && hipHostMalloc((void **)&x_.small, kXSmall, hipHostMallocDefault) != hipSuccess) {
+    if (!x_.small && ++x_.asks > kXAsks && hipHostMalloc((void **)&x_.small, kXSmall, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
       x_.small = nullptr;
     }
