@@ -101,6 +101,7 @@ using BLdsFn = void (*)(const KArgs *, const LdsMeas *, const int2 *, int, int);
 // variants add bit 5: the wide setting of the partner gathers in flight per lane (global path)
 constexpr int kVarChunk4 = 32;
 constexpr size_t kGroupBytes = size_t(192) << 20;   // spins of a replica group
+constexpr size_t kGroupMax = 3 * kGroupBytes;        // spins of a batch that is split
 constexpr int kNarrow = 2;   // the narrow setting, as set_chain_chunk and info name it
 template <int MODE, int LAY, bool HB, bool HD, int CH>
 BPhaseFn bp4(bool self) { return self ? k_bphase<MODE, LAY, HB, HD, true, CH> : k_bphase<MODE, LAY, HB, HD, false, CH>; }
@@ -387,7 +388,9 @@ int build_plan(esp_batch *b, double tilt, uint64_t seed) {
   // Replica groups: a sweep runs all colours of one group, then of the next.  A colour phase reads
   // most of its replicas' spins, so the phases of more state than the memory-side cache (256 MB)
   // come from HBM each time; a launch more costs about 4 us.  24 chains of 369 MB, 60 rounds, in
-  // groups of 32 / 64 / 96 / 128 / 192 MB and in one: 65 / 52 / 46 / 43 / 41 / 43 ms.
+  // groups of 32 / 64 / 96 / 128 / 192 MB and in one: 65 / 52 / 46 / 43 / 41 / 43 ms.  Much larger
+  // batches stay in one: a launch is long there, and with few large replicas to a group the XCDs
+  // end unevenly (256 chains, 11.3 GB: 24.3 G updates/s in one, 24.0 in 59 groups).
   // Chains with as many colours stand together (a group's last colours would run a few chains).
   std::vector<std::vector<int4>> groups;              // (chain, first replica, end)
   {
@@ -397,7 +400,7 @@ int build_plan(esp_batch *b, double tilt, uint64_t seed) {
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b->chains[x].hm.ncol > b->chains[y].hm.ncol; });
     size_t total = 0, left = 0;
     for (int k : order) total += sizeof(double) * 3 * b->chains[k].Ns * b->chains[k].R;
-    const size_t ng = std::max<size_t>(1, (total + kGroupBytes / 2) / kGroupBytes);
+    const size_t ng = total > kGroupMax ? 1 : std::max<size_t>(1, (total + kGroupBytes / 2) / kGroupBytes);
     for (int k : order) {
       const size_t rep = sizeof(double) * 3 * b->chains[k].Ns;
       for (int r = 0; r < b->chains[k].R; ++r) {
