@@ -11,8 +11,8 @@
 // k_obs_cells (one thread per cell: the cell sums, block partials of OP and SM, the P(m)
 // counts through a histogram in LDS), k_obs_spincorr (one thread per site and several
 // replicas, device order), k_sf_pack / k_sf_main / k_sf_fin (S(q) as a phase-matrix times
-// spin-matrix product: one phase per q-point, site and 8 replicas; k_sf_lat for lattice
-// positions: phases from per-q tables) and k_obs_final (per replica: fixed-order sums of the
+// spin-matrix product: one phase per q-point, site and 8 replicas; k_sf_plane / k_sf_q for lattice
+// positions: summed axis by axis) and k_obs_final (per replica: fixed-order sums of the
 // block partials, accumulation into the replica's slot).
 // Histogram counts are integers, so they do not depend on the order of the atomic additions;
 // every floating-point sum has a fixed order.

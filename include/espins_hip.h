@@ -100,8 +100,9 @@ int esp_plan_model(int N, int nb, const double *mag,
                    int zB, const int *b_cnt, const int *b_nbr, const double *b_val,
                    int zD, const int *d_cnt, const int *d_nbr, const double *d_vec,
                    const int *L3, int *ncol, int *colour, int *info);
-/* Sweep kernel choice: 0 = automatic (LDS-resident when a replica fits in LDS), 1 = global-
- * memory colour phases, 2 = LDS-resident (EINVAL if the replica does not fit). */
+/* Sweep kernel choice: 0 = automatic (LDS-resident when a replica fits in LDS; middle-sized
+ * replicas, and small ones with frequent exchanges, on clusters of blocks), 1 = global-memory
+ * colour phases, 2 = LDS-resident (EINVAL if the replica does not fit). */
 int esp_set_path(esp_ctx *ctx, int path);
 /* Philox stream of replica r is base + r (default 0); the exchange stream is
  * 0xFFFFFFFF - base.  A batch gives chain k the base k << 16. */
