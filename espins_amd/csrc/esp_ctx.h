@@ -133,6 +133,7 @@ struct esp_ctx {
   // graph cache
   hipGraphExec_t gexec = nullptr;
   std::string gkey;
+  bool g_mpart_valid = false, g_mpart_learned = false;   // what a replay leaves in mpart_valid, _learned
 };
 
 namespace esp {

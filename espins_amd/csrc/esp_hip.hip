@@ -898,6 +898,9 @@ int esp_run(esp_ctx *c, int n_rounds, int steps_per_round, int steps_measure, in
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     rc = enqueue_round(c, steps_per_round, steps_measure, do_measure, do_exchange, mode, tilt, seed);
     hipError_t ce = hipStreamEndCapture(c->stream, &g);
+    c->g_mpart_valid = c->mpart_valid;
+    c->g_mpart_learned = c->mpart_learned;
+    c->mpart_valid = false;          // (captured, not run)
     if (rc) return rc;
     if (ce != hipSuccess) return fail(c, ESP_EHIP, std::string("capture: ") + hipGetErrorString(ce));
     hipError_t ie = hipGraphInstantiate(&c->gexec, g, nullptr, nullptr, 0);
@@ -909,8 +912,11 @@ int esp_run(esp_ctx *c, int n_rounds, int steps_per_round, int steps_measure, in
     c->gkey = key;
   }
   c->w_dirty = true;
+  c->mpart_valid = false;
   for (int k = 0; k < n_rounds; ++k) HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->mpart_valid = c->g_mpart_valid;
+  c->mpart_learned = c->g_mpart_learned;
   return ESP_OK;
 }
 
