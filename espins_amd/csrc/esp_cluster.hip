@@ -440,6 +440,19 @@ size_t cluster_lds(const esp::HostModel &m, int nl_max, int R) {
          (m.compressed ? (size_t)m.nb * groups_compiled(m) * kGroup * nc * sizeof(double) : 0) + fin_lds_bytes(R);
 }
 
+// A block's LDS beside the kernel's static share.
+bool cluster_fits(const esp::HostModel &m, int nl_max, int R, size_t lds_max) {
+  return nl_max < 65535 && cluster_lds(m, nl_max, R) + 1024 <= lds_max;
+}
+
+// Parts to cut a replica into; 0 where clusters do not serve the model.
+int cluster_parts(const esp::HostModel &m, int R, int num_cu) {
+  if (m.ncol < 2 || m.ncol > kCMaxCol || m.zmax > kCMaxGroups * kGroup ||
+      (!m.compressed && (m.zmax > kGroup || m.has_B || m.has_D)))
+    return 0;
+  return std::min(num_cu / R, m.N / m.ncol / 64);
+}
+
 struct Plan {
   std::vector<Part> part;
   std::vector<int> own_dev, own_ref, hal_dev, col_off, hal_off, nbs;
@@ -475,7 +488,7 @@ bool make_plan(const esp::HostModel &m, int k, int R, size_t lds_max, Plan &p) {
       if (mark[j][d]) hal[j].push_back(d);                    // device order: by colour
     p.nl_max = std::max(p.nl_max, (int)(own[j].size() + hal[j].size()));
   }
-  if (p.nl_max >= 65535 || cluster_lds(m, p.nl_max, R) + 1024 > lds_max) return false;
+  if (!cluster_fits(m, p.nl_max, R, lds_max)) return false;
   for (int j = 0; j < k; ++j) {
     Part t{};
     t.nown = (int)own[j].size();
@@ -550,15 +563,13 @@ void cluster_free(esp_ctx *c) {
 }
 
 // Decides whether clusters serve this context and builds their tables, once per (model, replica
-// count): they depend on the model and k only.  c->cluster stays null if not.
+// count).  c->cluster stays null if not.
 int cluster_prepare(esp_ctx *c) {
   if (c->cluster_R == c->R) return ESP_OK;
   const HostModel &m = c->hm;
-  int k = std::min(c->num_cu / c->R, m.N / std::max(1, m.ncol) / 64);
-  if (m.ncol < 2 || m.ncol > kCMaxCol || m.zmax > kCMaxGroups * kGroup ||
-      (!m.compressed && (m.zmax > kGroup || m.has_B || m.has_D)))
-    k = 0;
-  if (c->cluster && c->cluster->k == k) {
+  int k = cluster_parts(m, c->R, c->num_cu);
+  // (the tables depend on the model and k, the LDS of a block also on the replica count)
+  if (c->cluster && c->cluster->k == k && cluster_fits(m, c->cluster->nl_max, c->R, c->lds_max)) {
     c->cluster_R = c->R;
     return ESP_OK;
   }
@@ -650,3 +661,33 @@ int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, in
 }
 
 }  // namespace esp
+
+extern "C" {
+
+int esp_plan_clusters(int N, int nb, const double *mag, int zJ, const int *j_cnt, const int *j_nbr,
+                      const double *j_val, int zB, const int *b_cnt, const int *b_nbr, const double *b_val, int zD,
+                      const int *d_cnt, const int *d_nbr, const double *d_vec, const int *L, int R, int num_cu,
+                      int64_t lds_bytes, int64_t *out) {
+  if (R < 1 || num_cu < 1 || lds_bytes < 1 || !out) return ESP_EINVAL;
+  esp::HostModel hm;
+  if (!esp::prepare_model(hm, N, nb, mag, zJ, j_cnt, j_nbr, j_val, zB, b_cnt, b_nbr, b_val, zD, d_cnt, d_nbr, d_vec, 0,
+                          nullptr, nullptr, 0, nullptr, nullptr, L).empty())
+    return ESP_EINVAL;
+  int k = cluster_parts(hm, R, num_cu);
+  Plan p;
+  while (k >= 2 && !make_plan(hm, k, R, (size_t)lds_bytes, p)) --k;
+  const bool on = k >= 2;
+  out[0] = on ? k : 0;
+  out[1] = on ? p.nl_max : 0;
+  out[2] = on ? (int64_t)cluster_lds(hm, p.nl_max, R) : 0;
+  return ESP_OK;
+}
+
+int esp_get_cluster_info(esp_ctx *c, int64_t *out) {
+  if (!c || !out) return ESP_EINVAL;
+  out[0] = c->cluster && c->cluster_R == c->R ? c->cluster->k : 0;
+  out[1] = c->cluster_sweeps;
+  return ESP_OK;
+}
+
+}  // extern "C"

@@ -385,6 +385,7 @@ bool cluster_sweeps(const esp_ctx *c, int mode, bool exchange, int round, int ns
 int run_clusters(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, int M, bool measure, bool exchange,
                  int round, int *ran) {
   *ran = 0;
+  c->cluster_sweeps = 0;
   if (!cluster_sweeps(c, mode, exchange, round, nsteps)) return ESP_OK;
   int rc = esp::cluster_prepare(c);
   if (rc || !c->cluster) return rc;
@@ -394,7 +395,9 @@ int run_clusters(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, i
     HIPCHK(c, hipGetLastError());
     c->w_dirty = false;
   }
-  return esp::cluster_run(c, mode, tilt, seed, nsteps, M, measure, exchange, round, ran);
+  rc = esp::cluster_run(c, mode, tilt, seed, nsteps, M, measure, exchange, round, ran);
+  c->cluster_sweeps = (int64_t)*ran * M;
+  return rc;
 }
 
 // One MC "round": steps x (M sweeps [+ measure]) [+ exchange]; advances the clock.

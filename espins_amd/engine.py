@@ -129,6 +129,13 @@ class Engine:
                     layout=("bond", "basis", "implicit")[int(out[3])], lds=bool(out[4]),
                     tps=int(out[5]))
 
+    def cluster_info(self):
+        """Clusters of blocks (the automatic path of middle-sized replicas): parts per replica (0: none)
+        and the sweeps of the last sweep() or run() that they ran."""
+        out = np.zeros(2, np.int64)
+        self._chk(E.lib.esp_get_cluster_info(self._h, E.ptr(out, C.c_int64)))
+        return dict(parts=int(out[0]), sweeps=int(out[1]))
+
     # ---- replicas --------------------------------------------------------------------
     def set_replicas(self, tems, spins):
         tems = E.f64(tems)
@@ -425,8 +432,8 @@ def mcarlo(eng: Engine, steps_warmup, steps_mc, steps_measure=1, mode="random", 
     return obs, st0, st
 
 
-def plan_model(m: Model):
-    """Host-only: (ncol, colour[N], info) that esp_set_model would use for model m."""
+def _with_tables(m: Model, f):
+    """f(*arguments of the model's tables), as esp_plan_model takes them first."""
     d, i = C.c_double, C.c_int
 
     def tab(t):
@@ -439,13 +446,24 @@ def plan_model(m: Model):
     zB, bc, bn, bv = tab(m.B)
     zD, dc, dn, dv = tab(m.D)
     Ls = np.array(m.L, np.int32) if getattr(m, "L", None) is not None else None
+    E.check(f(m.N, m.nb, E.ptr(mag, d), zJ, E.ptr(jc, i), E.ptr(jn, i), E.ptr(jv, d), zB, E.ptr(bc, i),
+              E.ptr(bn, i), E.ptr(bv, d), zD, E.ptr(dc, i), E.ptr(dn, i), E.ptr(dv, d), E.ptr(Ls, i)))
+
+
+def plan_clusters(m: Model, R, num_cu=256, lds_bytes=160 * 1024):
+    """Host-only: the clusters of blocks that R replicas of model m would run on (esp_plan_clusters)."""
+    out = np.zeros(3, np.int64)
+    _with_tables(m, lambda *t: E.lib.esp_plan_clusters(*t, int(R), int(num_cu), int(lds_bytes), E.ptr(out, C.c_int64)))
+    return dict(parts=int(out[0]), sites=int(out[1]), lds=int(out[2]))
+
+
+def plan_model(m: Model):
+    """Host-only: (ncol, colour[N], info) that esp_set_model would use for model m."""
+    i = C.c_int
     n = C.c_int()
     col = np.zeros(m.N, np.int32)
     info = np.zeros(5, np.int32)
-    E.check(E.lib.esp_plan_model(m.N, m.nb, E.ptr(mag, d), zJ, E.ptr(jc, i), E.ptr(jn, i),
-                                 E.ptr(jv, d), zB, E.ptr(bc, i), E.ptr(bn, i), E.ptr(bv, d),
-                                 zD, E.ptr(dc, i), E.ptr(dn, i), E.ptr(dv, d), E.ptr(Ls, i),
-                                 C.byref(n), E.ptr(col, i), E.ptr(info, i)))
+    _with_tables(m, lambda *t: E.lib.esp_plan_model(*t, C.byref(n), E.ptr(col, i), E.ptr(info, i)))
     return n.value, col, dict(N=int(info[0]), zmax=int(info[1]), ncol=int(info[2]),
                               compressed=bool(info[3]),
                               layout=("bond", "basis", "implicit")[int(info[3])])

@@ -100,6 +100,14 @@ int esp_plan_model(int N, int nb, const double *mag,
                    int zB, const int *b_cnt, const int *b_nbr, const double *b_val,
                    int zD, const int *d_cnt, const int *d_nbr, const double *d_vec,
                    const int *L3, int *ncol, int *colour, int *info);
+/* Host-only planning of the clusters of blocks (see esp_set_path) for R replicas on a GPU of
+ * num_cu compute units with lds_bytes of LDS each: out[0] = parts per replica (0: none),
+ * out[1] = most sites of a part with those its bonds reach, out[2] = LDS bytes of a block. */
+int esp_plan_clusters(int N, int nb, const double *mag,
+                      int zJ, const int *j_cnt, const int *j_nbr, const double *j_val,
+                      int zB, const int *b_cnt, const int *b_nbr, const double *b_val,
+                      int zD, const int *d_cnt, const int *d_nbr, const double *d_vec,
+                      const int *L3, int R, int num_cu, int64_t lds_bytes, int64_t *out3);
 /* Sweep kernel choice: 0 = automatic (LDS-resident when a replica fits in LDS; middle-sized
  * replicas, and small ones with frequent exchanges, on clusters of blocks), 1 = global-memory
  * colour phases, 2 = LDS-resident (EINVAL if the replica does not fit). */
@@ -114,6 +122,9 @@ int esp_get_coloring(esp_ctx *ctx, int *ncol, int *colour);
  * the implicit lattice geometry), out[4]=1 if the LDS-resident sweep is used, out[5]=lanes per
  * site in the sweep kernels. */
 int esp_get_model_info(esp_ctx *ctx, int *out6);
+/* Clusters of blocks: out[0] = parts per replica their tables are laid out for (0: none),
+ * out[1] = sweeps of the last esp_sweep or esp_run that they ran. */
+int esp_get_cluster_info(esp_ctx *ctx, int64_t *out2);
 /* Neighbour indexing of the global-memory colour phases: 0 = compute partner and reference
  * site indices from the device index when the supercell is periodic and translation
  * invariant (the geometry is verified against the tables for every site and slot first),
