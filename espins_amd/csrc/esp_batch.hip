@@ -778,7 +778,10 @@ int esp_batch_run(esp_batch *b, int n_rounds, int steps_per_round, int steps_mea
   }
   hipLaunchKernelGGL(k_set_clock, dim3(1), dim3(1), 0, b->stream, b->d_clock, Clock{sweep0, step0, start_parity, 0});
   BCHK(b, hipGetLastError());
-  if (!use_graph) {
+  int64_t per_sweep = 0;             // launches of a sweep
+  for (const auto &v : b->vars)
+    for (int n : v.ntiles) per_sweep += n > 0;
+  if (!use_graph || steps_per_round * (steps_measure * per_sweep + 2) > kCaptureMax) {
     for (int k = 0; k < n_rounds; ++k)
       if ((rc = enqueue_round(b, steps_per_round, steps_measure, do_measure, do_exchange, mode))) return rc;
     b->gkey = key;

@@ -884,7 +884,8 @@ int esp_run(esp_ctx *c, int n_rounds, int steps_per_round, int steps_measure, in
     }
     n_rounds -= ran / steps_per_round;
   }
-  if (!use_graph) {
+  const int64_t launches = lds_sweeps(c, mode) ? 2 : (int64_t)steps_per_round * ((int64_t)steps_measure * c->hm.ncol + 1);
+  if (!use_graph || launches > kCaptureMax) {
     for (int k = 0; k < n_rounds; ++k) {
       rc = enqueue_round(c, steps_per_round, steps_measure, do_measure, do_exchange, mode, tilt, seed);
       if (rc) return rc;
