@@ -41,6 +41,7 @@ constexpr int kCBlock = 512;
 constexpr int kGroup = 6;                         // bonds whose partners are read together
 constexpr int kCMaxGroups = 8;                    // bond groups of a site at most
 constexpr int kCMaxCol = 64;
+constexpr int kPhases = 1 << 18;                  // colour phases of one launch at most: a second or less
 template <bool HB, bool HD>
 constexpr int kTabCoef = 1 + (HB ? 1 : 0) + (HD ? 3 : 0);
 
@@ -70,7 +71,8 @@ struct CArgs {
   double *partial;                                // [2][R][k][4]
   int *slots;                                     // [R] slots after an exchange
   int k, nl_max, ngroup, xcd;
-  int nsteps, M, measure, exchange, round;        // exchange after every `round` steps
+  // steps of M sweeps; an exchange after every `round` steps, the first of them being step0 of a round
+  int nsteps, M, measure, exchange, round, step0;
 };
 
 // What blocks exchange during a launch -- spins, partial sums, slots, flags -- moves by ald and ast
@@ -117,7 +119,7 @@ __global__ __launch_bounds__(kCBlock) void k_cluster(CArgs c) {
   extern __shared__ double s_dyn[];
   __shared__ double s_red[4 * (kCBlock / 64)];
   __shared__ int s_ok, s_col[kCMaxCol + 1], s_hal[kCMaxCol + 1];
-  __shared__ unsigned s_rej;
+  __shared__ unsigned long long s_rej;
   const KArgs &a = c.a;
   int r, j;
   {
@@ -323,7 +325,7 @@ __global__ __launch_bounds__(kCBlock) void k_cluster(CArgs c) {
       }
     }
     const bool last = st + 1 == c.nsteps;
-    const bool xch = c.exchange && (st + 1) % c.round == 0;
+    const bool xch = c.exchange && (c.step0 + st + 1) % c.round == 0;
     if (!c.measure && !xch && !last) continue;
     // Two sets of partial sums take turns, each with its own count: a block may start the next
     // step before a slower one has added to this one, but it reuses a set only when block 0 has
@@ -334,7 +336,7 @@ __global__ __launch_bounds__(kCBlock) void k_cluster(CArgs c) {
     for (int i = tid; i < P.nown; i += kCBlock) { v[0] += lx[i]; v[1] += ly[i]; v[2] += lz[i]; }
     const double t4 = wave_total4(wsum, v[0], v[1], v[2]);
     if ((tid & 63) < 4) s_red[(tid & 63) * (kCBlock / 64) + (tid >> 6)] = t4;
-    unsigned nr = nrej;
+    unsigned long long nr = nrej;     // (a thread's own count fits 32 bits: a launch has kPhases phases at most)
     for (int o = 32; o > 0; o >>= 1) nr += __shfl_down(nr, o, 64);
     nrej = 0;
     if ((tid & 63) == 0 && nr) atomicAdd(&s_rej, nr);
@@ -353,7 +355,7 @@ __global__ __launch_bounds__(kCBlock) void k_cluster(CArgs c) {
       stores_done();
       if (tid == 0) {
         __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (s_rej) gadd(&a.rej[(size_t)(blockIdx.x % kRejSub) * a.R + slot], (unsigned long long)s_rej);
+        if (s_rej) gadd(&a.rej[(size_t)(blockIdx.x % kRejSub) * a.R + slot], s_rej);
         s_rej = 0;
       }
     }
@@ -606,10 +608,11 @@ int cluster_prepare(esp_ctx *c) {
   return ESP_OK;
 }
 
-// nsteps steps of M sweeps [+ measurement], an exchange after every `round` steps, from the
-// device clock.  *ran = 0: the blocks were not all resident and nothing changed.
+// nsteps steps of M sweeps [+ measurement], an exchange after every `round` steps, from the device
+// clock; launches end within steps where those are longer than kPhases.  *ran: sweeps finished; fewer
+// than nsteps M where the blocks of a launch were not all resident (it changed nothing).
 int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, int M, bool measure, bool exchange,
-                int round, int *ran) {
+                int round, int64_t *ran) {
   const HostModel &m = c->hm;
   esp_cluster *q = c->cluster;
   *ran = 0;
@@ -625,7 +628,7 @@ int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, in
   x.partial = q->partial; x.own_mag = q->own_mag; x.own_j = q->own_j; x.slots = q->slots;
   x.k = q->k; x.nl_max = q->nl_max; x.ngroup = q->ngroup;
   x.xcd = c->R % 8 == 0;
-  x.M = M; x.measure = measure; x.exchange = exchange; x.round = round;
+  x.round = round;
   x.f.N = m.N; x.f.R = c->R;
   x.f.e_base = c->d_ebase; x.f.e_run = c->d_erun; x.f.acc = c->d_acc; x.f.nmeas = c->d_nmeas;
   x.f.slot_rep = c->d_slot_rep; x.f.rep_slot = c->d_rep_slot; x.f.beta_slot = c->d_beta; x.f.nswap = c->d_nswap;
@@ -636,11 +639,16 @@ int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, in
   const size_t shm = cluster_lds(m, q->nl_max, c->R);
   if (shm > 65536)
     HIPCHK(c, hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-  // launches of at most about half a second: whole rounds, 2^18 phases
-  const long long per = std::max<long long>(1, (1ll << 18) / ((long long)M * m.ncol * round));
+  const int most = std::max(1, kPhases / m.ncol);           // sweeps of a launch
   const size_t nctl = sizeof(Ctl) + sizeof(unsigned) * (size_t)c->R * q->k;
-  for (int done = 0; done < nsteps;) {
-    x.nsteps = (int)std::min<long long>(nsteps - done, per * round);
+  int done = 0, part = 0;                                   // steps done, sweeps of the next one done
+  while (done < nsteps) {
+    const bool whole = M - part <= most;                    // the launch ends a step
+    x.nsteps = whole && part == 0 ? std::min(nsteps - done, most / M) : 1;
+    x.M = whole ? M - part : most;
+    x.measure = whole && measure;
+    x.exchange = whole && exchange;
+    x.step0 = done % round;
     HIPCHK(c, hipMemsetAsync(q->ctl, 0, nctl, c->stream));
     hipLaunchKernelGGL(fn, dim3(c->R * q->k), dim3(kCBlock), shm, c->stream, x);
     HIPCHK(c, hipGetLastError());
@@ -652,10 +660,12 @@ int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, in
       HIPCHK(c, rd.finish());
     }
     if (h.failed) return fail(c, ESP_EHIP, "cluster sweep: a block stopped making progress");
-    if (h.decided != kGo) return ESP_OK;     // *ran: steps finished so far
+    if (h.decided != kGo) return ESP_OK;
     c->mpart_valid = false;
-    done += x.nsteps;
-    *ran = done;
+    ++c->cluster_launches;
+    *ran += (int64_t)x.nsteps * x.M;
+    done += whole ? x.nsteps : 0;
+    part = whole ? 0 : part + x.M;
   }
   return ESP_OK;
 }
@@ -687,6 +697,7 @@ int esp_get_cluster_info(esp_ctx *c, int64_t *out) {
   if (!c || !out) return ESP_EINVAL;
   out[0] = c->cluster && c->cluster_R == c->R ? c->cluster->k : 0;
   out[1] = c->cluster_sweeps;
+  out[2] = c->cluster_launches;
   return ESP_OK;
 }
 

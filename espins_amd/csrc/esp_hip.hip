@@ -381,11 +381,11 @@ bool cluster_sweeps(const esp_ctx *c, int mode, bool exchange, int round, int ns
   return early && ncol * (passes - 1) > 4;
 }
 
-// The steps of a run on clusters, as far as they serve it: *ran of nsteps (from the device clock).
+// A run on clusters, as far as they serve it: *ran of its nsteps M sweeps (from the device clock).
 int run_clusters(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, int M, bool measure, bool exchange,
-                 int round, int *ran) {
+                 int round, int64_t *ran) {
   *ran = 0;
-  c->cluster_sweeps = 0;
+  c->cluster_sweeps = c->cluster_launches = 0;
   if (!cluster_sweeps(c, mode, exchange, round, nsteps)) return ESP_OK;
   int rc = esp::cluster_prepare(c);
   if (rc || !c->cluster) return rc;
@@ -396,7 +396,7 @@ int run_clusters(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, i
     c->w_dirty = false;
   }
   rc = esp::cluster_run(c, mode, tilt, seed, nsteps, M, measure, exchange, round, ran);
-  c->cluster_sweeps = (int64_t)*ran * M;
+  c->cluster_sweeps = *ran;
   return rc;
 }
 
@@ -798,9 +798,9 @@ int esp_sweep(esp_ctx *c, int nsweeps, int mode, double tilt, uint64_t seed, uin
     return fail(c, ESP_EINVAL, "bad nsweeps / mode");
   if (nsweeps == 0) return ESP_OK;
   if ((rc = set_clock(c, sweep0, 0, 1))) return rc;
-  int ran = 0;
+  int64_t ran = 0;
   if ((rc = run_clusters(c, mode, tilt, seed, nsweeps, 1, false, false, 1, &ran))) return rc;
-  if ((nsweeps -= ran) == 0) return ESP_OK;      // (the device clock has moved on by ran)
+  if ((nsweeps -= (int)ran) == 0) return ESP_OK; // (the device clock has moved on by ran)
   if (lds_sweeps(c, mode)) rc = enqueue_lds_sweeps(c, mode, tilt, seed, nsweeps, 0);
   else rc = enqueue_phase_sweeps(c, mode, tilt, seed, nsweeps, 0);
   if (rc) return rc;
@@ -873,16 +873,31 @@ int esp_run(esp_ctx *c, int n_rounds, int steps_per_round, int steps_measure, in
   if (n_rounds == 0) return ESP_OK;
   if ((rc = set_clock(c, sweep0, step0, start_parity))) return rc;
   if ((int64_t)n_rounds * steps_per_round < (1ll << 30)) {
-    int ran = 0;
+    int64_t ran = 0;
     if ((rc = run_clusters(c, mode, tilt, seed, n_rounds * steps_per_round, steps_measure, do_measure, do_exchange,
                            do_exchange ? steps_per_round : 1, &ran)))
       return rc;
-    if (ran == n_rounds * steps_per_round) return ESP_OK;
-    if (ran % steps_per_round) {     // (no exchanges: finish the round step by step)
-      for (; ran % steps_per_round; ++ran)
-        if ((rc = enqueue_round(c, 1, steps_measure, do_measure, false, mode, tilt, seed))) return rc;
+    if (ran > 0) {                   // the rest of the round that the clusters left, then whole rounds
+      const int64_t steps = ran / steps_measure;
+      const int part = (int)(ran % steps_measure);
+      int at = (int)(steps % steps_per_round);
+      n_rounds -= (int)(steps / steps_per_round);
+      if (part) {
+        const bool last = ++at == steps_per_round;
+        if ((rc = enqueue_round(c, 1, steps_measure - part, do_measure, do_exchange && last, mode, tilt, seed)))
+          return rc;
+        if (last) { at = 0; --n_rounds; }
+      }
+      if (at) {
+        if ((rc = enqueue_round(c, steps_per_round - at, steps_measure, do_measure, do_exchange, mode, tilt, seed)))
+          return rc;
+        --n_rounds;
+      }
+      if (n_rounds == 0) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return ESP_OK;
+      }
     }
-    n_rounds -= ran / steps_per_round;
   }
   const int64_t launches = lds_sweeps(c, mode) ? 2 : (int64_t)steps_per_round * ((int64_t)steps_measure * c->hm.ncol + 1);
   if (!use_graph || launches > kCaptureMax) {

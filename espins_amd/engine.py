@@ -131,10 +131,10 @@ class Engine:
 
     def cluster_info(self):
         """Clusters of blocks (the automatic path of middle-sized replicas): parts per replica (0: none)
-        and the sweeps of the last sweep() or run() that they ran."""
-        out = np.zeros(2, np.int64)
+        and the sweeps of the last sweep() or run() that they ran, in how many launches."""
+        out = np.zeros(3, np.int64)
         self._chk(E.lib.esp_get_cluster_info(self._h, E.ptr(out, C.c_int64)))
-        return dict(parts=int(out[0]), sweeps=int(out[1]))
+        return dict(parts=int(out[0]), sweeps=int(out[1]), launches=int(out[2]))
 
     # ---- replicas --------------------------------------------------------------------
     def set_replicas(self, tems, spins):

@@ -123,8 +123,9 @@ int esp_get_coloring(esp_ctx *ctx, int *ncol, int *colour);
  * site in the sweep kernels. */
 int esp_get_model_info(esp_ctx *ctx, int *out6);
 /* Clusters of blocks: out[0] = parts per replica their tables are laid out for (0: none),
- * out[1] = sweeps of the last esp_sweep or esp_run that they ran. */
-int esp_get_cluster_info(esp_ctx *ctx, int64_t *out2);
+ * out[1] = sweeps of the last esp_sweep or esp_run that they ran, out[2] = in how many launches
+ * (of at most 2^18 colour phases). */
+int esp_get_cluster_info(esp_ctx *ctx, int64_t *out3);
 /* Neighbour indexing of the global-memory colour phases: 0 = compute partner and reference
  * site indices from the device index when the supercell is periodic and translation
  * invariant (the geometry is verified against the tables for every site and slot first),
