@@ -978,12 +978,15 @@ int esp_set_sfactor(esp_ctx *c, int nq, const double *q, const double *pos, cons
               if (std::fabs(at(x0, x1, x2, a)[m] - r) > tol) { lat = false; break; }
             }
     if (lat) {
-      // distinct pairs (q.A0, q.A1)
+      // distinct pairs (q.A0, q.A1), told apart by their bits (NaN has no place in an order; adding
+      // zero makes both zeros one)
       auto along = [&](int iq, int k) {
-        const double *qq = q + 3 * (size_t)iq;
-        return qq[0] * A[k][0] + qq[1] * A[k][1] + qq[2] * A[k][2];
+        const double *qq = q + 3 * (size_t)iq, v = qq[0] * A[k][0] + qq[1] * A[k][1] + qq[2] * A[k][2] + 0.0;
+        uint64_t bits;
+        std::memcpy(&bits, &v, sizeof bits);
+        return bits;
       };
-      std::map<std::pair<double, double>, int> pairs;
+      std::map<std::pair<uint64_t, uint64_t>, int> pairs;
       std::vector<int> pair(nq), first;
       for (int iq = 0; iq < nq; ++iq) {
         const auto it = pairs.insert({{along(iq, 0), along(iq, 1)}, (int)first.size()});

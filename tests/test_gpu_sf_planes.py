@@ -41,3 +41,24 @@ def test_sfactor_by_planes(kind, L, R, qk, n):
     want = np.stack([B.sfactor(s[r], pos, q, polar) for r in range(R)])
     assert count == 1
     assert np.allclose(got, want, rtol=1e-11, atol=1e-13 * m.N ** 2)
+
+
+@pytest.mark.parametrize("bad", [[0], [3], [0, 5, 6]])
+def test_points_that_are_not_numbers(bad):
+    """A q-point that is not a number spoils its own S(q) only."""
+    from espins_amd.engine import Engine
+    m = Lt.cubic_model("sc", 6, J=(1.0,))
+    pos, q, polar = Lt.site_positions("sc", 6), q_points("random", 9), np.array([0.2, -0.5, 0.7])
+    q[bad, 0] = [np.nan, np.inf, np.nan][:len(bad)]
+    with Engine(0) as eng:
+        eng.set_path(1)
+        eng.set_model(m)
+        eng.set_replicas([0.5, 1.0], Lt.random_spins(m.N, 2, 4))
+        eng.set_sfactor(q, pos, polar, every=1)
+        eng.run(1, measure=True, exchange=False, seed=2)
+        got, _ = eng.obs(16, (2, 3, len(q)))
+        s = eng.spins()
+    good = np.setdiff1d(np.arange(len(q)), bad)
+    want = np.stack([B.sfactor(s[r], pos, q[good], polar) for r in range(2)])
+    assert np.allclose(got[:, :, good], want, rtol=1e-11, atol=1e-13 * m.N ** 2)
+    assert np.isnan(got[:, 0, bad]).all()
