@@ -120,11 +120,16 @@ struct esp_ctx {
     int have_polar = 0;
     double *d_q = nullptr, *d_pos = nullptr;   // [nq][3], [N][3] by device site
     double *d_sfspin = nullptr;    // [replica groups][N][8 or 4][3] spins of an S(q) evaluation
-    double *d_sfpart = nullptr;    // [site chunks][R][6][nq] partial F0; lattice: [R][L2 nb][6][npq]
-    int sf_chunk = 0, sf_nchunk = 0;      // site chunks; lattice: replica groups at a time
-    int sf_lat = 0, sfL[3] = {0, 0, 0};   // lattice positions: phases from tables
-    int npq = 0;                          // distinct pairs (q.A0, q.A1)
+    double *d_sfpart = nullptr;    // [site chunks][R][6][nq] partial F0; planes: [R][L2 nb][6][npq]
+    int sf_chunk = 0, sf_nchunk = 0;      // site chunks; planes: replica groups at a time
+    int sf_lat = 0, sfL[3] = {0, 0, 0};   // lattice positions: the way they are summed (kSfPlanes, kSfRows)
+    int npq = 0;                          // distinct pairs (q.A0, q.A1) (rows: nq)
     int *d_sfpair = nullptr;              // [nq] pair of each q-point
+    struct {                              // a lattice's q-points, steps and cell, pairs; first q-point of each
+      std::vector<double> q, B;
+      double A[3][3];
+      std::vector<int> pair, first;
+    } sflat;
     double2 *d_sftab = nullptr;    // [L0 + L1][npq], [L2 + nb][nq]: exp(i q.x A_k), exp(i q.B_a)
     double *d_sf = nullptr;        // [R][3][nq]
     unsigned long long *d_sfn = nullptr;      // structure-factor measurements

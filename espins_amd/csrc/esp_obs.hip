@@ -12,7 +12,7 @@
 // counts through a histogram in LDS), k_obs_spincorr (one thread per site and several
 // replicas, device order), k_sf_pack / k_sf_main / k_sf_fin (S(q) as a phase-matrix times
 // spin-matrix product: one phase per q-point, site and 8 replicas; k_sf_plane / k_sf_q for lattice
-// positions: summed axis by axis) and k_obs_final (per replica: fixed-order sums of the
+// positions: summed axis by axis; k_sf_lat for lattices of few sites to a plane or of few planes) and k_obs_final (per replica: fixed-order sums of the
 // block partials, accumulation into the replica's slot).
 // Histogram counts are integers, so they do not depend on the order of the atomic additions;
 // every floating-point sum has a fixed order.
@@ -38,6 +38,7 @@ constexpr int kSfRep = 8;             // replicas per structure-factor wave (sin
 constexpr int kSfRepLat = 4;          // replicas per structure-factor wave (lattice path)
 constexpr int kSfWaves = 4096;        // structure-factor waves aimed at (site chunks fill up to it)
 constexpr int kSfMaxChunks = 64;
+enum { kSfPlanes = 1, kSfRows = 2 };  // lattice positions: axis by axis, or a phase per site (sf_planes)
 constexpr size_t kSfPlaneBytes = size_t(256) << 20;   // plane sums held at a time (lattice path)
 constexpr int kPmLdsBins = 12288;     // P(m) bins counted in LDS (48 KiB); more use global atomics
 
@@ -65,7 +66,7 @@ struct ObsArgs {
   double *sfspin, *sfpart;
   int sf_chunk, sf_nchunk;
   // lattice positions r = B_a + x0 A0 + x1 A1 + x2 A2 (reference order ((x2 L1 + x1) L0 + x0) nb
-  // + a): phase tables exp(i q.x0 A0), exp(i q.x1 A1) by distinct pair (q.A0, q.A1), [x][pair], and
+  // + a): phase tables exp(i q.x0 A0), exp(i q.x1 A1) by distinct pair (q.A0, q.A1), [x][pair] (by rows: [x][q]), and
   // exp(i q.x2 A2), exp(i q.B_a), [k][q]; sfpair: the pair of each q-point
   int sf_lat, sfL[3], sf_rep;         // sf_rep: replicas per group of the packed spins
   int npq, sf_g0;                     // pairs; first replica group of the launch
@@ -271,10 +272,11 @@ __device__ __forceinline__ bool sf_due(const ObsArgs &o) {
 
 __global__ __launch_bounds__(kObsBlock) void k_sf_pack(ObsArgs o) {
   if (!sf_due(o)) return;
-  const int j = blockIdx.x * kObsBlock + threadIdx.x;    // device site, or place ((x2 nb + a) L1 + x1) L0 + x0
+  // device site; by planes: place ((x2 nb + a) L1 + x1) L0 + x0; by rows: reference site
+  const int j = blockIdx.x * kObsBlock + threadIdx.x;
   if (j >= o.N) return;
-  int d = j;
-  if (o.sf_lat) {
+  int d = o.sf_lat == kSfRows ? gldi(o.ref2dev, j) : j;
+  if (o.sf_lat == kSfPlanes) {
     const int L0 = o.sfL[0], L1 = o.sfL[1], x0 = j % L0, x1 = j / L0 % L1, pl = j / (L0 * L1);
     d = gldi(o.ref2dev, (((pl / o.nb) * L1 + x1) * L0 + x0) * o.nb + pl % o.nb);
   }
@@ -436,6 +438,71 @@ __global__ __launch_bounds__(kObsBlock) void k_sf_q(ObsArgs o) {
   sf_accumulate(o, iq, r, fr, fi);
 }
 
+// Lattices of which axis-by-axis sums make little (sf_planes): the phase of site (x0, x1, x2, a) is
+// the product of the four table entries, one complex product per site and q-point.  A chunk is a
+// range of (x1, x2) rows, sites in reference order inside a row; k_sf_fin adds the chunks.
+__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
+  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+__global__ __launch_bounds__(kSfQ) void k_sf_lat(ObsArgs o) {
+  constexpr int RV = kSfRepLat * 3;                 // spin values of one site and group
+  if (!sf_due(o)) return;
+  const int iq0 = blockIdx.x * kSfQ + threadIdx.x;
+  const int iq = min(iq0, o.nq - 1);                 // lanes past nq compute q nq-1, store nothing
+  const int g = blockIdx.y, ch = blockIdx.z;
+  const int L0 = o.sfL[0], L1 = o.sfL[1], nb = o.nb;
+  const int rows = L1 * o.sfL[2];
+  const int w0 = ch * o.sf_chunk, w1 = min(rows, w0 + o.sf_chunk);
+  double fr[kSfRepLat][3], fi[kSfRepLat][3];
+#pragma unroll
+  for (int u = 0; u < kSfRepLat; ++u)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { fr[u][k] = 0.0; fi[u][k] = 0.0; }
+  auto add = [&](const double (&v)[RV], double2 ph) {
+#pragma unroll
+    for (int u = 0; u < kSfRepLat; ++u)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        fr[u][k] += v[3 * u + k] * ph.x;
+        fi[u][k] += v[3 * u + k] * ph.y;
+      }
+  };
+  const double *spg = o.sfspin + (size_t)g * o.N * RV;
+  for (int w = w0; w < w1; ++w) {
+    const double2 byz = cmul(ld2(o.sfey, (size_t)(w % L1) * o.nq + iq), ld2(o.sfez, (size_t)(w / L1) * o.nq + iq));
+    for (int x0 = 0; x0 < L0; ++x0) {
+      const double2 bx = cmul(ld2(o.sfex, (size_t)x0 * o.nq + iq), byz);
+      const double *sv0 = spg + ((size_t)w * L0 + x0) * nb * RV;
+      int a = 0;
+      for (; a + 1 < nb; a += 2) {     // two sites per wait on the (out-of-order) scalar loads
+        double v0[RV], v1[RV];
+#pragma unroll
+        for (int k = 0; k < RV; ++k) { v0[k] = sv0[(size_t)a * RV + k]; v1[k] = sv0[(size_t)(a + 1) * RV + k]; }
+        add(v0, cmul(bx, ld2(o.sfeb, (size_t)a * o.nq + iq)));
+        add(v1, cmul(bx, ld2(o.sfeb, (size_t)(a + 1) * o.nq + iq)));
+      }
+      if (a < nb) {
+        double v0[RV];
+#pragma unroll
+        for (int k = 0; k < RV; ++k) v0[k] = sv0[(size_t)a * RV + k];
+        add(v0, cmul(bx, ld2(o.sfeb, (size_t)a * o.nq + iq)));
+      }
+    }
+  }
+  if (iq0 >= o.nq) return;
+#pragma unroll
+  for (int u = 0; u < kSfRepLat; ++u) {
+    const int r = g * kSfRepLat + u;
+    if (r >= o.R) break;
+    double *out = o.sfpart + ((size_t)ch * o.R + r) * 6 * o.nq + iq;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      gsti(out, (size_t)k * o.nq, fr[u][k]);
+      gsti(out, (size_t)(3 + k) * o.nq, fi[u][k]);
+    }
+  }
+}
+
 __global__ __launch_bounds__(kObsBlock) void k_sf_fin(ObsArgs o) {
   if (!sf_due(o)) return;
   const int iq = blockIdx.x * kObsBlock + threadIdx.x;
@@ -575,6 +642,70 @@ int need_model(esp_ctx *c) {
   return ESP_OK;
 }
 
+// Chunks of `units` pieces of the sum over N sites, nq q-points, ng replica groups: enough waves to
+// fill the chip, at least 64 sites each.
+int sf_chunks(int units, int N, int nq, int ng) {
+  const int w = ng * ((nq + kSfQ - 1) / kSfQ);
+  return std::max(1, std::min({(kSfWaves + w - 1) / w, kSfMaxChunks, units, (N + 63) / 64}));
+}
+
+// Bytes of the plane sums of one replica group.
+size_t sf_plane_bytes(const int (&L)[3], int nb, int npq) {
+  return sizeof(double) * kSfRepLat * 6 * L[2] * nb * npq;
+}
+
+// Whether a lattice's S(q) is summed axis by axis (k_sf_plane, k_sf_q) rather than with a phase per
+// site (k_sf_lat): estimates in us, each the longer of one wave's chain and the whole work at the rate
+// measured.  A plane's wave takes 0.15 us a site and 0.45 a row, k_sf_q 0.2 a plane and a rate bound by
+// the planes' sums it reads; k_sf_lat 0.5 us a site, 150 ns for 64 q-points, 4 replicas and 1000 sites.
+// us an evaluation, planes / rows, 2601 q-points sharing 51 pairs, 32 replicas: 32^3 231 / 1651, fcc
+// 16^3 100 / 533, 8x8x64 54 / 223, 64x8x8 101 / 221, 4x4x256 123 / 256, 2x2x1024 422 / 297, 64x64x1
+// 679 / 220, 1x1x4096 1614 / 386; one replica: 194 / 312, 51 / 110, 36 / 68, 93 / 72, 76 / 73, 285 / 79,
+// 643 / 72, 1107 / 95.  Over 84 lattices, counts and sets of q-points the choice was never slower than
+// k_sf_lat by more than the runs differ.
+bool sf_planes(const int (&L)[3], int nb, int npq, int nq, int R) {
+  if ((int64_t)L[2] * nb > 65535 || sf_plane_bytes(L, nb, npq) > kSfPlaneBytes) return false;
+  const int ng = (R + kSfRepLat - 1) / kSfRepLat;
+  const double planes = (double)L[2] * nb, sites = planes * L[0] * L[1];
+  const double qw = (nq + kSfQ - 1) / kSfQ * (double)ng, pw = (npq + kSfQ - 1) / kSfQ * (double)ng;
+  const double t_planes = std::max(L[1] * (0.15 * L[0] + 0.45), 2.9e-6 * pw * planes * L[1] * (24.0 * L[0] + 48.0)) +
+                          std::max(0.2 * planes, R * planes * (4.7e-6 * nq + 3.5e-5 * npq));
+  const int units = L[1] * L[2], nch = sf_chunks(units, (int)sites, nq, ng);
+  const double t_rows = std::max(20.0 + 0.5 * ((units + nch - 1) / nch) * L[0] * nb, 1.5e-4 * qw * sites);
+  return t_planes < t_rows;
+}
+
+// Phase tables of lattice positions for the way S(q) is summed with R replicas: exp(i q.x0 A0) and
+// exp(i q.x1 A1) per pair (planes) or q-point (rows), exp(i q.x2 A2) and exp(i q.B_a) per q-point.
+int sf_tables(esp_ctx *c) {
+  auto &b = c->obs;
+  const int nb = c->hm.nb, nq = b.nq;
+  const auto &sl = b.sflat;
+  const int way = sf_planes(b.sfL, nb, (int)sl.first.size(), nq, c->R) ? kSfPlanes : kSfRows;
+  if (b.sf_lat == way && b.d_sftab) return ESP_OK;
+  const bool planes = way == kSfPlanes;
+  const int np = planes ? (int)sl.first.size() : nq;
+  std::vector<double2> tab((size_t)(b.sfL[0] + b.sfL[1]) * np + (size_t)(b.sfL[2] + nb) * nq);
+  size_t at0 = 0;
+  auto phase = [&](int iq, double x, double y, double z) {
+    const double *qq = &sl.q[3 * (size_t)iq];
+    const double ph = qq[0] * x + qq[1] * y + qq[2] * z;
+    tab[at0++] = make_double2(std::cos(ph), std::sin(ph));
+  };
+  for (int k = 0; k < 3; ++k)
+    for (int x = 0; x < b.sfL[k]; ++x)
+      for (int i = 0; i < (k < 2 ? np : nq); ++i)
+        phase(k < 2 && planes ? sl.first[i] : i, x * sl.A[k][0], x * sl.A[k][1], x * sl.A[k][2]);
+  for (int a = 0; a < nb; ++a)
+    for (int iq = 0; iq < nq; ++iq) phase(iq, sl.B[3 * (size_t)a], sl.B[3 * (size_t)a + 1], sl.B[3 * (size_t)a + 2]);
+  int rc;
+  if ((rc = upload(c, b.d_sftab, tab)) || (rc = upload(c, b.d_sfpair, sl.pair))) return rc;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  b.npq = np;
+  b.sf_lat = way;
+  return ESP_OK;
+}
+
 // Model-level tables of one observable changed: drop the graph, resize the accumulators.
 int changed(esp_ctx *c) {
   drop_graph(c);
@@ -628,22 +759,21 @@ int obs_resize(esp_ctx *c) {
   if (b.flags & ESP_OBS_SFACTOR) {
     if ((rc = dalloc(c, b.d_sf, (size_t)R * 3 * b.nq))) return rc;
     if ((rc = dalloc(c, b.d_sfn, 1))) return rc;
+    if (b.sf_lat && (rc = sf_tables(c))) return rc;
     const int srep = b.sf_lat ? kSfRepLat : kSfRep;
     const int ng = (R + srep - 1) / srep;
     size_t npart;
-    if (b.sf_lat) {
+    if (b.sf_lat == kSfPlanes) {
       // plane sums of as many replica groups at a time as kSfPlaneBytes hold
-      const size_t per = (size_t)srep * b.sfL[2] * nb * 6 * b.npq;
-      b.sf_chunk = (int)std::max<size_t>(1, std::min<size_t>(ng, kSfPlaneBytes / (per * sizeof(double))));
+      const size_t per = sf_plane_bytes(b.sfL, nb, b.npq);
+      b.sf_chunk = (int)std::min<size_t>(ng, kSfPlaneBytes / per);
       b.sf_nchunk = (ng + b.sf_chunk - 1) / b.sf_chunk;
-      npart = per * b.sf_chunk;
+      npart = per / sizeof(double) * b.sf_chunk;
     } else {
-      // site chunks: enough waves to fill the chip, at least 64 sites each
-      const int nqb = (b.nq + kSfQ - 1) / kSfQ;
-      int nch = (kSfWaves + ng * nqb - 1) / (ng * nqb);
-      nch = std::max(1, std::min({nch, kSfMaxChunks, N, (N + 63) / 64}));
-      b.sf_chunk = (N + nch - 1) / nch;
-      b.sf_nchunk = (N + b.sf_chunk - 1) / b.sf_chunk;
+      // site chunks (lattice: chunks of (x1, x2) rows)
+      const int units = b.sf_lat ? b.sfL[1] * b.sfL[2] : N, nch = sf_chunks(units, N, b.nq, ng);
+      b.sf_chunk = (units + nch - 1) / nch;
+      b.sf_nchunk = (units + b.sf_chunk - 1) / b.sf_chunk;
       npart = (size_t)b.sf_nchunk * R * 6 * b.nq;
     }
     if ((rc = dalloc(c, b.d_sfspin, (size_t)ng * N * srep * 3))) return rc;
@@ -692,7 +822,7 @@ int obs_enqueue(esp_ctx *c) {
     const int srep = b.sf_lat ? kSfRepLat : kSfRep;
     const int ng = (c->R + srep - 1) / srep;
     hipLaunchKernelGGL(k_sf_pack, dim3((o.N + kObsBlock - 1) / kObsBlock, ng), dim3(kObsBlock), 0, c->stream, o);
-    if (b.sf_lat) {
+    if (b.sf_lat == kSfPlanes) {
       ObsArgs p = o;
       for (int g0 = 0; g0 < ng; g0 += b.sf_chunk) {
         const int n = std::min(b.sf_chunk, ng - g0), nr = std::min(c->R - g0 * srep, n * srep);
@@ -701,7 +831,8 @@ int obs_enqueue(esp_ctx *c) {
         hipLaunchKernelGGL(k_sf_q, dim3((b.nq + kObsBlock - 1) / kObsBlock, nr), dim3(kObsBlock), 0, c->stream, p);
       }
     } else {
-      hipLaunchKernelGGL(k_sf_main, dim3((b.nq + kSfQ - 1) / kSfQ, ng, b.sf_nchunk), dim3(kSfQ), 0, c->stream, o);
+      hipLaunchKernelGGL(b.sf_lat ? k_sf_lat : k_sf_main, dim3((b.nq + kSfQ - 1) / kSfQ, ng, b.sf_nchunk), dim3(kSfQ), 0,
+                         c->stream, o);
       hipLaunchKernelGGL(k_sf_fin, dim3((b.nq + kObsBlock - 1) / kObsBlock, c->R), dim3(kObsBlock), 0, c->stream, o);
     }
   }
@@ -938,6 +1069,7 @@ int esp_set_sfactor(esp_ctx *c, int nq, const double *q, const double *pos, cons
   b.flags &= ~ESP_OBS_SFACTOR;
   b.nq = 0;
   b.sf_lat = 0;
+  b.sflat = {};
   if (nq == 0) return changed(c);
   if (nq < 0 || !q || !pos || every < 1) return fail(c, ESP_EINVAL, "esp_set_sfactor: bad arguments");
   const int N = c->hm.N;
@@ -987,31 +1119,18 @@ int esp_set_sfactor(esp_ctx *c, int nq, const double *q, const double *pos, cons
         return bits;
       };
       std::map<std::pair<uint64_t, uint64_t>, int> pairs;
-      std::vector<int> pair(nq), first;
+      std::vector<int> &pair = b.sflat.pair, &first = b.sflat.first;
+      pair.resize(nq);
       for (int iq = 0; iq < nq; ++iq) {
         const auto it = pairs.insert({{along(iq, 0), along(iq, 1)}, (int)first.size()});
         if (it.second) first.push_back(iq);
         pair[iq] = it.first->second;
       }
-      const int np = (int)first.size();
-      std::vector<double2> tab((size_t)(L[0] + L[1]) * np + (size_t)(L[2] + nb) * nq);
-      size_t at0 = 0;
-      auto phase = [&](int iq, double x, double y, double z) {
-        const double *qq = q + 3 * (size_t)iq;
-        const double ph = qq[0] * x + qq[1] * y + qq[2] * z;
-        tab[at0++] = make_double2(std::cos(ph), std::sin(ph));
-      };
-      for (int k = 0; k < 3; ++k)
-        for (int x = 0; x < L[k]; ++x)
-          for (int i = 0; i < (k < 2 ? np : nq); ++i)
-            phase(k < 2 ? first[i] : i, x * A[k][0], x * A[k][1], x * A[k][2]);
-      for (int a = 0; a < nb; ++a)
-        for (int iq = 0; iq < nq; ++iq) phase(iq, pos[3 * (size_t)a], pos[3 * (size_t)a + 1], pos[3 * (size_t)a + 2]);
-      if ((rc = upload(c, b.d_sftab, tab)) || (rc = upload(c, b.d_sfpair, pair))) return rc;
-      HIPCHK(c, hipStreamSynchronize(c->stream));
-      b.npq = np;
-      b.sf_lat = 1;
+      b.sflat.q.assign(q, q + 3 * (size_t)nq);
+      b.sflat.B.assign(pos, pos + 3 * (size_t)nb);
+      std::memcpy(b.sflat.A, A, sizeof A);
       for (int k = 0; k < 3; ++k) b.sfL[k] = L[k];
+      b.sf_lat = kSfRows;                        // (sf_tables decides with the replica count)
     }
   }
   b.nq = nq;
