@@ -464,33 +464,34 @@ struct Plan {
   int nl_max = 0, ngroup = 0;
 };
 
-// Cuts the sites (reference order) into k parts and builds their tables; false if a part does
-// not fit.
+// Cuts the sites (reference order) into k parts and builds their tables; false, as soon as that is
+// known, if a part does not fit.  (A replica whose k parts do not fit needs more CUs: fewer parts
+// have more sites each and reach as many others.)
 bool make_plan(const esp::HostModel &m, int k, int R, size_t lds_max, Plan &p) {
   const int N = m.N;
   p = Plan{};
-  if ((size_t)((N + k - 1) / k) * 3 * sizeof(double) > lds_max) return false;
+  if (!cluster_fits(m, (N + k - 1) / k, R, lds_max)) return false;
   p.ngroup = (m.zmax + kGroup - 1) / kGroup;
   const int npair = p.ngroup * kGroup / 2;
-  std::vector<int> part_of(N), local(N, -1);          // by device site
+  std::vector<int> part_of(N), local(N, -1), seen(N, -1);     // by device site
   for (int d = 0; d < N; ++d) part_of[d] = (int)((long long)m.dev2ref[d] * k / N);
   std::vector<std::vector<int>> own(k), hal(k);
   for (int d = 0; d < N; ++d) own[part_of[d]].push_back(d);   // device order: by colour
   std::vector<std::vector<char>> touch(k, std::vector<char>(k, 0));
-  std::vector<std::vector<char>> mark(k, std::vector<char>(N, 0));
-  for (int l = 0; l < m.zmax; ++l)
-    for (int d = 0; d < N; ++d) {
-      const int q = m.nbr[(size_t)l * N + d], j = part_of[d];
-      if (q == N || part_of[q] == j || mark[j][q]) continue;
-      touch[j][part_of[q]] = touch[part_of[q]][j] = 1;        // reader and writer wait for each other
-      mark[j][q] = 1;
-    }
   for (int j = 0; j < k; ++j) {
-    for (int d = 0; d < N; ++d)
-      if (mark[j][d]) hal[j].push_back(d);                    // device order: by colour
+    for (int l = 0; l < m.zmax; ++l) {
+      for (int d : own[j]) {
+        const int q = m.nbr[(size_t)l * N + d];
+        if (q == N || part_of[q] == j || seen[q] == j) continue;
+        touch[j][part_of[q]] = touch[part_of[q]][j] = 1;      // reader and writer wait for each other
+        seen[q] = j;
+        hal[j].push_back(q);
+      }
+      if (!cluster_fits(m, (int)(own[j].size() + hal[j].size()), R, lds_max)) return false;
+    }
+    std::sort(hal[j].begin(), hal[j].end());                  // device order: by colour
     p.nl_max = std::max(p.nl_max, (int)(own[j].size() + hal[j].size()));
   }
-  if (!cluster_fits(m, p.nl_max, R, lds_max)) return false;
   for (int j = 0; j < k; ++j) {
     Part t{};
     t.nown = (int)own[j].size();
@@ -569,7 +570,7 @@ void cluster_free(esp_ctx *c) {
 int cluster_prepare(esp_ctx *c) {
   if (c->cluster_R == c->R) return ESP_OK;
   const HostModel &m = c->hm;
-  int k = cluster_parts(m, c->R, c->num_cu);
+  const int k = cluster_parts(m, c->R, c->num_cu);
   // (the tables depend on the model and k, the LDS of a block also on the replica count)
   if (c->cluster && c->cluster->k == k && cluster_fits(m, c->cluster->nl_max, c->R, c->lds_max)) {
     c->cluster_R = c->R;
@@ -578,8 +579,7 @@ int cluster_prepare(esp_ctx *c) {
   cluster_free(c);
   c->cluster_R = c->R;
   Plan p;
-  while (k >= 2 && !make_plan(m, k, c->R, c->lds_max, p)) --k;      // (fewer parts only grow)
-  if (k < 2) return ESP_OK;
+  if (k < 2 || !make_plan(m, k, c->R, c->lds_max, p)) return ESP_OK;
   esp_cluster *q = c->cluster = new esp_cluster();
   q->k = k; q->nl_max = p.nl_max; q->ngroup = p.ngroup;
   std::vector<char> img;
@@ -683,10 +683,9 @@ int esp_plan_clusters(int N, int nb, const double *mag, int zJ, const int *j_cnt
   if (!esp::prepare_model(hm, N, nb, mag, zJ, j_cnt, j_nbr, j_val, zB, b_cnt, b_nbr, b_val, zD, d_cnt, d_nbr, d_vec, 0,
                           nullptr, nullptr, 0, nullptr, nullptr, L).empty())
     return ESP_EINVAL;
-  int k = cluster_parts(hm, R, num_cu);
+  const int k = cluster_parts(hm, R, num_cu);
   Plan p;
-  while (k >= 2 && !make_plan(hm, k, R, (size_t)lds_bytes, p)) --k;
-  const bool on = k >= 2;
+  const bool on = k >= 2 && make_plan(hm, k, R, (size_t)lds_bytes, p);
   out[0] = on ? k : 0;
   out[1] = on ? p.nl_max : 0;
   out[2] = on ? (int64_t)cluster_lds(hm, p.nl_max, R) : 0;
