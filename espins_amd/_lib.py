@@ -62,6 +62,7 @@ _SIGS = {
     "esp_plan_clusters": (_i, [_i, _i, _dp, _i, _ip, _ip, _dp, _i, _ip, _ip, _dp, _i, _ip, _ip, _dp,
                                _ip, _i, _i, C.c_int64, _i64p]),
     "esp_get_cluster_info": (_i, [_p, _i64p]),
+    "esp_set_cluster_limit": (_i, [_p, _i]),
     "esp_get_coloring": (_i, [_p, _ip, _ip]),
     "esp_get_model_info": (_i, [_p, _ip]),
     "esp_set_replicas": (_i, [_p, _i, _dp, _dp]),

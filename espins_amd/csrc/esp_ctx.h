@@ -63,6 +63,8 @@ struct esp_ctx {
   esp_cluster *cluster = nullptr;
   int cluster_R = 0;
   int64_t cluster_sweeps = 0, cluster_launches = 0;   // of the last esp_sweep / esp_run, what clusters ran
+  int cluster_limit = -1;         // launches after which they leave (-1: no limit; for tests)
+  int cluster_skip = 0, cluster_wait = 0;   // runs to go without them, and how many the last time
   bool w_dirty = false;           // d_w may hold sums (the launch-per-colour path ran since a fold)
   // host-fed staging
   double *d_prop = nullptr, *d_unif = nullptr;
@@ -146,7 +148,7 @@ namespace esp {
 // Clusters (esp_cluster.hip): decide and build tables once per (model, replicas); run; free.
 int cluster_prepare(esp_ctx *c);
 int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, int M, bool measure, bool exchange,
-                int round, int64_t *ran);
+                int round, int64_t *ran, bool *left);
 void cluster_free(esp_ctx *c);
 }  // namespace esp
 
@@ -205,6 +207,7 @@ void free_replicas(esp_ctx *c) {
   c->trace_cap = 0;
   c->w_dirty = false;
   c->cluster_sweeps = c->cluster_launches = 0;
+  c->cluster_skip = c->cluster_wait = 0;
   dfree(c->d_mpart); dfree(c->d_mpart_l);
   c->mpart_nw = 0;
   c->mpart_valid = false;

@@ -9,6 +9,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -349,6 +350,17 @@ bool lds_sweeps(const esp_ctx *c, int mode) {
   return c->use_lds && mode != ESP_MODE_LEARNED && !c->d_trace && !c->obs.flags;
 }
 
+// Runs of contexts on one device at the moment.
+std::atomic<int> &running(const esp_ctx *c) {
+  static std::atomic<int> n[64];
+  return n[c->device & 63];
+}
+struct Running {
+  std::atomic<int> &n;
+  explicit Running(const esp_ctx *c) : n(running(c)) { ++n; }
+  ~Running() { --n; }
+};
+
 // Clusters of blocks may serve the plain proposals of the automatic path.
 bool cluster_possible(const esp_ctx *c, int mode) {
   return c->path == 0 && !c->tps_user && (mode == ESP_MODE_RANDOM || mode == ESP_MODE_CONST) && !c->obs.flags;
@@ -358,6 +370,7 @@ bool cluster_possible(const esp_ctx *c, int mode) {
 // that one block holds (k_lds) get them in a run that is long enough to pay for it (0.6 ms).
 constexpr int kClusterMinSites = 384;
 constexpr int kClusterLateSteps = 256;
+constexpr int kClusterSkip = 256;
 bool cluster_early(const esp_ctx *c, int mode) {
   return cluster_possible(c, mode) && (!lds_sweeps(c, mode) || c->hm.N / std::max(1, c->hm.ncol) >= kClusterMinSites);
 }
@@ -370,9 +383,11 @@ bool cluster_early(const esp_ctx *c, int mode) {
 // cluster 8 + 2.7 per phase: 11.2 / 7.4 (sc 12^3, 2 colours, 2 passes), 14.0 / 13.6 (sc 16^3, 4),
 // 18.4 / 16.4 (with second neighbours, 4 colours, 2 passes), 18.8 / 23.5 (sc 14^3, 4 and 3),
 // 28.3 / 32.6 (fcc 10^3, 8 and 2).
+// Beside runs of other contexts k_lds leaves them the CUs that it does not need.
 bool cluster_sweeps(const esp_ctx *c, int mode, bool exchange, int round, int nsteps) {
   if (!cluster_possible(c, mode)) return false;
   if (!lds_sweeps(c, mode)) return true;
+  if (running(c) > 1) return false;
   const bool early = cluster_early(c, mode);
   if (exchange && round <= 3)
     return early || (c->cluster && c->cluster_R == c->R) || nsteps >= kClusterLateSteps;
@@ -389,13 +404,24 @@ int run_clusters(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, i
   if (!cluster_sweeps(c, mode, exchange, round, nsteps)) return ESP_OK;
   int rc = esp::cluster_prepare(c);
   if (rc || !c->cluster) return rc;
+  // A launch that found its CUs taken cost its wait: 1, 2, 4, ... kClusterSkip runs go without
+  // before the next try.
+  if (c->cluster_skip > 0) {
+    --c->cluster_skip;
+    return ESP_OK;
+  }
   if (c->w_dirty) {          // the clusters count their accepted dE on top of e_base
     hipLaunchKernelGGL(k_fold_w, dim3((c->R + 255) / 256), dim3(256), 0, c->stream, c->d_w,
                        c->hm.ncol * c->mpart_nw, c->R, c->d_ebase);
     HIPCHK(c, hipGetLastError());
     c->w_dirty = false;
   }
-  rc = esp::cluster_run(c, mode, tilt, seed, nsteps, M, measure, exchange, round, ran);
+  bool left = false;
+  rc = esp::cluster_run(c, mode, tilt, seed, nsteps, M, measure, exchange, round, ran, &left);
+  if (left)
+    c->cluster_skip = c->cluster_wait = std::min(kClusterSkip, std::max(1, 2 * c->cluster_wait));
+  else if (*ran > 0)
+    c->cluster_wait = 0;
   c->cluster_sweeps = *ran;
   return rc;
 }
@@ -797,6 +823,7 @@ int esp_sweep(esp_ctx *c, int nsweeps, int mode, double tilt, uint64_t seed, uin
   if (nsweeps < 0 || (mode != ESP_MODE_RANDOM && mode != ESP_MODE_CONST && mode != ESP_MODE_LEARNED))
     return fail(c, ESP_EINVAL, "bad nsweeps / mode");
   if (nsweeps == 0) return ESP_OK;
+  const Running here(c);
   if ((rc = set_clock(c, sweep0, 0, 1))) return rc;
   int64_t ran = 0;
   if ((rc = run_clusters(c, mode, tilt, seed, nsweeps, 1, false, false, 1, &ran))) return rc;
@@ -871,6 +898,7 @@ int esp_run(esp_ctx *c, int n_rounds, int steps_per_round, int steps_measure, in
       (mode != ESP_MODE_RANDOM && mode != ESP_MODE_CONST && mode != ESP_MODE_LEARNED))
     return fail(c, ESP_EINVAL, "bad esp_run arguments");
   if (n_rounds == 0) return ESP_OK;
+  const Running here(c);
   if ((rc = set_clock(c, sweep0, step0, start_parity))) return rc;
   if ((int64_t)n_rounds * steps_per_round < (1ll << 30)) {
     int64_t ran = 0;

@@ -131,10 +131,15 @@ class Engine:
 
     def cluster_info(self):
         """Clusters of blocks (the automatic path of middle-sized replicas): parts per replica (0: none)
-        and the sweeps of the last sweep() or run() that they ran, in how many launches."""
-        out = np.zeros(3, np.int64)
+        the sweeps of the last sweep() or run() that they ran, in how many launches, and the runs
+        that go without them before they are tried again."""
+        out = np.zeros(4, np.int64)
         self._chk(E.lib.esp_get_cluster_info(self._h, E.ptr(out, C.c_int64)))
-        return dict(parts=int(out[0]), sweeps=int(out[1]), launches=int(out[2]))
+        return dict(parts=int(out[0]), sweeps=int(out[1]), launches=int(out[2]), skip=int(out[3]))
+
+    def set_cluster_limit(self, launches):
+        """For tests: cluster launches after the next `launches` find their CUs taken (-1: no limit)."""
+        self._chk(E.lib.esp_set_cluster_limit(self._h, int(launches)))
 
     # ---- replicas --------------------------------------------------------------------
     def set_replicas(self, tems, spins):

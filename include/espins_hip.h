@@ -124,8 +124,12 @@ int esp_get_coloring(esp_ctx *ctx, int *ncol, int *colour);
 int esp_get_model_info(esp_ctx *ctx, int *out6);
 /* Clusters of blocks: out[0] = parts per replica their tables are laid out for (0: none),
  * out[1] = sweeps of the last esp_sweep or esp_run that they ran, out[2] = in how many launches
- * (of at most 2^18 colour phases). */
-int esp_get_cluster_info(esp_ctx *ctx, int64_t *out3);
+ * (of at most 2^18 colour phases), out[3] = runs that go without them before they are tried
+ * again (a launch found its CUs taken by other work). */
+int esp_get_cluster_info(esp_ctx *ctx, int64_t *out4);
+/* For tests: the clusters' launches after the next `launches` find their CUs taken (-1, the
+ * default: no limit). */
+int esp_set_cluster_limit(esp_ctx *ctx, int launches);
 /* Neighbour indexing of the global-memory colour phases: 0 = compute partner and reference
  * site indices from the device index when the supercell is periodic and translation
  * invariant (the geometry is verified against the tables for every site and slot first),
