@@ -1168,6 +1168,7 @@ int esp_batch_reset_stats(esp_batch *b) {
     hipLaunchKernelGGL(k_zero_stats, dim3((kRejSub * c.R + 255) / 256), dim3(256), 0, b->stream, c.acc, c.rej, c.nswap,
                        c.nmeas, c.R);
   BCHK(b, hipGetLastError());
+  BCHK(b, hipStreamSynchronize(b->stream));
   return ESP_OK;
 }
 

@@ -1109,7 +1109,9 @@ int esp_reset_stats(esp_ctx *c) {
   hipLaunchKernelGGL(k_zero_stats, dim3((kRejSub * R + 255) / 256), dim3(256), 0, c->stream, c->d_acc, c->d_rej,
                      c->d_nswap, c->d_nmeas, R);
   HIPCHK(c, hipGetLastError());
-  return esp::obs_clear(c);      // (in stream order: every later call sees them cleared)
+  if ((rc = esp::obs_clear(c))) return rc;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return ESP_OK;
 }
 
 int esp_sync(esp_ctx *c) {
