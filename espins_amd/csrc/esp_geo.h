@@ -58,6 +58,20 @@ ESP_HD uint32_t fdiv(uint32_t n, const FastDiv &f) {
   return (t + ((n - t) >> f.s1)) >> f.s2;
 }
 
+// Replica r and block b that block L of a launch of nblk blocks for each of R replicas takes
+// (full = xcd_full(R, nblk), dnblk divides by nblk).  Blocks go round-robin over the 8 XCDs, each
+// with an L2 of its own: eight replicas at a time are dealt one to an XCD, with all their blocks;
+// the last R % 8 are spread.  A replica whose blocks run on every XCD is read into every L2: us per
+// colour phase with all replicas spread / so: FCC 16^3 x 244, three shells 75.6 / 38.8, FCC 32^3 x 60
+// 62.5 / 40.6, BCC 20^3 x 100 24.6 / 17.8, SC 64^3 x 30 75.1 / 66.5, FCC 18^3 x 41 learned 29.8 / 26.2.
+ESP_HD void place_block(uint32_t L, uint32_t full, const FastDiv &dnblk, int &r, int &b) {
+  const bool own = L < full;
+  const uint32_t q = own ? L >> 3 : L, w = fdiv(q, dnblk);
+  b = (int)(q - w * dnblk.d);
+  r = (int)(own ? (L & 7u) + 8u * w : w);
+}
+inline uint32_t xcd_full(int R, int nblk) { return (uint32_t)(R / 8 * 8) * (uint32_t)nblk; }
+
 // Geometry of one model (host-built, passed by value to the kernels).
 struct Geo {
   FastDiv mt, m0, m1;            // Mt, M0, M1

@@ -198,7 +198,6 @@ KArgs phase_args(esp_ctx *c, double tilt, uint64_t seed) {
   KArgs a = base_args(c);
   a.tilt = tilt;
   a.key0 = (uint32_t)seed; a.key1 = (uint32_t)(seed >> 32);
-  a.xcd_remap = (c->R % 8 == 0) ? 1 : 0;
   a.mpart = c->d_mpart;
   a.mpart_nw = c->mpart_nw;
   return a;
@@ -211,6 +210,7 @@ void set_colour(KArgs &a, const esp::HostModel &m, int col, int lay) {
   a.c_count = m.col_off[col + 1] - m.col_off[col];
   a.nblk = colour_blocks(m, col, a.tps, lay == LAY_IMP);
   a.dnblk = espg::make_fastdiv((uint32_t)std::max(1, a.nblk));
+  a.xcd_full = espg::xcd_full(a.R, a.nblk);
   if (lay == LAY_IMP) a.dngc = geo_ngc(m, col);
 }
 
@@ -855,7 +855,6 @@ int esp_sweep_hostfed(esp_ctx *c, const double *prop, const double *unif, uint8_
   PhaseFn fn = phase_fn(M_HOSTFED, c, launch_lanes(c));
   if ((rc = set_clock(c, 0, 0, 1))) return rc;
   a.tps = 1;
-  a.xcd_remap = (c->R % 8 == 0);
   const int lay = phase_kernel_layout(c, 1);
   for (int col = 0; col < m.ncol; ++col) {
     set_colour(a, m, col, lay);

@@ -91,7 +91,8 @@ struct KArgs {
   int N, Ns, nb, zmax, R, ncol;
   int c_begin, c_count, nblk;
   espg::FastDiv dnblk;           // by nblk
-  int has_si, has_h, xcd_remap;
+  int has_si, has_h;
+  unsigned xcd_full;             // blocks of the replicas that keep to one XCD (espg::place_block)
   int sweep_off, tps;            // tps: lanes cooperating on one site (1, 2, 4, 8)
   double tilt;
   uint32_t key0, key1, stream_base;
@@ -405,13 +406,6 @@ __device__ __forceinline__ bool decide(const KArgs &a, int b, const Proposal &p,
   return (de > 0.0) && (exp(-beta * de) < p.u3);
 }
 
-__device__ __forceinline__ void decode_block(const KArgs &a, int &r, int &b) {
-  // blocks go round-robin over the 8 XCDs: keep a replica on one XCD/L2
-  const unsigned L = blockIdx.x, q = a.xcd_remap ? L >> 3 : L, w = espg::fdiv(q, a.dnblk);
-  b = (int)(q - w * a.dnblk.d);
-  r = (int)(a.xcd_remap ? (L & 7u) + 8u * w : w);
-}
-
 // Lane moves of a double without LDS traffic: DPP within a row of 16 lanes, and the sum of a
 // value with its neighbour row's / half wave's (v_permlane16_swap, v_permlane32_swap).
 template <int CTRL>
@@ -582,7 +576,7 @@ template <int MODE, int LAY, bool HB, bool HD, bool SELF, int CH>
 __global__ __launch_bounds__(kPhaseBlock) ESP_PHASE_ATTR void k_phase(KArgs a) {
   extern __shared__ double s_ctab[];
   int r, b;
-  decode_block(a, r, b);
+  espg::place_block(blockIdx.x, a.xcd_full, a.dnblk, r, b);
   if (r >= a.R) return;  // uniform per block
   phase_body<MODE, LAY, HB, HD, SELF, CH>(a, r, b, s_ctab);
 }

@@ -452,7 +452,7 @@ template <bool CMP, bool HB, bool HD>
 __global__ __launch_bounds__(kBlock) ESP_LEARN_ATTR void k_phase_learned(KArgs a, const uint16_t *wbf16) {
   extern __shared__ double s_dyn[];  // [ctab][weights as float]
   int r, b;
-  decode_block(a, r, b);
+  espg::place_block(blockIdx.x, a.xcd_full, a.dnblk, r, b);
   if (r >= a.R) return;
   const int nct = CMP ? a.nb * a.zmax * 5 : 0;
   double *ctab = s_dyn;
@@ -959,7 +959,7 @@ int learn_enqueue_sweeps(esp_ctx *c, uint64_t seed, int nsweeps, int off0, hipEv
       if (a.c_count == 0) continue;
       a.nblk = (a.c_count + kBlock - 1) / kBlock;
       a.dnblk = espg::make_fastdiv((uint32_t)a.nblk);
-      a.xcd_remap = (c->R % 8 == 0) ? 1 : 0;
+      a.xcd_full = espg::xcd_full(c->R, a.nblk);
       a.sweep_off = off0 + s;
       if (ev)
         hipExtLaunchKernelGGL(fn, dim3(a.nblk * c->R), dim3(kBlock), shm, c->stream, ev[2 * k], ev[2 * k + 1], 0,
