@@ -79,6 +79,13 @@ struct Geo {
   int ngroups, zmax, N;
 };
 
+// Tiles of a wave's 64 lanes that a group of mt sites is cut into, evenly.  They serve the colour
+// phases where at least half of their lanes have a site, which is from 32 sites; else the phases read
+// the tables.  us per colour phase, tiles / tables: 27 sites 21.3 / 14.2 (FCC 18^3 x 64) and 8.9 / 7.1
+// (SC 6^3 x 1000), 64 sites 15.1 / 16.9 (FCC 24^3 x 32), 125 sites 24.5 / 31.2 (FCC 30^3 x 32).
+ESP_HD int tile_count(int mt) { return (mt + 63) / 64; }
+ESP_HD bool tiles_serve(int mt) { return 2 * mt >= 64 * tile_count(mt); }
+
 // Per-group record: basis atom and residue, packed a | r0 << 8 | r1 << 16 | r2 << 24.
 ESP_HD int grp_pack(int a, int r0, int r1, int r2) { return a | (r0 << 8) | (r1 << 16) | (r2 << 24); }
 

@@ -1041,13 +1041,11 @@ inline void sum_rej_sub(const std::vector<int64_t> &sub, int R, int64_t *out) {
   }
 }
 
-// Geometry-group tiles of a colour (host): a group's sites in tseg tiles of at most 64, evenly.
-// Worth it from 16 sites per group; below, most lanes of a tile would idle and the tables win.
-constexpr int kGeoMinSites = 16;
+// Geometry-group tiles of a colour (host).
 inline bool geo_tiles(const esp::HostModel &m, int tps) {
-  return m.implicit && m.compressed && tps == 1 && (int)m.geo.mt.d >= kGeoMinSites;
+  return m.implicit && m.compressed && tps == 1 && espg::tiles_serve((int)m.geo.mt.d);
 }
-inline int geo_tseg(const esp::HostModel &m) { return ((int)m.geo.mt.d + 63) / 64; }
+inline int geo_tseg(const esp::HostModel &m) { return espg::tile_count((int)m.geo.mt.d); }
 inline void geo_args(KArgs &a, const esp::HostModel &m) {
   constexpr int kW = kPhaseBlock / 64;
   a.tseg = geo_tseg(m);

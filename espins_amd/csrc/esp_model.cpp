@@ -409,8 +409,9 @@ void build_implicit(HostModel &hm, const int L[3], const int P[3], const double 
       if (espg::geo_partner(G, sg, e[0], e[1]) != hm.nbr[(size_t)l * N + d]) return;
     }
   }
-  // Groups of a few sites (a colouring whose period is most of the box) fill no wave: the colour
-  // phases read the tables anyway, and the records would be larger than those.
+  // Models with many group records for their sites keep the tables' layout: groups of a few sites,
+  // which fill no wave (espg::tiles_serve), under long bond lists.  (From 32 sites a group the line
+  // takes some 400 bonds to a site.)
   const size_t rows = std::min<size_t>(ngroups, 255 / mt + 2);
   if (sizeof(double) * kCoef * nb * zp + sizeof(int) * rows * (2 * zp + 1) > 49152) return;
   hm.implicit = true;
