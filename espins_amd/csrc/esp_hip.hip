@@ -371,6 +371,7 @@ bool cluster_possible(const esp_ctx *c, int mode) {
 constexpr int kClusterMinSites = 384;
 constexpr int kClusterLateSteps = 256;
 constexpr int kClusterSkip = 256;
+constexpr int kClusterShort = 7;
 bool cluster_early(const esp_ctx *c, int mode) {
   return cluster_possible(c, mode) && (!lds_sweeps(c, mode) || c->hm.N / std::max(1, c->hm.ncol) >= kClusterMinSites);
 }
@@ -384,8 +385,14 @@ bool cluster_early(const esp_ctx *c, int mode) {
 // 18.4 / 16.4 (with second neighbours, 4 colours, 2 passes), 18.8 / 23.5 (sc 14^3, 4 and 3),
 // 28.3 / 32.6 (fcc 10^3, 8 and 2).
 // Beside runs of other contexts k_lds leaves them the CUs that it does not need.
-bool cluster_sweeps(const esp_ctx *c, int mode, bool exchange, int round, int nsteps) {
+// A call of clusters costs about 28 us more than one of launches (clearing the flags, filling the LDS,
+// reading back how the launch went) and saves 4 us or so a phase: calls of fewer than kClusterShort
+// phases, a measured step counting as one more, take the other paths.  us a call, cluster / phases: one
+// sweep of sc 18^3 x 24 (2 colours) 48 / 26, with second neighbours (4) 55 / 42, fcc 12^3 x 64 (4) 55 /
+// 44; one step of fcc 20^3 x 3 (6) 74 / 78.  They cross at 6 to 12 phases, for sc 64^3 at 4.
+bool cluster_sweeps(const esp_ctx *c, int mode, int M, bool measure, bool exchange, int round, int nsteps) {
   if (!cluster_possible(c, mode)) return false;
+  if ((int64_t)nsteps * ((int64_t)M * c->hm.ncol + (measure || exchange)) < kClusterShort) return false;
   if (!lds_sweeps(c, mode)) return true;
   if (running(c) > 1) return false;
   const bool early = cluster_early(c, mode);
@@ -401,7 +408,7 @@ int run_clusters(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, i
                  int round, int64_t *ran) {
   *ran = 0;
   c->cluster_sweeps = c->cluster_launches = 0;
-  if (!cluster_sweeps(c, mode, exchange, round, nsteps)) return ESP_OK;
+  if (!cluster_sweeps(c, mode, M, measure, exchange, round, nsteps)) return ESP_OK;
   int rc = esp::cluster_prepare(c);
   if (rc || !c->cluster) return rc;
   // A launch that found its CUs taken cost its wait: 1, 2, 4, ... kClusterSkip runs go without
