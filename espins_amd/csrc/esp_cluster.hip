@@ -571,6 +571,8 @@ void cluster_free(esp_ctx *c) {
   delete q;
 }
 
+int cluster_built(const esp_ctx *c) { return c->cluster && c->cluster_R == c->R ? c->cluster->k : 0; }
+
 // Decides whether clusters serve this context and builds their tables, once per (model, replica
 // count).  c->cluster stays null if not.
 int cluster_prepare(esp_ctx *c) {
@@ -712,7 +714,7 @@ int esp_plan_clusters(int N, int nb, const double *mag, int zJ, const int *j_cnt
 
 int esp_get_cluster_info(esp_ctx *c, int64_t *out) {
   if (!c || !out) return ESP_EINVAL;
-  out[0] = c->cluster && c->cluster_R == c->R ? c->cluster->k : 0;
+  out[0] = esp::cluster_built(c);
   out[1] = c->cluster_sweeps;
   out[2] = c->cluster_launches;
   out[3] = c->cluster_skip;

@@ -149,6 +149,7 @@ namespace esp {
 int cluster_prepare(esp_ctx *c);
 int cluster_run(esp_ctx *c, int mode, double tilt, uint64_t seed, int nsteps, int M, bool measure, bool exchange,
                 int round, int64_t *ran, bool *left);
+int cluster_built(const esp_ctx *c);   // parts per replica that tables are laid out for, or 0
 void cluster_free(esp_ctx *c);
 }  // namespace esp
 

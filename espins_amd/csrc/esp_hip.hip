@@ -377,13 +377,15 @@ bool cluster_early(const esp_ctx *c, int mode) {
 }
 
 // Where one block holds a replica, both serve.  k_lds pays a launch and an exchange kernel per
-// exchange (14 us), a cluster the flags between its blocks in every phase and step.  us per step,
-// cluster / k_lds, with an exchange every step: sc 8^3 10.8 / 16.9, sc 12^3 12.5 / 21.0, fcc 8^3
-// 22.0 / 28.6; every 10 steps: 8.3 / 4.5, sc 14^3 12.7 / 11.8 -- the lines cross at 2 to 6 steps.
-// Without exchanges k_lds takes about 2 us per phase and pass of its threads over the colour, a
-// cluster 8 + 2.7 per phase: 11.2 / 7.4 (sc 12^3, 2 colours, 2 passes), 14.0 / 13.6 (sc 16^3, 4),
-// 18.4 / 16.4 (with second neighbours, 4 colours, 2 passes), 18.8 / 23.5 (sc 14^3, 4 and 3),
-// 28.3 / 32.6 (fcc 10^3, 8 and 2).
+// exchange (16 us), a cluster the flags between its blocks in every phase and 4 to 8 us a measured
+// step.  us per step, cluster / k_lds, with an exchange every step: sc 8^3 10.8 / 16.9, sc 12^3 x 85
+// 15.2 / 22.2, fcc 8^3 x 85 22.9 / 29.7; every 3 steps 16.8 / 12.6, 23.7 / 20.0, and where k_lds takes
+// more than four passes of its threads over the colours of a sweep sc 14^3 x 85 18.0 / 16.2, with
+// second neighbours 24.4 / 29.1, fcc 10^3 x 85 26.4 / 33.3; every 10 steps sc 8^3 8.3 / 4.5.
+// Otherwise k_lds takes 1.5 to 3.5 us per phase and pass, a cluster 3.7 per phase and pass of its
+// parts: 11.2 / 7.4 (sc 12^3, 2 colours, 2 passes), 13.5 / 14.3 (sc 16^3 x 48: 2, 4 against 1),
+// 17.3 / 14.3 (x 85: 4 against 2), 18.1 / 13.3 (bcc 12^3 x 85: 4 against 2), 21.2 / 24.2 (sc 14^3 x
+// 64 with second neighbours), 22.7 / 28.0 (fcc 10^3 x 85); unmeasured sweeps of sc 16^3 x 85 10.8 / 13.9.
 // Beside runs of other contexts k_lds leaves them the CUs that it does not need.
 // A call of clusters costs about 28 us more than one of launches (clearing the flags, filling the LDS,
 // reading back how the launch went) and saves 4 us or so a phase: calls of fewer than kClusterShort
@@ -396,11 +398,12 @@ bool cluster_sweeps(const esp_ctx *c, int mode, int M, bool measure, bool exchan
   if (!lds_sweeps(c, mode)) return true;
   if (running(c) > 1) return false;
   const bool early = cluster_early(c, mode);
-  if (exchange && round <= 3)
-    return early || (c->cluster && c->cluster_R == c->R) || nsteps >= kClusterLateSteps;
-  const int ncol = std::max(1, c->hm.ncol);
+  const int ncol = std::max(1, c->hm.ncol), per = c->hm.N / ncol, k = esp::cluster_built(c);
   const int passes = (c->hm.N * c->tps / ncol + kLdsBlock - 1) / kLdsBlock;
-  return early && ncol * (passes - 1) > 4;
+  if (exchange && (round <= 2 || (round == 3 && ncol * passes > 4)))
+    return early || k > 0 || nsteps >= kClusterLateSteps;
+  const int own = measure && k > 0 ? std::max(1, (per / k + kLdsBlock - 1) / kLdsBlock) : 1;   // a part's passes
+  return early && ncol * (passes - own) > 4;
 }
 
 // A run on clusters, as far as they serve it: *ran of its nsteps M sweeps (from the device clock).
