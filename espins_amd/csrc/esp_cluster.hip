@@ -119,13 +119,35 @@ __device__ __forceinline__ FinLds fin_lds(double *p, int R) {
   return f;
 }
 
+// Sums of a replica's parts where they are more than 16 (of at most 15 replicas): 16 threads to a sum.
+// One thread made 32 round trips for one replica on 256 CUs; a measured step of sc 32^3 took 28.3 us,
+// 18.7 so.  Not inlined: the registers of the colour phases stay as they are without it (inlined, 60
+// steps of fcc 15^3 x 37 took 3064 us, 3022 without, 3005 so).
+__device__ __attribute__((noinline)) void sum_many(const double *part, int k, int R, double *out) {
+  const int each = (k + 15) >> 4, b1 = (threadIdx.x & 15) * each, b2 = min(k, b1 + each);
+  for (int q = threadIdx.x >> 4; q < R * 4; q += kCBlock / 16) {
+    double x = 0.0;
+    const double *p = part + (size_t)(q >> 2) * k * 4 + (q & 3);
+    for (int b0 = b1; b0 < b2; b0 += 8) {
+      double t[8];
+#pragma unroll
+      for (int b = 0; b < 8; ++b) t[b] = b0 + b < b2 ? ald(p + 4 * (b0 + b)) : 0.0;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) x += t[b];
+    }
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) x += __shfl_xor(x, o);
+    if (b1 == 0) out[q] = x;
+  }
+}
+
 template <int MODE, bool CMP, bool HB, bool HD, bool SELF, int NG>
 __global__ __launch_bounds__(kCBlock) void k_cluster(CArgs c) {
   constexpr int ZP = NG * kGroup / 2;            // partner pairs held in registers
   extern __shared__ double s_dyn[];
   __shared__ double s_red[4 * (kCBlock / 64)];
   __shared__ int s_ok, s_col[kCMaxCol + 1], s_hal[kCMaxCol + 1];
-  __shared__ unsigned long long s_rej;
+  __shared__ unsigned s_rej;
   const KArgs &a = c.a;
   int r, j;
   {
@@ -342,7 +364,7 @@ __global__ __launch_bounds__(kCBlock) void k_cluster(CArgs c) {
     for (int i = tid; i < P.nown; i += kCBlock) { v[0] += lx[i]; v[1] += ly[i]; v[2] += lz[i]; }
     const double t4 = wave_total4(wsum, v[0], v[1], v[2]);
     if ((tid & 63) < 4) s_red[(tid & 63) * (kCBlock / 64) + (tid >> 6)] = t4;
-    unsigned long long nr = nrej;     // (a thread's own count fits 32 bits: a launch has kPhases phases at most)
+    unsigned nr = nrej;     // (32 bits: a block of 6826 sites at most makes kPhases / 2 sweeps a launch at most)
     for (int o = 32; o > 0; o >>= 1) nr += __shfl_down(nr, o, 64);
     nrej = 0;
     if ((tid & 63) == 0 && nr) atomicAdd(&s_rej, nr);
@@ -361,7 +383,7 @@ __global__ __launch_bounds__(kCBlock) void k_cluster(CArgs c) {
       stores_done();
       if (tid == 0) {
         __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (s_rej) gadd(&a.rej[(size_t)(blockIdx.x % kRejSub) * a.R + slot], s_rej);
+        if (s_rej) gadd(&a.rej[(size_t)(blockIdx.x % kRejSub) * a.R + slot], (unsigned long long)s_rej);
         s_rej = 0;
       }
     }
@@ -370,24 +392,21 @@ __global__ __launch_bounds__(kCBlock) void k_cluster(CArgs c) {
       __syncthreads();
       if (!s_ok) { if (tid == 0) ast(&c.ctl->failed, 1u); return; }
       // block 0 sums the parts, runs the estimators and the exchange and publishes the slots
-      // (2^ll threads to a sum, of up to 16 parts each: for one replica on 256 CUs one thread made 32
-      // round trips; a measured step of sc 32^3 took 28.3 us, 18.7 so)
-      int ll = 0;
-      while ((16 << ll) < c.k && (a.R * 8 << ll) <= kCBlock) ++ll;
-      const int each = (c.k + (1 << ll) - 1) >> ll;
-      for (int q0 = tid; q0 < a.R * 4 << ll; q0 += kCBlock) {
-        const int q = q0 >> ll, b1 = (q0 & ((1 << ll) - 1)) * each, b2 = min(c.k, b1 + each);
-        double x = 0.0;
-        const double *p = part + (size_t)(q >> 2) * c.k * 4 + (q & 3);
-        for (int b0 = b1; b0 < b2; b0 += 8) {
-          double t[8];
+      if (c.k > 16) {
+        sum_many(part, c.k, a.R, fl.part);
+      } else {
+        for (int q = tid; q < a.R * 4; q += kCBlock) {
+          double x = 0.0;
+          const double *p = part + (size_t)(q >> 2) * c.k * 4 + (q & 3);
+          for (int b0 = 0; b0 < c.k; b0 += 8) {
+            double t[8];
 #pragma unroll
-          for (int b = 0; b < 8; ++b) t[b] = b0 + b < b2 ? ald(p + 4 * (b0 + b)) : 0.0;
+            for (int b = 0; b < 8; ++b) t[b] = b0 + b < c.k ? ald(p + 4 * (b0 + b)) : 0.0;
 #pragma unroll
-          for (int b = 0; b < 8; ++b) x += t[b];
+            for (int b = 0; b < 8; ++b) x += t[b];
+          }
+          fl.part[q] = x;
         }
-        for (int o = 0; o < ll; ++o) x += __shfl_xor(x, 1 << o);
-        if (b1 == 0) fl.part[q] = x;
       }
       __syncthreads();
       FinArgs f = c.f;
