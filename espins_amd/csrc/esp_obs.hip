@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <type_traits>
 #include <vector>
 
 #include "esp_ctx.h"
@@ -93,6 +94,9 @@ __device__ __forceinline__ int pm_bin(const ObsArgs &o, double x) {
   return k > o.nfreq - 1 ? o.nfreq - 1 : k;
 }
 
+template <int N>
+using Count = std::integral_constant<int, N>;
+
 // kCellsPerThread cells per thread (nb consecutive reference sites each), cells in the order
 // of cdev: a block covers kObsBlock x kCellsPerThread cells, so the P(m) histogram in LDS is
 // cleared and flushed (one global atomic per non-empty bin) once per that many cells.
@@ -114,17 +118,17 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_cells(ObsArgs o) {
     if (c >= o.ncell) break;
     V3 m = {0.0, 0.0, 0.0}, st = {0.0, 0.0, 0.0};
     double op = 0.0;
-    for (int a0 = 0; a0 < o.nb; a0 += 4) {       // four atoms' loads in flight together
-      int d[4];
-      V3 sp[4];
+    auto atoms = [&](auto count, int a0) {       // the loads of `count` atoms in flight together
+      constexpr int n = decltype(count)::value;
+      int d[n];
+      V3 sp[n];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) d[k] = gldi(o.cdev, (size_t)min(a0 + k, o.nb - 1) * o.ncell + c);
+      for (int k = 0; k < n; ++k) d[k] = gldi(o.cdev, (size_t)(a0 + k) * o.ncell + c);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) sp[k] = spin_at(o, r, d[k]);
+      for (int k = 0; k < n; ++k) sp[k] = spin_at(o, r, d[k]);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < n; ++k) {
         const int a = a0 + k;
-        if (a >= o.nb) break;
         const V3 s = sp[k];
         m.x += s.x; m.y += s.y; m.z += s.z;
         if (OP) op += s.x * cldi(o.axes, 3 * a) + s.y * cldi(o.axes, 3 * a + 1) + s.z * cldi(o.axes, 3 * a + 2);
@@ -133,7 +137,14 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_cells(ObsArgs o) {
           st.x += w * s.x; st.y += w * s.y; st.z += w * s.z;
         }
       }
-    }
+    };
+    // four atoms at a time, then what is left (repeating the last atom to fill a group took 11.4 us
+    // for cells of one atom, sc 24^3 x 64, against 8.5 so)
+    int a0 = 0;
+    for (; a0 + 4 <= o.nb; a0 += 4) atoms(Count<4>{}, a0);
+    if (o.nb - a0 == 3) atoms(Count<3>{}, a0);
+    else if (o.nb - a0 == 2) atoms(Count<2>{}, a0);
+    else if (o.nb - a0 == 1) atoms(Count<1>{}, a0);
     v[0] += op; v[1] += st.x; v[2] += st.y; v[3] += st.z;
     if (PM) {
       int bins[3], nbin = 0;
