@@ -181,9 +181,11 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_cells(ObsArgs o) {
 // replicas and one spin gather per replica; rows go in groups of kRows, whose table loads and then
 // gathers are in flight together (one round trip per group instead of per row).  (Keeping a replica group on one
 // XCD, as the sweep does, measured slower here: 468 against 404 us on FCC 32^3 x 64.)
+// Rows past the last whole group go one by one: eight shells of one row each, sc 24^3 x 64, took 77 us
+// with whole groups only (the last row repeated), 59 so.  (Three kinds need 128 VGPRs for four waves.)
 constexpr int kRows = 3;
 template <int NS, int REP>
-__global__ __launch_bounds__(kObsBlock) void k_obs_spincorr(ObsArgs o) {
+__global__ __launch_bounds__(kObsBlock, NS == 3 ? 4 : 1) void k_obs_spincorr(ObsArgs o) {
   constexpr int NV = 2 * NS * NS * REP;
   __shared__ double red[NV * (kObsBlock / 64)];
   const int b = blockIdx.x;
@@ -207,25 +209,24 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_spincorr(ObsArgs o) {
     for (int u = 0; u < REP; ++u)
 #pragma unroll
       for (int y = 0; y < NS; ++y) { v[u][0][y] = v[u][1][y] = vr[u][0][y] = vr[u][1][y] = 0.0; }
-    const int l1 = gldi(o.soff, s + 1);
-    for (int l0 = gldi(o.soff, s); l0 < l1; l0 += kRows) {
-      unsigned e[kRows];
-      double w[kRows], wr[kRows];
-      V3 sj[kRows][REP];
+    auto rows = [&](auto count, int l0) {
+      constexpr int n = decltype(count)::value;
+      unsigned e[n];
+      double w[n], wr[n];
+      V3 sj[n][REP];
 #pragma unroll
-      for (int k = 0; k < kRows; ++k) {          // rows past the shell repeat its last, weight 0
-        const int l = min(l0 + k, l1 - 1);
+      for (int k = 0; k < n; ++k) {
+        const int l = l0 + k;
         e[k] = gldi(o.sbond, (size_t)l * o.N + d);
         w[k] = gldi(o.sw, (size_t)l * o.N + d);
         wr[k] = NS > 1 ? gldi(o.sw, ((size_t)o.srows + l) * o.N + d) : 0.0;
-        if (l0 + k >= l1) { w[k] = 0.0; wr[k] = 0.0; }
       }
 #pragma unroll
-      for (int k = 0; k < kRows; ++k)
+      for (int k = 0; k < n; ++k)
 #pragma unroll
         for (int u = 0; u < REP; ++u) sj[k][u] = spin_at(o, ru[u], (int)(e[k] & kBondIdx));
 #pragma unroll
-      for (int k = 0; k < kRows; ++k) {
+      for (int k = 0; k < n; ++k) {
         const int kj = NS > 1 ? (int)(e[k] >> kBondKindShift) : 0;
 #pragma unroll
         for (int u = 0; u < REP; ++u) {
@@ -239,7 +240,11 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_spincorr(ObsArgs o) {
             }
         }
       }
-    }
+    };
+    int l = gldi(o.soff, s);
+    const int l1 = gldi(o.soff, s + 1);
+    for (; l + kRows <= l1; l += kRows) rows(Count<kRows>{}, l);
+    for (; l < l1; ++l) rows(Count<1>{}, l);
     double f[NV];
 #pragma unroll
     for (int u = 0; u < REP; ++u)
