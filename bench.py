@@ -349,8 +349,8 @@ def extras_into(out, args):
         r = run_single(args, cfg, steps, warm, with_cpu=False, emit=False)
         rf = r["roofline"]
         ex[cfg] = {"workload": r["config"]["workload"], "value": r["value"], "unit": "updates/s",
-                   "ms_per_step": r["ms_per_step"], "steps": steps, "kernel": rf["kernel"],
-                   "mean_launch_us": rf["mean_launch_us"], "roofline_frac": rf["frac"],
+                   "ms_per_step": r["ms_per_step"], "steps": steps, "kernel": r["config"]["run_kernel"],
+                   "roofline_kernel": rf["kernel"], "mean_launch_us": rf["mean_launch_us"], "roofline_frac": rf["frac"],
                    "bytes_per_update": rf["bytes_per_update"]}
     out["extras"] = ex
     ess = profile_ess()
@@ -594,6 +594,8 @@ def run_single(args, config, steps, warmup, with_cpu=True, emit=True):
     dt = time.perf_counter() - t0
     updates = m.N * R * steps
     value = updates / dt
+    served = eng.cluster_info()["sweeps"] > 0          # replicas on clusters of blocks
+    run_kernel = "k_cluster" if served else "k_lds" if info["lds"] else "k_phase"
     st = eng.stats()
     acc_rate = 1.0 - st["rejected"].sum() / float(updates)
     sr, ns = eng.pt_map()
@@ -601,7 +603,8 @@ def run_single(args, config, steps, warmup, with_cpu=True, emit=True):
     log(f"{config} timed: {steps} steps in {dt:.3f} s -> {value / 1e9:.3f} G updates/s; "
         f"acceptance {acc_rate:.4f}, swap acceptance {swap_rate:.4f}")
 
-    # sweep-kernel roofline (HIP events around each launch on the engine's stream)
+    # sweep-kernel roofline (HIP events around each launch on the engine's stream): of the launches
+    # that time_sweeps makes, k_lds or k_phase, also where clusters served the timed steps
     nsw = max(10, min(200, steps // 10))
     tm = eng.time_sweeps(nsw, mode="random", seed=seed + 1, sweep0=10 ** 9)
     pb = phase_bytes(m)[0] * R                  # minimal bytes of one sweep of every replica
@@ -632,7 +635,8 @@ def run_single(args, config, steps, warmup, with_cpu=True, emit=True):
         "data": "synthetic",
         "config": {"workload": desc, "N": m.N, "replicas": R, "sweeps_per_step": 1,
                    "exchange_every": 1 if pt else 0, "mode": "random", "colours": info["ncol"],
-                   "kernel_path": "lds" if info["lds"] else "global", "graph": graph,
+                   "kernel_path": "clusters" if served else "lds" if info["lds"] else "global", "graph": graph,
+                   "run_kernel": run_kernel,
                    "observables": getattr(args, "observables", None)},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
