@@ -102,7 +102,7 @@ using BLdsFn = void (*)(const KArgs *, const LdsMeas *, const int2 *, int, int);
 constexpr int kVarChunk4 = 32;
 constexpr size_t kGroupBytes = size_t(192) << 20;   // spins of a replica group
 constexpr size_t kGroupMax = 3 * kGroupBytes;        // spins of a batch that is split
-constexpr int kNarrow = 2;   // the narrow setting, as set_chain_chunk and info name it
+constexpr int kNarrow = 2;   // the narrow setting (kChunk in flight), as set_chain_chunk and info name it
 template <int MODE, int LAY, bool HB, bool HD, int CH>
 BPhaseFn bp4(bool self) { return self ? k_bphase<MODE, LAY, HB, HD, true, CH> : k_bphase<MODE, LAY, HB, HD, false, CH>; }
 template <int MODE, int LAY, bool HB, int CH>
@@ -390,7 +390,10 @@ int build_plan(esp_batch *b, double tilt, uint64_t seed) {
   // come from HBM each time; a launch more costs about 4 us.  24 chains of 369 MB, 60 rounds, in
   // groups of 32 / 64 / 96 / 128 / 192 MB and in one: 65 / 52 / 46 / 43 / 41 / 43 ms.  Much larger
   // batches stay in one: a launch is long there, and with few large replicas to a group the XCDs
-  // end unevenly (256 chains, 11.3 GB: 24.3 G updates/s in one, 24.0 in 59 groups).
+  // end unevenly (256 chains, 11.3 GB: 24.3 G updates/s in one, 24.0 in 59 groups).  The line between
+  // is cautious.  us a round in one / in groups: L = 32, 394 MB 739 / 664, 697 MB 1359 / 1251, 1179 MB
+  // 2360 / 2131, 2364 MB 4417 / 4024; L = 24, 710 MB 1296 / 1167, 1766 MB 3088 / 2763; L = 48, 805 MB
+  // 1508 / 1465, 2352 MB 4180 / 4205.
   // Chains with as many colours stand together (a group's last colours would run a few chains).
   std::vector<std::vector<int4>> groups;              // (chain, first replica, end)
   {

@@ -31,9 +31,10 @@ using namespace espd;
 
 constexpr int kBlock = 256;      // reduce and measurement kernels (4 waves)
 constexpr int kPhaseBlock = 256; // colour-phase kernels (64 and 512 measured the same, 1024 slower)
-// Launches of a round that is captured into a graph at most.  The captured chain has a
-// node per launch, and 528k of them ended in a segmentation fault of the host (within the runtime,
-// whose graph calls most likely recurse along the chain).  A longer round is launched as it is; the host enqueues a launch in 3 us or less, the shortest phases take 4.
+// Launches of a round that is captured into a graph at most.  The captured chain has a node per
+// launch, and 528k of them ended in a segmentation fault of the host (within the runtime, whose graph
+// calls most likely recurse along the chain).  A longer round is launched as it is; the host enqueues
+// a launch in 3 us or less, the shortest phases take 4.
 constexpr int64_t kCaptureMax = 4096;
 constexpr int kLdsBlock = 512;   // LDS-resident kernel (8 waves per replica)
 // Tuning constants (compile-time; the defaults are the measured best on MI355X).  Fewer

@@ -12,8 +12,8 @@
 // counts through a histogram in LDS), k_obs_spincorr (one thread per site and several
 // replicas, device order), k_sf_pack / k_sf_main / k_sf_fin (S(q) as a phase-matrix times
 // spin-matrix product: one phase per q-point, site and 8 replicas; k_sf_plane / k_sf_q for lattice
-// positions: summed axis by axis; k_sf_lat for lattices of few sites to a plane or of few planes) and k_obs_final (per replica: fixed-order sums of the
-// block partials, accumulation into the replica's slot).
+// positions: summed axis by axis; k_sf_lat for lattices of few sites to a plane or of few planes) and
+// k_obs_final (per replica: fixed-order sums of the block partials, accumulation into the replica's slot).
 // Histogram counts are integers, so they do not depend on the order of the atomic additions;
 // every floating-point sum has a fixed order.
 #include <hip/hip_runtime.h>

@@ -566,7 +566,8 @@ class Batch:
         return dict(kernel_ms=kms.value, nlaunch=nl.value, wall_ms=wall.value, updates=upd.value)
 
     def set_chain_chunk(self, k, chunk):
-        """Partner gathers in flight per lane on chain k's global-memory colour phases (2 or 4)."""
+        """Partner gathers in flight per lane on chain k's global-memory colour phases: 2 names the narrow
+        setting (three in flight), or 4."""
         self._chk(E.lib.esp_batch_set_chain_chunk(self._h, int(k), int(chunk)))
 
     def info(self, k):

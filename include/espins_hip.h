@@ -110,7 +110,10 @@ int esp_plan_clusters(int N, int nb, const double *mag,
                       const int *L3, int R, int num_cu, int64_t lds_bytes, int64_t *out3);
 /* Sweep kernel choice: 0 = automatic (LDS-resident when a replica fits in LDS; middle-sized
  * replicas, and small ones with frequent exchanges, on clusters of blocks), 1 = global-memory
- * colour phases, 2 = LDS-resident (EINVAL if the replica does not fit). */
+ * colour phases, 2 = LDS-resident (EINVAL if the replica does not fit).
+ * The kernels add a site's bonds in different orders, so results agree to rounding between paths;
+ * with 0 which of them serves a call depends on its length, on other work on the GPU and on earlier
+ * calls, and equal calls need not give equal bits.  With 1 or 2 they do. */
 int esp_set_path(esp_ctx *ctx, int path);
 /* Philox stream of replica r is base + r (default 0); the exchange stream is
  * 0xFFFFFFFF - base.  A batch gives chain k the base k << 16. */
@@ -323,9 +326,10 @@ int esp_batch_add_chain(esp_batch *b, int N, int nb, const double *mag,
                         int *chain_id);
 /* Per-chain kernel shape: path 0 auto / 1 global / 2 LDS, tps lanes per site. */
 int esp_batch_set_chain_config(esp_batch *b, int chain, int path, int tps);
-/* Partner gathers in flight per lane on chain k's global-memory colour phases: 2 (default)
- * or 4 (more memory-level parallelism per wave, more registers).  A kernel shape with no
- * counterpart in the reference; the autotuner searches it. */
+/* Partner gathers in flight per lane on chain k's global-memory colour phases: 2, the
+ * narrow setting (default; the kernels keep three in flight under that name), or 4 (more
+ * memory-level parallelism per wave, more registers).  A kernel shape with no counterpart in the
+ * reference; the autotuner searches it. */
 int esp_batch_set_chain_chunk(esp_batch *b, int chain, int chunk);
 int esp_batch_get_chain_chunk(esp_batch *b, int chain, int *chunk);
 /* Upload every chain (after the last esp_batch_add_chain). */
