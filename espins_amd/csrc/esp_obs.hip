@@ -181,11 +181,14 @@ __global__ __launch_bounds__(kObsBlock) void k_obs_cells(ObsArgs o) {
 // replicas and one spin gather per replica; rows go in groups of kRows, whose table loads and then
 // gathers are in flight together (one round trip per group instead of per row).  (Keeping a replica group on one
 // XCD, as the sweep does, measured slower here: 468 against 404 us on FCC 32^3 x 64.)
-// Rows past the last whole group go one by one: eight shells of one row each, sc 24^3 x 64, took 77 us
-// with whole groups only (the last row repeated), 59 so.  (Three kinds need 128 VGPRs for four waves.)
+// Rows past the last whole group go one by one: eight shells of one row each, sc 24^3 x 64, took 75 us
+// with whole groups only (the last row repeated), 63 so.  Waves per SIMD: one kind left to itself takes 8
+// with fewer loads in flight (fcc 16^3 x 32, two shells: 17.9 us; 16.7 with 6), three kinds 3 (137 us for
+// three shells of bcc 20^3 x 32; 125 with 4).
 constexpr int kRows = 3;
 template <int NS, int REP>
-__global__ __launch_bounds__(kObsBlock, NS == 3 ? 4 : 1) void k_obs_spincorr(ObsArgs o) {
+__global__ __launch_bounds__(kObsBlock) __attribute__((amdgpu_waves_per_eu(NS == 1 ? 6 : NS == 3 ? 4 : 1, NS == 1 ? 6 : 8)))
+void k_obs_spincorr(ObsArgs o) {
   constexpr int NV = 2 * NS * NS * REP;
   __shared__ double red[NV * (kObsBlock / 64)];
   const int b = blockIdx.x;
